@@ -64,7 +64,11 @@ double now_ms() {
 // the name is a stand-in, not a device address): it uses the address
 // hipGetSymbolAddress returns for the current device, looked up once per
 // device when the first context is created on it.
-constexpr size_t SCRATCH_BYTES = size_t(64) << 20;
+// Calls are accepted by the sizes the header states (SCRATCH_LIMIT); the
+// array is larger by what the symmetric far field's partial sums (20 MB at
+// FAR_SYM_MAX patches) and small SpMV items may take beyond them.
+constexpr size_t SCRATCH_LIMIT = size_t(64) << 20;
+constexpr size_t SCRATCH_BYTES = size_t(96) << 20;
 __device__ __align__(256) unsigned char scratch[SCRATCH_BYTES];
 constexpr int SCRATCH_MAX_DEVICES = 64;
 std::mutex g_scratch_mu;
@@ -93,12 +97,14 @@ struct beep_hip_ctx {
     // yfar; the context stream adds it to y (fork / join through events)
     hipStream_t far_stream = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_pack = nullptr;
+    static constexpr int SPMV_CAP_AUTO = -1;
     bool overlap = true;
     int n_cu = 256;               // compute units of the device
     // near-SpMV settings per coefficient mode (0: FP64, 1: FP32, 2: FP32
     // coefficients with FP64 sums): residency cap in blocks per CU (0: one
     // block per work item) and loads in flight per thread (x 4 FP64, x 8 FP32)
-    int spmv_cap[3] = {1, 1, 1};
+    // (SPMV_CAP_AUTO: 1 beside an FMM far field, else uncapped)
+    int spmv_cap[3] = {SPMV_CAP_AUTO, SPMV_CAP_AUTO, SPMV_CAP_AUTO};
     int spmv_depth[3] = {1, 1, 1};
     std::string err;
 
@@ -141,9 +147,15 @@ struct beep_hip_ctx {
     SpmvPlan fly;
     int near_mode = BEEP_NEAR_PRECOMPUTE;
     bool fly_ns64 = true;
+    int64_t spmv_rows_large = 0;  // partial rows of the SpMV in 256-row items
     int64_t nnz = 0;
     long long n_nb = 0;  // neighbourhood entries (nb_ptr[L])
     bool have_tree = false;
+    bool all_explicit = false;  // every pair of patches is an explicit pair, once
+    // this context's near field was shared (beep_hip_share_near): its
+    // coefficients store full - 1 point from then on (see folded)
+    bool keep_1pt = false;
+    std::mutex share_mu;
 
     // precomputed operator
     DevBuf<double> diag;
@@ -182,7 +194,9 @@ struct beep_hip_ctx {
     DevBuf<NsRec> guard_rec;
     DevBuf<unsigned> guard_cnt;
     // far-field plan each coefficient set was built for (0: none, the direct
-    // far field): pairs of the FMM leaf pass keep the full rule
+    // far field; UID_FOLDED: no far field at all, see folded): pairs of the
+    // FMM leaf pass keep the full rule
+    static constexpr unsigned long long UID_FOLDED = ~0ull;
     unsigned long long uid32 = 0, uid64 = 0;
     double kappa = 0;
 
@@ -372,6 +386,59 @@ void timing_collect(beep_hip_ctx* c) {
     while (c->ring_pending > 0) timing_pop(c);
 }
 
+// When every pair of patches is explicit (one octree leaf: up to 4 nbsize
+// patches), full - 1 point coefficients plus the direct far field over all
+// pairs is the full rule taken apart and put together again: an FP64
+// precompute then keeps the full rule (UID_FOLDED) and mat-vecs with that set
+// are the SpMV alone.  Not the FP32 set: the refinement residual applies it
+// beside an FP64 far field, and full - 1 point rounds smaller numbers (3.9e-9
+// against about 2e-8 of the mat-vec at 2,562 patches).  With the far field
+// chosen by size only (BEEP_FAR_AUTO): a caller that asks for the direct far
+// field gets it, and a near field that is shared keeps full - 1 point.
+bool fold_next(const beep_hip_ctx* c, int precision) {
+    return precision == BEEP_FP64 && c->far_mode == BEEP_FAR_AUTO && !c->use_fmm && c->all_explicit &&
+           !c->share && !c->keep_1pt;
+}
+
+unsigned long long built_for(const beep_hip_ctx* c, int precision) {
+    return precision == BEEP_FP64 ? c->uid64 : c->uid32;
+}
+
+// mat-vecs with this precision's set have no far field
+bool folded(const beep_hip_ctx* c, int precision) {
+    return !c->use_fmm && !c->share && built_for(c, precision) == beep_hip_ctx::UID_FOLDED;
+}
+
+// this precision's set fits the far field in use (either form of it without
+// the FMM)
+bool coef_plan_ok(const beep_hip_ctx* c, int precision) {
+    const unsigned long long built = built_for(c, precision);
+    if (c->use_fmm) return c->fmm && c->fmm->uid == built;
+    return built == 0 || built == beep_hip_ctx::UID_FOLDED;
+}
+
+// blocks of the near SpMV (0: one per work item)
+int spmv_blocks(const beep_hip_ctx* c, int mode) {
+    const int cap = c->spmv_cap[mode];
+    return (cap == beep_hip_ctx::SPMV_CAP_AUTO ? (c->use_fmm ? 1 : 0) : cap) * c->n_cu;
+}
+
+// the direct far field as symmetric tile pairs (far_sym.hpp)
+bool far_is_sym(const beep_hip_ctx* c) { return !c->use_fmm && c->N <= FAR_SYM_MAX; }
+
+// buffers of a mat-vec's far field
+void far_buffers(beep_hip_ctx* c) {
+    if (far_is_sym(c)) {
+        c->far_part.alloc(far_sym_values(c->N));
+        return;
+    }
+    c->yfar.alloc(size_t(2) * c->N);
+    if (c->use_fmm) return;
+    c->src.alloc(size_t(c->N));
+    const int ns = far_direct_splits(c->N, c->n_cu);
+    if (ns > 1) c->far_part.alloc(size_t(2) * c->N * ns);
+}
+
 // near-SpMV coefficient mode of a mat-vec precision
 int spmv_mode(int precision) {
     return precision == BEEP_FP64 ? 0 : (precision == BEEP_FP32 ? 1 : 2);
@@ -388,8 +455,7 @@ void matvec_dev(beep_hip_ctx* c, const double* dx, double* dy, int precision) {
         require(precision == BEEP_FP64 ? c->share->have64 : c->share->have32,
                 "the shared near field lacks this precision's coefficients");
     } else {
-        const unsigned long long built = precision == BEEP_FP64 ? c->uid64 : c->uid32;
-        require(c->use_fmm ? (c->fmm && c->fmm->uid == built) : built == 0,
+        require(coef_plan_ok(c, precision),
                 "near coefficients were precomputed for another far field: call "
                 "beep_hip_precompute again");
     }
@@ -401,11 +467,33 @@ void matvec_dev(beep_hip_ctx* c, const double* dx, double* dy, int precision) {
     if (timed && c->ring_pending == beep_hip_ctx::RING) timing_pop(c);
     hipEvent_t* ev = c->ev[c->ring_head];
     const int n2 = 2 * c->N;
-    c->yfar.alloc(size_t(n2));
-    if (!c->use_fmm) c->src.alloc(size_t(c->N));
+    const int mode = spmv_mode(precision);
+    const int far32 = precision == BEEP_FP32 ? 1 : 0;
+    const bool fold = folded(c, precision);
+    const bool sym = far_is_sym(c);
+    if (!c->capturing && !fold) far_buffers(c);
     if (timed) hip_check(hipEventRecord(ev[0], s), "hipEventRecord");
+    auto matvec_timed = [&](bool with_m2l) {
+        if (!timed) return;
+        hip_check(hipEventRecord(ev[2], s), "hipEventRecord");
+        c->slot_fmm[c->ring_head] = with_m2l;
+        c->ring_head = (c->ring_head + 1) % beep_hip_ctx::RING;
+        c->ring_pending += 1;
+    };
+    if (sym && !fold && c->overlap && !c->share && c->near_mode == BEEP_NEAR_PRECOMPUTE) {
+        // near and far field side by side in one launch, one that sums them
+        launch_direct_matvec(s, mode, c->N, c->spmv, c->leaf_ptr.p, c->leaf_idx.p, c->nb_ptr.p, c->nb_idx.p,
+                             c->coef_off.p, c->coef32.p, c->coef64.p, c->diag.p, c->patches.p, c->kappa, dx,
+                             c->spmv_part.p, c->far_part.p, dy);
+        if (timed) {
+            hip_check(hipEventRecord(ev[1], s), "hipEventRecord");
+            hip_check(hipEventRecord(ev[3], s), "hipEventRecord");
+        }
+        matvec_timed(false);
+        return;
+    }
     hipStream_t sf = s;
-    if (c->overlap) {
+    if (c->overlap && !fold) {
         sf = c->far_stream;
         hip_check(hipEventRecord(c->ev_fork, s), "hipEventRecord");
         hip_check(hipStreamWaitEvent(sf, c->ev_fork, 0), "hipStreamWaitEvent");
@@ -413,7 +501,6 @@ void matvec_dev(beep_hip_ctx* c, const double* dx, double* dy, int precision) {
     // near field (explicit pairs) + diagonal into y, launched first: the
     // SpMV is the longer of the two, and the far field's dozen short kernels
     // take the host a while to launch
-    const int mode = spmv_mode(precision);
     if (c->share) {
         // every copy of the shared patches (rows and columns at its offset,
         // f and h halves N apart), then this context's own pairs
@@ -422,32 +509,41 @@ void matvec_dev(beep_hip_ctx* c, const double* dx, double* dy, int precision) {
         for (int k = 0; k < nco; k += 2)
             launch_near_spmv(s, mode, c->N, h->spmv, h->leaf_ptr.p, h->leaf_idx.p, h->nb_ptr.p,
                              h->nb_idx.p, h->coef_off.p, h->coef32.p, h->coef64.p, h->diag.p, dx,
-                             c->spmv_part.p, dy, c->spmv_cap[mode] * c->n_cu, c->spmv_depth[mode],
+                             c->spmv_part.p, dy, spmv_blocks(c, mode), c->spmv_depth[mode],
                              std::min(2, nco - k), c->share_off.data() + k);
         launch_pair_spmv(s, mode, c->N, c->n_pair_rows, c->pair_rows.p, c->pair_ptr.p, c->pair_col.p,
                          c->pcoef32.p, c->pcoef64.p, dx, dy);
     } else if (c->near_mode == BEEP_NEAR_ON_THE_FLY) {
         launch_near_fly(s, mode, c->N, c->fly, c->leaf_ptr.p, c->leaf_idx.p, c->nb_ptr.p, c->nb_idx.p,
                         c->patches.p, c->qual_ptr.p, c->qual32.p, c->qual64.p, c->quad_ptr.p, c->quad32.p,
-                        c->quad64.p, c->kappa, c->use_fmm ? c->fmm->cellkey : nullptr, c->fly_ns64 ? 1 : 0,
+                        c->quad64.p, c->kappa, fold ? 0 : 1, c->use_fmm ? c->fmm->cellkey : nullptr, c->fly_ns64 ? 1 : 0,
                         c->guard_max, c->diag.p, dx, c->spmv_part.p, dy);
     } else {
         launch_near_spmv(s, mode, c->N, c->spmv, c->leaf_ptr.p, c->leaf_idx.p, c->nb_ptr.p,
                          c->nb_idx.p, c->coef_off.p, c->coef32.p, c->coef64.p, c->diag.p, dx,
-                         c->spmv_part.p, dy, c->spmv_cap[mode] * c->n_cu, c->spmv_depth[mode]);
+                         c->spmv_part.p, dy, spmv_blocks(c, mode), c->spmv_depth[mode]);
     }
     if (timed) hip_check(hipEventRecord(ev[1], s), "hipEventRecord");
-    // far field (1-point interaction of all pairs) into yfar
-    launch_fill(sf, n2, 0.0, c->yfar.p);
-    if (c->use_fmm) {
-        fmm_evaluate(c->fmm, sf, precision == BEEP_FP32 ? 1 : 0, c->patches.p, dx, c->kappa,
-                     c->yfar.p, timed ? &ev[4] : nullptr, c->ev_pack);
+    if (fold) {
+        // no far field: the event of its phase is recorded empty
+        if (timed) hip_check(hipEventRecord(ev[3], s), "hipEventRecord");
+        matvec_timed(false);
+        return;
+    }
+    // far field (1-point interaction of all pairs), the FMM's and the large
+    // direct sum's into yfar
+    if (sym) {
+        launch_far_sym(sf, far32, c->N, c->leaf_idx.p, c->patches.p, dx, c->kappa, c->far_part.p);
     } else {
-        launch_far_pack(sf, c->N, c->patches.p, c->leaf_idx.p, dx, c->src.p);
-        const int ns = far_direct_splits(c->N, c->n_cu);
-        if (ns > 1 && !c->capturing) c->far_part.alloc(size_t(2) * c->N * ns);
-        launch_far_direct(sf, precision == BEEP_FP32 ? 1 : 0, c->N, ns, c->leaf_idx.p,
-                          c->patches.p, c->src.p, c->kappa, c->yfar.p, c->far_part.p);
+        launch_fill(sf, n2, 0.0, c->yfar.p);
+        if (c->use_fmm) {
+            fmm_evaluate(c->fmm, sf, far32, c->patches.p, dx, c->kappa, c->yfar.p, timed ? &ev[4] : nullptr,
+                         c->ev_pack);
+        } else {
+            launch_far_pack(sf, c->N, c->patches.p, c->leaf_idx.p, dx, c->src.p);
+            launch_far_direct(sf, far32, c->N, far_direct_splits(c->N, c->n_cu), c->leaf_idx.p, c->patches.p,
+                              c->src.p, c->kappa, c->yfar.p, c->far_part.p);
+        }
     }
     if (timed) hip_check(hipEventRecord(ev[3], sf), "hipEventRecord");
     if (c->overlap) hip_check(hipEventRecord(c->ev_join, sf), "hipEventRecord");
@@ -455,15 +551,12 @@ void matvec_dev(beep_hip_ctx* c, const double* dx, double* dy, int precision) {
         // the P2P part (VALU) follows the SpMV on this stream, beside the
         // MFMA-bound M2L of the far stream; it needs the packed sources
         if (c->overlap) hip_check(hipStreamWaitEvent(s, c->ev_pack, 0), "hipStreamWaitEvent");
-        fmm_p2p(c->fmm, s, precision == BEEP_FP32 ? 1 : 0, c->patches.p, c->kappa, dy);
+        fmm_p2p(c->fmm, s, far32, c->patches.p, c->kappa, dy);
     }
     if (c->overlap) hip_check(hipStreamWaitEvent(s, c->ev_join, 0), "hipStreamWaitEvent");
-    launch_axpby(s, n2, 1.0, c->yfar.p, 1.0, dy);
-    if (!timed) return;
-    hip_check(hipEventRecord(ev[2], s), "hipEventRecord");
-    c->slot_fmm[c->ring_head] = c->use_fmm;
-    c->ring_head = (c->ring_head + 1) % beep_hip_ctx::RING;
-    c->ring_pending += 1;
+    if (sym) launch_far_sym_add(s, far32, c->N, c->leaf_idx.p, c->far_part.p, dy);
+    else launch_axpby(s, n2, 1.0, c->yfar.p, 1.0, dy);
+    matvec_timed(c->use_fmm);
 }
 
 double dev_dot(beep_hip_ctx* c, const double* a, const double* b, int n) {
@@ -509,12 +602,8 @@ void arnoldi_step(beep_hip_ctx* c, int precision, int m) {
     }
     // everything the captured launches bake in: buffers, plan, sizes
     ensure_far(c, precision == BEEP_FP32 ? BEEP_FP32 : BEEP_FP64);
-    c->yfar.alloc(size_t(2) * c->N);
-    if (!c->use_fmm) {
-        c->src.alloc(size_t(c->N));
-        const int ns = far_direct_splits(c->N, c->n_cu);
-        if (ns > 1) c->far_part.alloc(size_t(2) * c->N * ns);
-    }
+    const bool fold = folded(c, precision);
+    if (!fold) far_buffers(c);
     const std::vector<const void*> key = {
         reinterpret_cast<const void*>(uintptr_t(c->gen)), reinterpret_cast<const void*>(intptr_t(precision)),
         reinterpret_cast<const void*>(intptr_t(m)), reinterpret_cast<const void*>(intptr_t(c->N)),
@@ -522,7 +611,7 @@ void arnoldi_step(beep_hip_ctx* c, int precision, int m) {
         c->yfar.p, c->src.p, c->far_part.p, c->coef32.p, c->coef64.p, c->diag.p,
         c->spmv_part.p, c->fmm, c->hvec2.p, c->share, c->pair_ptr.p, c->pcoef32.p, c->pcoef64.p,
         reinterpret_cast<const void*>(intptr_t(c->gs_passes)),
-        reinterpret_cast<const void*>(intptr_t(c->overlap)),
+        reinterpret_cast<const void*>(intptr_t(c->overlap)), reinterpret_cast<const void*>(intptr_t(fold)),
         reinterpret_cast<const void*>(intptr_t(c->near_mode * 2 + (c->fly_ns64 ? 1 : 0))),
         reinterpret_cast<const void*>(intptr_t(c->spmv_cap[spmv_mode(precision)])),
         reinterpret_cast<const void*>(intptr_t(c->spmv_depth[spmv_mode(precision)]))};
@@ -866,19 +955,56 @@ static void begin_tree(beep_hip_ctx* ctx) {
     ctx->share_off.clear();
     ctx->n_pairs = 0;
     ctx->n_pair_rows = 0;
+    ctx->all_explicit = ctx->keep_1pt = false;
     set_device(ctx);
     sync_streams(ctx);
     ctx->gen++;
+}
+
+// Work-item shape of the near SpMV.  256 rows x 512 columns where that gives
+// several items per CU (from about 2^25 pairs, 22,000 patches at nbsize 1500).
+// Below, an item of 512 columns is one block's long serial chain while most
+// CUs have none (642 patches: 6 blocks, 54 us for 13 MB; 2,562: 86 blocks),
+// so the columns shrink until the matrix gives about 1,024 items of 64 rows,
+// not below 32 columns (a thread then has two batches of loads): 4.7 us at
+// 642 patches (FP64), 12 at 2,562 (FP32, 48 before), 83 at 10,242 (FP64).  A leaf of up
+// to 128 rows stays whole: its columns are contiguous in memory.
+// The small shape's row partials stay within the large one's scratch, or 8 MiB.
+struct SpmvShape {
+    int rows = 256, cols = SPMV_CW;  // rows: partials per item
+    int step(int64_t R) const { return rows == 256 ? 256 : (R <= rows ? int(R) : 64); }
+    int64_t partial_rows(int64_t R, int64_t C) const { return items(R, C) * rows; }
+    int64_t items(int64_t R, int64_t C) const { return (R + step(R) - 1) / step(R) * ((C + cols - 1) / cols); }
+};
+static SpmvShape spmv_shape(int L, const int* leaf_ptr, const int* nb_ptr) {
+    const SpmvShape large;
+    SpmvShape small;
+    int64_t nnz = 0;
+    for (int l = 0; l < L; ++l)
+        nnz += int64_t(leaf_ptr[l + 1] - leaf_ptr[l]) * int64_t(nb_ptr[l + 1] - nb_ptr[l]);
+    if (nnz >= int64_t(1) << 25) return large;
+    small.rows = 128;
+    small.cols = int(std::max<int64_t>(32, std::min<int64_t>(SPMV_CW, (nnz / (1024 * 64) + 31) / 32 * 32)));
+    int64_t rows_large = 0, rows_small = 0;
+    for (int l = 0; l < L; ++l) {
+        const int64_t R = leaf_ptr[l + 1] - leaf_ptr[l], C = nb_ptr[l + 1] - nb_ptr[l];
+        if (R <= 0 || C <= 0) continue;  // refused by the caller
+        rows_large += large.partial_rows(R, C);
+        rows_small += small.partial_rows(R, C);
+    }
+    return rows_small <= std::max<int64_t>(rows_large, int64_t(1) << 19) ? small : large;
 }
 
 // The SpMV and on-the-fly plans of a tree whose leaf_idx and nb_idx are on
 // the device already: per leaf the offset of its coefficient block, and the
 // work items (row group x column slab) of both plans.
 static void install_tree(beep_hip_ctx* ctx, int L, const int* leaf_ptr, const int* nb_ptr) {
+    const SpmvShape shape = spmv_shape(L, leaf_ptr, nb_ptr);
     std::vector<int64_t> off(L + 1, 0);
     std::vector<int> cblk(L + 1, 0);
     std::vector<int4> work, groups, fwork, fgroups;
     std::vector<int> gnb, fgnb;
+    int64_t rows_large = 0;
     for (int l = 0; l < L; ++l) {
         const int64_t R = leaf_ptr[l + 1] - leaf_ptr[l];
         const int64_t C = nb_ptr[l + 1] - nb_ptr[l];
@@ -887,11 +1013,14 @@ static void install_tree(beep_hip_ctx* ctx, int L, const int* leaf_ptr, const in
         const int64_t nb = (R * C + 255) / 256;
         require(int64_t(cblk[l]) + nb < (int64_t(1) << 31), "too many coefficient blocks");
         cblk[l + 1] = cblk[l] + int(nb);
-        for (int r0 = 0; r0 < R; r0 += 256) {
+        rows_large += SpmvShape().partial_rows(R, C);
+        const int rstep = shape.step(R);
+        for (int r0 = 0; r0 < R; r0 += rstep) {
             const int first = int(work.size());
-            for (int c0 = 0; c0 < C; c0 += SPMV_CW)
-                work.push_back(make_int4(l, r0, c0, int(std::min<int64_t>(SPMV_CW, C - c0))));
-            groups.push_back(make_int4(l, r0, int(std::min<int64_t>(256, R - r0)), first));
+            const int rows = int(std::min<int64_t>(rstep, R - r0));
+            for (int c0 = 0; c0 < C; c0 += shape.cols)
+                work.push_back(make_int4(l, r0, c0, int(std::min<int64_t>(shape.cols, C - c0)) | rows << 16));
+            groups.push_back(make_int4(l, r0, rows, first));
             gnb.push_back(int(work.size()) - first);
         }
         for (int r0 = 0; r0 < R; r0 += FLY_RB) {
@@ -913,7 +1042,7 @@ static void install_tree(beep_hip_ctx* ctx, int L, const int* leaf_ptr, const in
     ctx->fly_work.upload(fwork.data(), fwork.size(), s);
     ctx->fly_groups.upload(fgroups.data(), fgroups.size(), s);
     ctx->fly_group_nblk.upload(fgnb.data(), fgnb.size(), s);
-    ctx->spmv_part.alloc(std::max(work.size() * 256, fwork.size() * FLY_RB) * 2);
+    ctx->spmv_part.alloc(std::max(work.size() * shape.rows, fwork.size() * FLY_RB) * 2);
     hip_check(hipStreamSynchronize(s), "sync tree upload");
     ctx->L = L;
     ctx->nnz = off[L];
@@ -923,6 +1052,8 @@ static void install_tree(beep_hip_ctx* ctx, int L, const int* leaf_ptr, const in
     ctx->spmv.groups = ctx->spmv_groups.p;
     ctx->spmv.group_nblk = ctx->spmv_group_nblk.p;
     ctx->spmv.n_groups = int(groups.size());
+    ctx->spmv.pstride = shape.rows;
+    ctx->spmv_rows_large = rows_large;
     ctx->fly = SpmvPlan{};
     ctx->fly.work = ctx->fly_work.p;
     ctx->fly.n_work = int(fwork.size());
@@ -960,6 +1091,18 @@ int beep_hip_set_tree(beep_hip_ctx* ctx, const beep_hip_tree* t) {
         ctx->leaf_idx.upload(t->leaf_idx, N, s);
         ctx->nb_idx.upload(t->nb_idx, nnb, s);
         install_tree(ctx, L, t->leaf_ptr, t->nb_ptr);
+        // every neighbourhood lists every patch once (an octree's
+        // neighbourhoods hold no patch twice; a caller's lists might)
+        ctx->all_explicit = ctx->nnz == int64_t(N) * N;
+        std::vector<int> last(ctx->all_explicit ? N : 0, -1);
+        for (int l = 0; l < L && ctx->all_explicit; ++l) {
+            ctx->all_explicit = t->nb_ptr[l + 1] - t->nb_ptr[l] == N;
+            for (int k = t->nb_ptr[l]; k < t->nb_ptr[l + 1] && ctx->all_explicit; ++k) {
+                int& seen_in = last[t->nb_idx[k]];
+                ctx->all_explicit = seen_in != l;
+                seen_in = l;
+            }
+        }
     });
 }
 
@@ -1047,6 +1190,7 @@ int beep_hip_build_tree(beep_hip_ctx* ctx, const double* centre, double edge, in
         launch_gather_segments(s, int(segl.size()), dsegl.p, S.p, ctx->leaf_idx.p);
         launch_gather_segments(s, int(segn.size()), dsegn.p, S.p, ctx->nb_idx.p);
         install_tree(ctx, L, leaf_ptr.data(), nb_ptr.data());  // synchronises the stream
+        ctx->all_explicit = ctx->nnz == int64_t(N) * N;  // boxes of one level are disjoint
         if (n_leaves) *n_leaves = L;
         if (n_nb) *n_nb = nb_ptr[L];
     });
@@ -1136,7 +1280,8 @@ void precompute_impl(beep_hip_ctx* ctx, double kappa, int precision) {
                     ctx->guard_max, gcnt + 3, ctx->diag.p);
     ctx->have_diag = true;
     const unsigned* cellkey = nullptr;
-    unsigned long long uid = 0;
+    const int sub_1pt = fold_next(ctx, precision) ? 0 : 1;
+    unsigned long long uid = sub_1pt ? 0 : beep_hip_ctx::UID_FOLDED;
     if (ctx->use_fmm) {
         // the leaf level and cell keys first (the rest of the plan is built on
         // the host while the coefficient kernel runs, below)
@@ -1175,7 +1320,7 @@ void precompute_impl(beep_hip_ctx* ctx, double kappa, int precision) {
         launch_near_coeffs_fp64(s, ctx->n_coef_blocks, ctx->L, ctx->coef_blk.p, ctx->leaf_ptr.p,
                                 ctx->leaf_idx.p, ctx->nb_ptr.p, ctx->nb_idx.p, ctx->coef_off.p,
                                 ctx->patches.p, ctx->qual_ptr.p, ctx->qual64.p, ctx->quad_ptr.p,
-                                ctx->quad64.p, kappa, 1, cellkey, guard, ctx->guard_max,
+                                ctx->quad64.p, kappa, sub_1pt, cellkey, guard, ctx->guard_max,
                                 ctx->coef64.p);
         launch_coef_repair(s, 0, guard, ctx->patches.p, ctx->qual_ptr.p, ctx->qual64.p,
                            ctx->quad_ptr.p, ctx->quad64.p, kappa, ctx->guard_max, gcnt + 1,
@@ -1202,7 +1347,7 @@ void precompute_impl(beep_hip_ctx* ctx, double kappa, int precision) {
         launch_near_coeffs_fp32(s, ctx->n_coef_blocks, ctx->L, ctx->coef_blk.p, ctx->leaf_ptr.p,
                                 ctx->leaf_idx.p, ctx->nb_ptr.p, ctx->nb_idx.p, ctx->coef_off.p,
                                 ctx->patches.p, ctx->qual_ptr.p, ctx->qual32.p, ctx->quad_ptr.p,
-                                ctx->quad32.p, float(kappa), 1, cellkey, ns, guard,
+                                ctx->quad32.p, float(kappa), sub_1pt, cellkey, ns, guard,
                                 ctx->guard_max, ctx->coef32.p);
         launch_near_fix64(s, ns, ctx->patches.p, ctx->qual_ptr.p, ctx->qual64.p, ctx->quad_ptr.p,
                           ctx->quad64.p, kappa, ctx->guard_max, gcnt + 2, ctx->coef32.p);
@@ -1270,6 +1415,17 @@ void share_common(beep_hip_ctx* ctx, beep_hip_ctx* src, int n_copies, const int*
             "a shared near field needs stored coefficients (near mode BEEP_NEAR_PRECOMPUTE)");
     require(src->have_geom && src->have_tree && src->have_diag && (src->have32 || src->have64),
             "the shared context must have its geometry, tree and coefficients");
+    {
+        // a folded source (no far field of its own) stores full - 1 point from
+        // now on; the first sharer recomputes its sets, the others wait here
+        std::lock_guard<std::mutex> lk(src->share_mu);
+        src->keep_1pt = true;
+        if (src->have64 && folded(src, BEEP_FP64)) {
+            set_device(src);
+            precompute_impl(src, src->kappa, BEEP_FP64);
+            sync_streams(src);
+        }
+    }
     require(src->uid32 == 0 && src->uid64 == 0,
             "the shared coefficients must be precomputed with the direct far field");
     require(n_copies >= 1 && copy_offset, "no copies");
@@ -1304,7 +1460,7 @@ void share_common(beep_hip_ctx* ctx, beep_hip_ctx* src, int n_copies, const int*
     for (int k = 0; k < n_copies; ++k)
         for (int q = 0; q < Ns; ++q) order.push_back(src_order[q] + copy_offset[k]);
     ctx->leaf_idx.upload(order.data(), order.size(), s);
-    ctx->spmv_part.alloc(size_t(2) * src->spmv.n_work * 256 * 2);  // two copies per pass
+    ctx->spmv_part.alloc(size_t(2) * src->spmv.n_work * src->spmv.pstride * 2);  // two copies per pass
     ctx->guard_rec.alloc(beep_hip_ctx::GUARD_CAP);
     hip_check(hipStreamSynchronize(s), "sync share");  // host arrays die here
 }
@@ -1505,15 +1661,14 @@ int beep_hip_sanity_check(beep_hip_ctx* ctx, long long* repaired) {
             // on the fly, the mat-vec guards every entry it integrates
             if (ctx->near_mode != BEEP_NEAR_PRECOMPUTE) continue;
             if (!(fp32 ? ctx->have32 : ctx->have64)) continue;
-            const unsigned long long built = fp32 ? ctx->uid32 : ctx->uid64;
-            require(ctx->use_fmm ? (ctx->fmm && ctx->fmm->uid == built) : built == 0,
+            require(coef_plan_ok(ctx, fp32 ? BEEP_FP32 : BEEP_FP64),
                     "near coefficients were precomputed for another far field: call "
                     "beep_hip_precompute again");
             const unsigned* cellkey = ctx->use_fmm ? ctx->fmm->cellkey : nullptr;
             void* coef = fp32 ? static_cast<void*>(ctx->coef32.p) : static_cast<void*>(ctx->coef64.p);
             launch_coef_scan(s, fp32, ctx->n_coef_blocks, ctx->L, ctx->coef_blk.p, ctx->leaf_ptr.p,
                              ctx->leaf_idx.p, ctx->nb_ptr.p, ctx->nb_idx.p, ctx->coef_off.p, cellkey,
-                             1, coef, ctx->guard_max, guard);
+                             folded(ctx, fp32 ? BEEP_FP32 : BEEP_FP64) ? 0 : 1, coef, ctx->guard_max, guard);
             launch_coef_repair(s, fp32, guard, ctx->patches.p, ctx->qual_ptr.p, ctx->qual64.p,
                                ctx->quad_ptr.p, ctx->quad64.p, ctx->kappa, ctx->guard_max, gcnt + 4,
                                coef);
@@ -1611,12 +1766,12 @@ int beep_hip_matvec_device_noalloc(beep_hip_ctx* ctx, const double* dx, double* 
                 "unknown precision");
         require(precision == BEEP_FP64 ? ctx->have64 : ctx->have32, "coefficients not precomputed");
         require(!ctx->use_fmm, "the allocation-free mat-vec runs with the direct far field only");
-        require((precision == BEEP_FP64 ? ctx->uid64 : ctx->uid32) == 0,
+        require(coef_plan_ok(ctx, precision),
                 "near coefficients were precomputed for another far field: call "
                 "beep_hip_precompute again");
         require(ctx->scratch != nullptr, "no scratch address for this device");
-        // carve the scratch array: sources, far vector, far partial sums,
-        // SpMV row partials (256-byte aligned pieces)
+        // the size it answers for: sources, far vector and partial sums of
+        // the one-directional far field, SpMV partials of 256-row items
         const int N = ctx->N, n2 = 2 * N;
         const int ns = far_direct_splits(N, ctx->n_cu);
         auto up = [](size_t b) { return (b + 255) / 256 * 256; };
@@ -1624,36 +1779,54 @@ int beep_hip_matvec_device_noalloc(beep_hip_ctx* ctx, const double* dx, double* 
         const size_t b_yfar = up(sizeof(double) * size_t(n2));
         const size_t b_part = ns > 1 ? up(sizeof(double) * size_t(n2) * ns) : 0;
         const bool fly = ctx->near_mode == BEEP_NEAR_ON_THE_FLY;
-        const size_t b_spmv = up(sizeof(double) * (fly ? size_t(ctx->fly.n_work) * FLY_RB
-                                                        : size_t(ctx->spmv.n_work) * 256) * 2);
-        const size_t need = b_src + b_yfar + b_part + b_spmv;
-        if (need > SCRATCH_BYTES)
+        const size_t fly_rows = size_t(ctx->fly.n_work) * FLY_RB;
+        const size_t need =
+            b_src + b_yfar + b_part + up(sizeof(double) * (fly ? fly_rows : size_t(ctx->spmv_rows_large)) * 2);
+        if (need > SCRATCH_LIMIT)
             throw std::runtime_error("the allocation-free mat-vec needs " + std::to_string(need) +
                                      " bytes of scratch for " + std::to_string(N) +
-                                     " patches; its limit is " + std::to_string(SCRATCH_BYTES));
+                                     " patches; its limit is " + std::to_string(SCRATCH_LIMIT));
+        const bool fold = folded(ctx, precision), sym = far_is_sym(ctx);
+        const int far32 = precision == BEEP_FP32 ? 1 : 0;
+        const size_t b_spmv =
+            up(sizeof(double) * (fly ? fly_rows : size_t(ctx->spmv.n_work) * ctx->spmv.pstride) * 2);
+        const size_t b_far = fold ? 0 : (sym ? up(sizeof(double) * far_sym_values(N)) : b_src + b_yfar + b_part);
+        require(b_spmv + b_far <= SCRATCH_BYTES, "allocation-free mat-vec: scratch layout");
         set_device(ctx);
         unsigned char* base = static_cast<unsigned char*>(ctx->scratch);
-        Src64* src = reinterpret_cast<Src64*>(base);
-        double* yfar = reinterpret_cast<double*>(base + b_src);
-        double* part = ns > 1 ? reinterpret_cast<double*>(base + b_src + b_yfar) : nullptr;
-        double* spart = reinterpret_cast<double*>(base + b_src + b_yfar + b_part);
+        double* spart = reinterpret_cast<double*>(base);
+        unsigned char* far = base + b_spmv;
+        Src64* src = reinterpret_cast<Src64*>(far);
+        double* yfar = reinterpret_cast<double*>(far + b_src);
+        double* part = ns > 1 ? reinterpret_cast<double*>(far + b_src + b_yfar) : nullptr;
         hipStream_t s = ctx->stream;
         // the kernels of matvec_dev with the direct far field, in its order,
         // all on the context stream
         const int mode = spmv_mode(precision);
+        if (sym && !fold && !fly) {
+            launch_direct_matvec(s, mode, N, ctx->spmv, ctx->leaf_ptr.p, ctx->leaf_idx.p, ctx->nb_ptr.p,
+                                 ctx->nb_idx.p, ctx->coef_off.p, ctx->coef32.p, ctx->coef64.p, ctx->diag.p,
+                                 ctx->patches.p, ctx->kappa, dx, spart, far, dy);
+            return;
+        }
         if (fly)
             launch_near_fly(s, mode, N, ctx->fly, ctx->leaf_ptr.p, ctx->leaf_idx.p, ctx->nb_ptr.p,
                             ctx->nb_idx.p, ctx->patches.p, ctx->qual_ptr.p, ctx->qual32.p, ctx->qual64.p,
-                            ctx->quad_ptr.p, ctx->quad32.p, ctx->quad64.p, ctx->kappa, nullptr,
+                            ctx->quad_ptr.p, ctx->quad32.p, ctx->quad64.p, ctx->kappa, fold ? 0 : 1, nullptr,
                             ctx->fly_ns64 ? 1 : 0, ctx->guard_max, ctx->diag.p, dx, spart, dy);
         else
             launch_near_spmv(s, mode, N, ctx->spmv, ctx->leaf_ptr.p, ctx->leaf_idx.p, ctx->nb_ptr.p,
                              ctx->nb_idx.p, ctx->coef_off.p, ctx->coef32.p, ctx->coef64.p, ctx->diag.p,
-                             dx, spart, dy, ctx->spmv_cap[mode] * ctx->n_cu, ctx->spmv_depth[mode]);
+                             dx, spart, dy, spmv_blocks(ctx, mode), ctx->spmv_depth[mode]);
+        if (fold) return;
+        if (sym) {
+            launch_far_sym(s, far32, N, ctx->leaf_idx.p, ctx->patches.p, dx, ctx->kappa, far);
+            launch_far_sym_add(s, far32, N, ctx->leaf_idx.p, far, dy);
+            return;
+        }
         launch_fill(s, n2, 0.0, yfar);
         launch_far_pack(s, N, ctx->patches.p, ctx->leaf_idx.p, dx, src);
-        launch_far_direct(s, precision == BEEP_FP32 ? 1 : 0, N, ns, ctx->leaf_idx.p, ctx->patches.p,
-                          src, ctx->kappa, yfar, part);
+        launch_far_direct(s, far32, N, ns, ctx->leaf_idx.p, ctx->patches.p, src, ctx->kappa, yfar, part);
         launch_axpby(s, n2, 1.0, yfar, 1.0, dy);
     });
 }

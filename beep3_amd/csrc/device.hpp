@@ -174,9 +174,10 @@ void launch_near_coeffs_fp64(hipStream_t s, int n_blocks, int n_leaves, const in
                              double2* coef);
 
 // Work decomposition of the near-field SpMV (built on the host from the
-// tree): work items (leaf, first row, first column, columns) of <= 256 rows x
-// <= SPMV_CW columns, and row groups (leaf, first row, rows, first work item)
-// with their work-item counts.
+// tree): work items (leaf, first row, first column, columns + rows << 16) of
+// <= 256 rows x <= SPMV_CW columns, and row groups (leaf, first row, rows,
+// first work item) with their work-item counts; the partials of consecutive
+// items are pstride rows apart.
 constexpr int SPMV_CW = 512;
 // rows per work item of the on-the-fly near field (launch_near_fly)
 constexpr int FLY_RB = 64;
@@ -186,15 +187,16 @@ struct SpmvPlan {
     const int4* groups = nullptr;
     const int* group_nblk = nullptr;
     int n_groups = 0;
+    int pstride = 256;
 };
 // y = near(x) + diag(x), overwriting y.  mode: 0 FP64 coef/FP64 sums,
 // 1 FP32 coef/FP32 sums, 2 FP32 coef/FP64 sums.  part: scratch of
-// n_work * 256 * 2 doubles.  max_blocks > 0 caps the grid (blocks then walk
+// n_work * pstride * 2 doubles.  max_blocks > 0 caps the grid (blocks then walk
 // the work items with a grid stride); depth (1, 2, 4) scales the coefficient
 // loads each thread keeps in flight.
 // ncopies (1 or 2) copies of the near field at patch offsets copy_offset
 // (null: 0) share one pass over the coefficients; part then holds ncopies x
-// n_work * 256 * 2 values.
+// n_work * pstride * 2 values.
 void launch_near_spmv(hipStream_t s, int mode, int n, const SpmvPlan& p, const int* leaf_ptr,
                       const int* leaf_idx, const int* nb_ptr, const int* nb_idx,
                       const int64_t* coef_off, const float4* coef32, const double2* coef64,
@@ -202,12 +204,13 @@ void launch_near_spmv(hipStream_t s, int mode, int n, const SpmvPlan& p, const i
                       int max_blocks, int depth, int ncopies = 1, const int* copy_offset = nullptr);
 // The same product with every explicit pair integrated on the fly (no
 // coefficients stored), over a plan of row groups of <= FLY_RB rows; part
-// holds 2 * FLY_RB values per work item.  cellkey: the FMM leaf cells (null
-// with the direct far field); ns64: FP32 near-singular pairs in FP64.
+// holds 2 * FLY_RB values per work item.  subtract_1pt: pairs give full - 1
+// point, except those of adjacent FMM leaf cells (cellkey; null with the
+// direct far field); ns64: FP32 near-singular pairs in FP64.
 void launch_near_fly(hipStream_t s, int mode, int n, const SpmvPlan& p, const int* leaf_ptr,
                      const int* leaf_idx, const int* nb_ptr, const int* nb_idx, const Patch64* patches,
                      const int* qual_ptr, const Pt32* qual32, const Pt64* qual64, const int* quad_ptr,
-                     const Pt32* quad32, const Pt64* quad64, double kappa, const unsigned* cellkey,
+                     const Pt32* quad32, const Pt64* quad64, double kappa, int subtract_1pt, const unsigned* cellkey,
                      int ns64, double maxv, const double* diag4, const double* x, void* part, double* y);
 
 // explicit pairs listed one by one: coefficients (FP64, rounded to FP32 as
@@ -238,6 +241,28 @@ void launch_far_pack(hipStream_t s, int n, const Patch64* patches, const int* or
                      const double* x, Src64* src);
 // source-run splits of the direct far field that fill the chip (n_cu CUs)
 int far_direct_splits(int n, int n_cu);
+// The direct far field over symmetric tile pairs (far_sym.hpp), up to
+// FAR_SYM_MAX patches: its partial sums are (nseg + npj) * 2 n values of the
+// far field's precision.
+constexpr int FAR_SYM_MAX = 20480;
+struct FarSymShape {
+    int nsup = 0, G = 1, nseg = 0, npj = 0;
+};
+FarSymShape far_sym_plan(int n);
+inline size_t far_sym_values(int n) {
+    const FarSymShape s = far_sym_plan(n);
+    return size_t(s.nseg + s.npj) * 2 * size_t(n);
+}
+// part = the far field's partial sums from x; then y += them
+void launch_far_sym(hipStream_t s, int fp32, int n, const int* order, const Patch64* patches, const double* x,
+                    double kappa, void* part);
+void launch_far_sym_add(hipStream_t s, int fp32, int n, const int* order, const void* part, double* y);
+// y = near(x) + diag(x) + direct far field(x) in two launches (modes as
+// launch_near_spmv; part as there, far_part far_sym_values(n) doubles)
+void launch_direct_matvec(hipStream_t s, int mode, int n, const SpmvPlan& p, const int* leaf_ptr,
+                          const int* leaf_idx, const int* nb_ptr, const int* nb_idx, const int64_t* coef_off,
+                          const float4* coef32, const double2* coef64, const double* diag4, const Patch64* patches,
+                          double kappa, const double* x, void* part, void* far_part, double* y);
 // y += direct far field; n_split > 1 needs part: 2 n n_split doubles
 void launch_far_direct(hipStream_t s, int fp32, int n, int n_split, const int* order,
                        const Patch64* patches, const Src64* src, double kappa, double* y,

@@ -21,6 +21,7 @@
 #include <stdexcept>
 
 #include "device.hpp"
+#include "far_sym.hpp"
 
 namespace beepdev {
 
@@ -68,6 +69,8 @@ struct alignas(16) SrcT {
     T dx, dy, dz, sh;
 };
 
+// One-directional tiles, above FAR_SYM_MAX patches (below, the symmetric tile
+// pairs of far_sym.hpp, whose partial sums grow as n^2).
 // Targets and sources both in leaf order (spatially compact runs); positions
 // are taken relative to the first target of the block, formed in FP64, so
 // that nearby pairs keep their relative accuracy in FP32.  A block covers 256
@@ -190,6 +193,56 @@ void launch_far_direct(hipStream_t s, int fp32, int n, int n_split, const int* o
                            n_split, part, y);
         hip_check(hipGetLastError(), "k_far_direct_sum launch");
     }
+}
+
+FarSymShape far_sym_plan(int n) { return far_sym_shape(n); }
+
+// The symmetric tile pairs as a launch of their own (a near field on the fly
+// or shared, or the streams not overlapped; else k_direct_part).
+template <typename T>
+__global__ __launch_bounds__(256) void k_far_sym(FarSymShape fs, int n, const int* __restrict__ order,
+                                                const Patch64* __restrict__ patches, const double* __restrict__ x,
+                                                T kappa, T* __restrict__ part) {
+    __shared__ FarSymLds<T> sm;
+    far_sym_block<T>(sm, blockIdx.x, fs, n, order, patches, x, kappa, part);
+}
+
+template <typename T>
+__global__ __launch_bounds__(64) void k_far_sym_add(FarSymShape fs, int n, const int* __restrict__ order,
+                                                   const T* __restrict__ part, double* __restrict__ y) {
+    const int t = blockIdx.x * 64 + threadIdx.x;
+    if (t >= n) return;
+    double f, h;
+    far_sym_row(fs, n, t, part, f, h);
+    const int i = order[t];
+    y[i] = fma(f, FOUR_PI_INV, y[i]);
+    y[n + i] = fma(h, FOUR_PI_INV, y[n + i]);
+}
+
+void launch_far_sym(hipStream_t s, int fp32, int n, const int* order, const Patch64* patches, const double* x,
+                    double kappa, void* part) {
+    if (n <= 0) return;
+    const FarSymShape fs = far_sym_shape(n);
+    const dim3 grid(unsigned(fs.nsup * fs.nseg));
+    if (fp32)
+        hipLaunchKernelGGL(k_far_sym<float>, grid, dim3(256), 0, s, fs, n, order, patches, x, float(kappa),
+                           static_cast<float*>(part));
+    else
+        hipLaunchKernelGGL(k_far_sym<double>, grid, dim3(256), 0, s, fs, n, order, patches, x, kappa,
+                           static_cast<double*>(part));
+    hip_check(hipGetLastError(), "k_far_sym launch");
+}
+
+void launch_far_sym_add(hipStream_t s, int fp32, int n, const int* order, const void* part, double* y) {
+    if (n <= 0) return;
+    const FarSymShape fs = far_sym_shape(n);
+    const dim3 grid(unsigned((n + 63) / 64));
+    if (fp32)
+        hipLaunchKernelGGL(k_far_sym_add<float>, grid, dim3(64), 0, s, fs, n, order, static_cast<const float*>(part), y);
+    else
+        hipLaunchKernelGGL(k_far_sym_add<double>, grid, dim3(64), 0, s, fs, n, order, static_cast<const double*>(part),
+                           y);
+    hip_check(hipGetLastError(), "k_far_sym_add launch");
 }
 
 }  // namespace beepdev

@@ -17,6 +17,7 @@
 #include <hipcub/hipcub.hpp>
 
 #include "device.hpp"
+#include "far_sym.hpp"
 
 namespace beepdev {
 
@@ -472,7 +473,8 @@ void launch_near_coeffs_fp64(hipStream_t s, int n_blocks, int n_leaves, const in
 // (LocalIntegrations::evaluate_local_contributions, local_integrations.h:123-130).
 //
 // Pass 1: a block handles one work item = (leaf, group of <= 256 rows, run of
-// <= SPMV_CW columns), so blocks carry similar byte counts.  The x values of
+// <= SPMV_CW columns), so blocks carry similar byte counts (spmv_shape: fewer
+// rows and columns per item where the matrix is small).  The x values of
 // its columns are gathered into LDS; thread (r, s) walks columns s, s+S, ...
 // of row r, so each step of the block reads one contiguous run of
 // coefficients, U steps in flight per thread.  Partial row sums go to a
@@ -504,29 +506,29 @@ __device__ __forceinline__ Coef4<TC> load_coef(const void* __restrict__ coef, in
 // NC copies of the same near field (instances of one mesh in a pose): copy q
 // reads x and writes y at patch offset xoff[q] (f and h halves still n
 // apart), so the coefficients are read once for all copies.  NC = 1 is the
-// plain mat-vec.  Partials of copy q: part + q * n_work * 512.
+// plain mat-vec.  Partials of copy q: part + q * n_work * 2 * pstride.
 struct CopyOffsets {
     int off[2];
 };
 
+template <typename TA, int NC>
+struct SpmvLds {
+    TA xs[NC][2][SPMV_CW];
+    TA red[NC][2][256];
+};
+
+// one work item of the SpMV, by a block of 256 threads
 template <typename TC, typename TA, int U, int NC>
-__global__ __launch_bounds__(256) void k_near_spmv_part(
-    const int4* __restrict__ work, int n_work, const int* __restrict__ leaf_ptr,
-    const int* __restrict__ nb_ptr, const int* __restrict__ nb_idx,
-    const int64_t* __restrict__ coef_off, const void* __restrict__ coef,
-    const double* __restrict__ x, CopyOffsets co, int n, TA* __restrict__ part) {
-    __shared__ TA xs[NC][2][SPMV_CW];
-    __shared__ TA red[NC][2][256];
-    // with fewer blocks than work items (a residency cap that leaves room on
-    // every CU for the far-field kernels of the other stream) a block walks
-    // the work items with a grid stride
-    for (int wi = blockIdx.x; wi < n_work; wi += gridDim.x) {
-    __syncthreads();  // xs / red of the previous item consumed
-    const int4 w = work[wi];  // leaf, first row, first column, columns
-    const int L = w.x, row0 = w.y, col0 = w.z, nc = w.w;
+__device__ __forceinline__ void spmv_item(SpmvLds<TA, NC>& sm, int wi, const int4* __restrict__ work, int n_work,
+                                          const int* __restrict__ leaf_ptr, const int* __restrict__ nb_ptr,
+                                          const int* __restrict__ nb_idx, const int64_t* __restrict__ coef_off,
+                                          const void* __restrict__ coef, const double* __restrict__ x,
+                                          CopyOffsets co, int n, int pstride, TA* __restrict__ part) {
+    const int4 w = work[wi];  // leaf, first row, first column, columns + rows << 16
+    const int L = w.x, row0 = w.y, col0 = w.z, nc = w.w & 0xffff;
     const int R = leaf_ptr[L + 1] - leaf_ptr[L];
     const int np = nb_ptr[L];
-    const int Rb = min(256, R - row0);
+    const int Rb = w.w >> 16;
     const int S = 256 / Rb;
     const int t = threadIdx.x;
     const int r = t % Rb, s = t / Rb;
@@ -535,8 +537,8 @@ __global__ __launch_bounds__(256) void k_near_spmv_part(
         const int j = nb_idx[np + col0 + k];
 #pragma unroll
         for (int q = 0; q < NC; ++q) {
-            xs[q][0][k] = TA(x[co.off[q] + j]);
-            xs[q][1][k] = TA(x[co.off[q] + n + j]);
+            sm.xs[q][0][k] = TA(x[co.off[q] + j]);
+            sm.xs[q][1][k] = TA(x[co.off[q] + n + j]);
         }
     }
     __syncthreads();
@@ -558,7 +560,7 @@ __global__ __launch_bounds__(256) void k_near_spmv_part(
             for (int u = 0; u < U; ++u) {
 #pragma unroll
                 for (int q = 0; q < NC; ++q) {
-                    const TA xf = xs[q][0][c + u * S], xh = xs[q][1][c + u * S];
+                    const TA xf = sm.xs[q][0][c + u * S], xh = sm.xs[q][1][c + u * S];
                     af[q] += TA(v[u].b) * xf - TA(v[u].a) * xh;
                     ah[q] += TA(v[u].d) * xf - TA(v[u].c) * xh;
                 }
@@ -568,7 +570,7 @@ __global__ __launch_bounds__(256) void k_near_spmv_part(
             const Coef4<TC> v = load_coef<TC>(coef, base + int64_t(c) * R);
 #pragma unroll
             for (int q = 0; q < NC; ++q) {
-                const TA xf = xs[q][0][c], xh = xs[q][1][c];
+                const TA xf = sm.xs[q][0][c], xh = sm.xs[q][1][c];
                 af[q] += TA(v.b) * xf - TA(v.a) * xh;
                 ah[q] += TA(v.d) * xf - TA(v.c) * xh;
             }
@@ -576,8 +578,8 @@ __global__ __launch_bounds__(256) void k_near_spmv_part(
     }
 #pragma unroll
     for (int q = 0; q < NC; ++q) {
-        red[q][0][t] = af[q];
-        red[q][1][t] = ah[q];
+        sm.red[q][0][t] = af[q];
+        sm.red[q][1][t] = ah[q];
     }
     __syncthreads();
     if (active && s == 0) {
@@ -585,19 +587,75 @@ __global__ __launch_bounds__(256) void k_near_spmv_part(
         for (int q = 0; q < NC; ++q) {
             TA f = af[q], h = ah[q];
             for (int k = 1; k < S; ++k) {
-                f += red[q][0][k * Rb + r];
-                h += red[q][1][k * Rb + r];
+                f += sm.red[q][0][k * Rb + r];
+                h += sm.red[q][1][k * Rb + r];
             }
-            TA* pq = part + size_t(q) * n_work * 512;
-            pq[2 * (size_t(wi) * 256 + r)] = f;
-            pq[2 * (size_t(wi) * 256 + r) + 1] = h;
+            TA* pq = part + size_t(q) * n_work * 2 * pstride;
+            pq[2 * (size_t(wi) * pstride + r)] = f;
+            pq[2 * (size_t(wi) * pstride + r) + 1] = h;
         }
     }
+}
+
+template <typename TC, typename TA, int U, int NC>
+__global__ __launch_bounds__(256) void k_near_spmv_part(
+    const int4* __restrict__ work, int n_work, const int* __restrict__ leaf_ptr,
+    const int* __restrict__ nb_ptr, const int* __restrict__ nb_idx,
+    const int64_t* __restrict__ coef_off, const void* __restrict__ coef,
+    const double* __restrict__ x, CopyOffsets co, int n, int pstride, TA* __restrict__ part) {
+    __shared__ SpmvLds<TA, NC> sm;
+    // with fewer blocks than work items (a residency cap that leaves room on
+    // every CU for the far-field kernels of the other stream) a block walks
+    // the work items with a grid stride
+    for (int wi = blockIdx.x; wi < n_work; wi += gridDim.x) {
+        __syncthreads();  // LDS of the previous item consumed
+        spmv_item<TC, TA, U, NC>(sm, wi, work, n_work, leaf_ptr, nb_ptr, nb_idx, coef_off, coef, x, co, n,
+                                 pstride, part);
     }
 }
 
 // grid (row groups, copies); a work item's partials are pstride rows apart
-// (256 for the SpMV, FLY_RB for the on-the-fly pass)
+// (the SpMV plan's, FLY_RB for the on-the-fly pass).  The block's 256 threads
+// are 256 / rows lanes per row: lane s adds the partials s, s + S, ... and the
+// lanes are added in order, so a row of many short items (small matrices)
+// does not wait on one chain of loads.
+template <typename TA>
+__device__ __forceinline__ int near_row_sum(int4 g, int nb, const int* __restrict__ leaf_ptr,
+                                            const int* __restrict__ leaf_idx, const double* __restrict__ diag4,
+                                            const double* __restrict__ x, int off, int n, int pstride,
+                                            const TA* __restrict__ pq, double& vf, double& vh) {
+    __shared__ TA red[2][256];
+    const int t = threadIdx.x;
+    const int S = min(256 / g.z, nb);
+    const int r = t % g.z, s = t / g.z;
+    TA af = 0, ah = 0;
+    if (s < S) {
+#pragma unroll 4
+        for (int k = s; k < nb; k += S) {
+            const size_t q = 2 * (size_t(g.w + k) * pstride + r);
+            af += pq[q];
+            ah += pq[q + 1];
+        }
+    }
+    if (S > 1) {  // uniform over the block
+        red[0][t] = af;
+        red[1][t] = ah;
+        __syncthreads();
+        if (s == 0)
+            for (int k = 1; k < S; ++k) {
+                af += red[0][k * g.z + r];
+                ah += red[1][k * g.z + r];
+            }
+    }
+    if (s > 0) return -1;
+    const int i = leaf_idx[leaf_ptr[g.x] + g.y + r];
+    const double* d = diag4 + 4 * size_t(i);
+    const double xf = x[off + i], xh = x[off + n + i];
+    vf = double(af) + (d[1] * xf - d[0] * xh);
+    vh = double(ah) + (d[3] * xf - d[2] * xh);
+    return i;
+}
+
 template <typename TA>
 __global__ __launch_bounds__(256) void k_near_spmv_sum(
     const int4* __restrict__ groups, const int* __restrict__ group_nblk,
@@ -605,22 +663,13 @@ __global__ __launch_bounds__(256) void k_near_spmv_sum(
     const double* __restrict__ diag4, const double* __restrict__ x, CopyOffsets co, int n, int n_work,
     int pstride, const TA* __restrict__ part, double* __restrict__ y) {
     const int4 g = groups[blockIdx.x];  // leaf, first row, rows, first work block
-    const int nb = group_nblk[blockIdx.x];
-    const int r = threadIdx.x;
-    if (r >= g.z) return;
     const int cq = blockIdx.y, off = co.off[cq];
-    const TA* pq = part + size_t(cq) * n_work * 2 * pstride;
-    TA af = 0, ah = 0;
-    for (int k = 0; k < nb; ++k) {
-        const size_t q = 2 * (size_t(g.w + k) * pstride + r);
-        af += pq[q];
-        ah += pq[q + 1];
-    }
-    const int i = leaf_idx[leaf_ptr[g.x] + g.y + r];
-    const double* d = diag4 + 4 * size_t(i);
-    const double xf = x[off + i], xh = x[off + n + i];
-    y[off + i] = double(af) + (d[1] * xf - d[0] * xh);
-    y[off + n + i] = double(ah) + (d[3] * xf - d[2] * xh);
+    double vf, vh;
+    const int i = near_row_sum(g, group_nblk[blockIdx.x], leaf_ptr, leaf_idx, diag4, x, off, n, pstride,
+                               part + size_t(cq) * n_work * 2 * pstride, vf, vh);
+    if (i < 0) return;
+    y[off + i] = vf;
+    y[off + n + i] = vh;
 }
 
 // Loads in flight per thread: U = 4 * depth (FP64 coefficients) or 8 * depth
@@ -633,10 +682,10 @@ static void spmv_part(hipStream_t s, int grid, const SpmvPlan& p, const int* lea
                       TA* part) {
     if (ncopies == 2)
         hipLaunchKernelGGL((k_near_spmv_part<TC, TA, U, 2>), dim3(grid), dim3(256), 0, s, p.work,
-                           p.n_work, leaf_ptr, nb_ptr, nb_idx, coef_off, coef, x, co, n, part);
+                           p.n_work, leaf_ptr, nb_ptr, nb_idx, coef_off, coef, x, co, n, p.pstride, part);
     else
         hipLaunchKernelGGL((k_near_spmv_part<TC, TA, U, 1>), dim3(grid), dim3(256), 0, s, p.work,
-                           p.n_work, leaf_ptr, nb_ptr, nb_idx, coef_off, coef, x, co, n, part);
+                           p.n_work, leaf_ptr, nb_ptr, nb_idx, coef_off, coef, x, co, n, p.pstride, part);
 }
 
 void launch_near_spmv(hipStream_t s, int mode, int n, const SpmvPlan& p, const int* leaf_ptr,
@@ -659,7 +708,7 @@ void launch_near_spmv(hipStream_t s, int mode, int n, const SpmvPlan& p, const i
                             spmv_part<double, double, 16>};
         f[d](s, grid, p, leaf_ptr, nb_ptr, nb_idx, coef_off, coef64, x, ncopies, co, n, (double*)part);
         hipLaunchKernelGGL((k_near_spmv_sum<double>), sgrid, dim3(256), 0, s, p.groups, p.group_nblk,
-                           leaf_ptr, leaf_idx, diag4, x, co, n, p.n_work, 256, (const double*)part, y);
+                           leaf_ptr, leaf_idx, diag4, x, co, n, p.n_work, p.pstride, (const double*)part, y);
     } else if (mode == 1) {
         using F = void (*)(hipStream_t, int, const SpmvPlan&, const int*, const int*, const int*,
                            const int64_t*, const void*, const double*, int, CopyOffsets, int, float*);
@@ -667,7 +716,7 @@ void launch_near_spmv(hipStream_t s, int mode, int n, const SpmvPlan& p, const i
                             spmv_part<float, float, 32>};
         f[d](s, grid, p, leaf_ptr, nb_ptr, nb_idx, coef_off, coef32, x, ncopies, co, n, (float*)part);
         hipLaunchKernelGGL((k_near_spmv_sum<float>), sgrid, dim3(256), 0, s, p.groups, p.group_nblk,
-                           leaf_ptr, leaf_idx, diag4, x, co, n, p.n_work, 256, (const float*)part, y);
+                           leaf_ptr, leaf_idx, diag4, x, co, n, p.n_work, p.pstride, (const float*)part, y);
     } else {
         using F = void (*)(hipStream_t, int, const SpmvPlan&, const int*, const int*, const int*,
                            const int64_t*, const void*, const double*, int, CopyOffsets, int, double*);
@@ -675,9 +724,96 @@ void launch_near_spmv(hipStream_t s, int mode, int n, const SpmvPlan& p, const i
                             spmv_part<float, double, 32>};
         f[d](s, grid, p, leaf_ptr, nb_ptr, nb_idx, coef_off, coef32, x, ncopies, co, n, (double*)part);
         hipLaunchKernelGGL((k_near_spmv_sum<double>), sgrid, dim3(256), 0, s, p.groups, p.group_nblk,
-                           leaf_ptr, leaf_idx, diag4, x, co, n, p.n_work, 256, (const double*)part, y);
+                           leaf_ptr, leaf_idx, diag4, x, co, n, p.n_work, p.pstride, (const double*)part, y);
     }
     hip_check(hipGetLastError(), "k_near_spmv launch");
+}
+
+// ---------------------------------------------------------------------------
+// The whole mat-vec of a problem with the direct far field (up to
+// FAR_SYM_MAX patches) in two launches: blocks that stream SpMV work items
+// and blocks that sum symmetric far-field tile pairs (far_sym.hpp) side by
+// side, the far ones spread evenly over the grid, so the SpMV's HBM time and
+// the far field's VALU time overlap without a second stream, its fork / join
+// events and the launches of a separate chain (fill, pack, sum, add).  The
+// sums are those of k_near_spmv_part and of the far field alone, so the
+// launches may also be made apart (n_far or n_near 0), for the same bits.
+// Whole mat-vecs against two streams with the one-directional far field:
+// 2,562 patches FP32 130 -> 54 us, 10,242 FP64 457 -> 223 us, 11,304 FP32
+// coefficients with FP64 sums 465 -> 250 us.  Up to FAR_SYM_MAX patches the
+// partial sums (n^2 / 32 values of partner sums, 13 MB at the limit) stay
+// cheap; above, the FMM is the default and the direct sum a reference.
+template <typename TC, typename TA, int U, typename TF>
+__global__ __launch_bounds__(256) void k_direct_part(
+    int n_near, int n_far, const int4* __restrict__ work, const int* __restrict__ leaf_ptr,
+    const int* __restrict__ nb_ptr, const int* __restrict__ nb_idx, const int64_t* __restrict__ coef_off,
+    const void* __restrict__ coef, const double* __restrict__ x, int n, int pstride, TA* __restrict__ part,
+    FarSymShape fs, const int* __restrict__ order, const Patch64* __restrict__ patches, TF kappa,
+    TF* __restrict__ far_part) {
+    union Lds {
+        SpmvLds<TA, 1> near;
+        FarSymLds<TF> far;
+        __device__ Lds() {}
+    };
+    __shared__ Lds sm;
+    const long long b = blockIdx.x, nb = n_near + n_far;
+    const int f0 = int(b * n_far / nb), f1 = int((b + 1) * n_far / nb);
+    if (f1 > f0) {
+        far_sym_block<TF>(sm.far, f0, fs, n, order, patches, x, kappa, far_part);
+    } else {
+        const CopyOffsets co{{0, 0}};
+        spmv_item<TC, TA, U, 1>(sm.near, int(b) - f0, work, n_near, leaf_ptr, nb_ptr, nb_idx, coef_off, coef, x,
+                                co, n, pstride, part);
+    }
+}
+
+// y of the same: near row sums, diagonal and far-field partials of each row
+template <typename TA, typename TF>
+__global__ __launch_bounds__(256) void k_direct_sum(
+    const int4* __restrict__ groups, const int* __restrict__ group_nblk, const int* __restrict__ leaf_ptr,
+    const int* __restrict__ leaf_idx, const double* __restrict__ diag4, const double* __restrict__ x, int n,
+    int pstride, const TA* __restrict__ part, FarSymShape fs, const TF* __restrict__ far_part,
+    double* __restrict__ y) {
+    const int4 g = groups[blockIdx.x];  // leaf, first row, rows, first work block
+    double vf, vh;
+    const int i = near_row_sum(g, group_nblk[blockIdx.x], leaf_ptr, leaf_idx, diag4, x, 0, n, pstride, part, vf, vh);
+    if (i < 0) return;
+    double af, ah;
+    far_sym_row(fs, n, leaf_ptr[g.x] + g.y + int(threadIdx.x), far_part, af, ah);
+    y[i] = fma(af, FOUR_PI_INV, vf);
+    y[n + i] = fma(ah, FOUR_PI_INV, vh);
+}
+
+template <typename TC, typename TA, int U, typename TF>
+static void direct_matvec(hipStream_t s, int n, const SpmvPlan& p, const int* leaf_ptr, const int* leaf_idx,
+                          const int* nb_ptr, const int* nb_idx, const int64_t* coef_off, const void* coef,
+                          const double* diag4, const Patch64* patches, double kappa, const double* x, TA* part,
+                          TF* far_part, double* y) {
+    const FarSymShape fs = far_sym_shape(n);
+    const int n_far = fs.nsup * fs.nseg;
+    hipLaunchKernelGGL((k_direct_part<TC, TA, U, TF>), dim3(unsigned(p.n_work + n_far)), dim3(256), 0, s, p.n_work,
+                       n_far, p.work, leaf_ptr, nb_ptr, nb_idx, coef_off, coef, x, n, p.pstride, part, fs, leaf_idx,
+                       patches, TF(kappa), far_part);
+    hip_check(hipGetLastError(), "k_direct_part launch");
+    hipLaunchKernelGGL((k_direct_sum<TA, TF>), dim3(unsigned(p.n_groups)), dim3(256), 0, s, p.groups, p.group_nblk,
+                       leaf_ptr, leaf_idx, diag4, x, n, p.pstride, (const TA*)part, fs, (const TF*)far_part, y);
+    hip_check(hipGetLastError(), "k_direct_sum launch");
+}
+
+void launch_direct_matvec(hipStream_t s, int mode, int n, const SpmvPlan& p, const int* leaf_ptr,
+                          const int* leaf_idx, const int* nb_ptr, const int* nb_idx, const int64_t* coef_off,
+                          const float4* coef32, const double2* coef64, const double* diag4, const Patch64* patches,
+                          double kappa, const double* x, void* part, void* far_part, double* y) {
+    if (p.n_work <= 0) return;
+    if (mode == 0)
+        direct_matvec<double, double, 4, double>(s, n, p, leaf_ptr, leaf_idx, nb_ptr, nb_idx, coef_off, coef64,
+                                                 diag4, patches, kappa, x, (double*)part, (double*)far_part, y);
+    else if (mode == 1)
+        direct_matvec<float, float, 8, float>(s, n, p, leaf_ptr, leaf_idx, nb_ptr, nb_idx, coef_off, coef32, diag4,
+                                              patches, kappa, x, (float*)part, (float*)far_part, y);
+    else
+        direct_matvec<float, double, 8, double>(s, n, p, leaf_ptr, leaf_idx, nb_ptr, nb_idx, coef_off, coef32,
+                                                diag4, patches, kappa, x, (double*)part, (double*)far_part, y);
 }
 
 // ---------------------------------------------------------------------------
@@ -725,7 +861,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 5) void k_near_fly_part(
     const int* __restrict__ leaf_idx, const int* __restrict__ nb_ptr, const int* __restrict__ nb_idx,
     const Patch64* __restrict__ patches, const int* __restrict__ qual_ptr,
     const Pt<T>* __restrict__ qual, const int* __restrict__ quad_ptr, const Pt<T>* __restrict__ quad,
-    const Pt64* __restrict__ qual64, const Pt64* __restrict__ quad64, double kappa,
+    const Pt64* __restrict__ qual64, const Pt64* __restrict__ quad64, double kappa, int subtract_1pt,
     const unsigned* __restrict__ cellkey, int ns64, double maxv, const double* __restrict__ x, int n,
     TA* __restrict__ part) {
     // FP32 pass: the near-singular pairs of a thread (up to DEF of them) are
@@ -766,7 +902,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 5) void k_near_fly_part(
             if (j == i) continue;  // the self pair is the diagonal's (stored as zero)
             const Patch64 pj = patches[j];
             const int pb = quad_ptr[j], pn = quad_ptr[j + 1] - pb;
-            const int sub = !(cellkey && fmm_cells_adjacent(ki, cellkey[j]));
+            const int sub = subtract_1pt && !(cellkey && fmm_cells_adjacent(ki, cellkey[j]));
             T v[4];
             bool redo = false;
             if constexpr (sizeof(T) == 4) {
@@ -843,12 +979,12 @@ template <typename T, typename TA>
 static void fly_launch(hipStream_t s, const SpmvPlan& p, const int* leaf_ptr, const int* leaf_idx,
                        const int* nb_ptr, const int* nb_idx, const Patch64* patches, const int* qual_ptr,
                        const Pt<T>* qual, const int* quad_ptr, const Pt<T>* quad, const Pt64* qual64,
-                       const Pt64* quad64, double kappa, const unsigned* cellkey, int ns64, double maxv,
-                       const double* diag4, const double* x, int n, TA* part, double* y) {
+                       const Pt64* quad64, double kappa, int subtract_1pt, const unsigned* cellkey, int ns64,
+                       double maxv, const double* diag4, const double* x, int n, TA* part, double* y) {
     auto k = kappa != 0.0 ? k_near_fly_part<T, TA, true> : k_near_fly_part<T, TA, false>;
     hipLaunchKernelGGL(k, dim3(unsigned(p.n_work)), dim3(256), 0, s, p.work, p.n_work, leaf_ptr, leaf_idx,
                        nb_ptr, nb_idx, patches, qual_ptr, qual, quad_ptr, quad, qual64, quad64, kappa,
-                       cellkey, ns64, maxv, x, n, part);
+                       subtract_1pt, cellkey, ns64, maxv, x, n, part);
     hip_check(hipGetLastError(), "k_near_fly_part launch");
     const CopyOffsets co{{0, 0}};
     hipLaunchKernelGGL((k_near_spmv_sum<TA>), dim3(unsigned(p.n_groups), 1u), dim3(256), 0, s, p.groups,
@@ -860,20 +996,20 @@ static void fly_launch(hipStream_t s, const SpmvPlan& p, const int* leaf_ptr, co
 void launch_near_fly(hipStream_t s, int mode, int n, const SpmvPlan& p, const int* leaf_ptr,
                      const int* leaf_idx, const int* nb_ptr, const int* nb_idx, const Patch64* patches,
                      const int* qual_ptr, const Pt32* qual32, const Pt64* qual64, const int* quad_ptr,
-                     const Pt32* quad32, const Pt64* quad64, double kappa, const unsigned* cellkey,
+                     const Pt32* quad32, const Pt64* quad64, double kappa, int subtract_1pt, const unsigned* cellkey,
                      int ns64, double maxv, const double* diag4, const double* x, void* part, double* y) {
     if (p.n_work <= 0) return;
     if (mode == 0)
         fly_launch<double, double>(s, p, leaf_ptr, leaf_idx, nb_ptr, nb_idx, patches, qual_ptr, qual64,
-                                   quad_ptr, quad64, qual64, quad64, kappa, cellkey, 0, maxv, diag4, x, n,
+                                   quad_ptr, quad64, qual64, quad64, kappa, subtract_1pt, cellkey, 0, maxv, diag4, x, n,
                                    (double*)part, y);
     else if (mode == 1)
         fly_launch<float, float>(s, p, leaf_ptr, leaf_idx, nb_ptr, nb_idx, patches, qual_ptr, qual32,
-                                 quad_ptr, quad32, qual64, quad64, kappa, cellkey, ns64, maxv, diag4, x,
+                                 quad_ptr, quad32, qual64, quad64, kappa, subtract_1pt, cellkey, ns64, maxv, diag4, x,
                                  n, (float*)part, y);
     else
         fly_launch<float, double>(s, p, leaf_ptr, leaf_idx, nb_ptr, nb_idx, patches, qual_ptr, qual32,
-                                  quad_ptr, quad32, qual64, quad64, kappa, cellkey, ns64, maxv, diag4, x,
+                                  quad_ptr, quad32, qual64, quad64, kappa, subtract_1pt, cellkey, ns64, maxv, diag4, x,
                                   n, (double*)part, y);
 }
 

@@ -245,9 +245,11 @@ int beep_hip_autotune_leaf(beep_hip_ctx* ctx, int precision, const int* leaf_tar
                            int reps, double* ms_out, int* best);
 
 /* Residency cap of the near-field SpMV: at most blocks_per_cu blocks per
- * compute unit walk the work items (default 1; 0: one block per work item).
- * A cap leaves room on every CU for the far-field kernels that run on the
- * other stream at the same time.  Sets the cap of every precision. */
+ * compute unit walk the work items (0: one block per work item; default: 1
+ * beside an FMM far field, else 0).  A cap leaves room on every CU for the
+ * far-field kernels that run on the other stream at the same time; up to
+ * 20,480 patches with the direct far field both run in one launch, which no
+ * cap applies to.  Sets the cap of every precision. */
 int beep_hip_set_spmv_residency(beep_hip_ctx* ctx, int blocks_per_cu);
 /* Autotuner for that cap: times `reps` whole mat-vecs of the given precision
  * (far field overlapped) for each candidate, writes the mean times to ms_out
@@ -381,9 +383,10 @@ int beep_hip_matvec_device(beep_hip_ctx* ctx, const double* d_x, double* d_y, in
 /* As beep_hip_matvec_device, but allocating nothing: no counterpart in the
  * reference; for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops).  Its scratch (source records, the far
- * vector, partial sums) is a 64 MiB array of the library, one per device,
- * held until the process ends; calls whose scratch would exceed it (with the
- * direct far field, about 100,000 patches) fail with a message, and so do
+ * vector, partial sums) is a 96 MiB array of the library, one per device,
+ * held until the process ends; calls whose sources, far vector and partial
+ * sums would exceed 64 MiB of it (with the direct far field, about 100,000
+ * patches) fail with a message, and so do
  * contexts with an FMM far field.  Every call on a device shares that
  * device's array: calls that overlap in time on one device (two contexts or
  * streams at once) race and must be serialised by the caller.  Stream-ordered

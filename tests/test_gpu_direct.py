@@ -1,0 +1,114 @@
+"""The direct far field as symmetric tile pairs and the FP64 set without a far
+field, against the FP64 CPU oracle, at the edges of the 256- and 64-patch
+tiles and of the SpMV's work items, over every route to them."""
+import numpy as np
+import pytest
+
+import oracle
+from beep3_amd.device import Device
+from beep3_amd.scene import Mesh, Scene
+
+pytestmark = pytest.mark.gpu
+
+
+
+def rel(a, b):
+    return float(np.linalg.norm(a - b) / np.linalg.norm(b))
+
+
+def bounds(orc, x, ref):
+    """Relative error bounds of a mat-vec: FP64 rounding, and for the FP32 set
+    first-order rounding of the products, c u ||K||x|| / |K x| with u = 2^-24:
+    c = 16 roundings to form a coefficient (about ten on its longest chain,
+    more where terms nearly cancel), twice that with FP32 products and sums
+    (at most 16 partial sums deep in blocks)."""
+    u = 2.0 ** -24 * np.linalg.norm(np.abs(orc.assemble()) @ np.abs(x)) / np.linalg.norm(ref)
+    return {"fp64": 1e-12, "fp32": 32 * u, "fp32_resid": 16 * u}
+
+
+def scene(levels, nbsize, kappa=0.125):
+    sc = Scene(80.0, kappa, 6, 0, nbsize)
+    for k, lv in enumerate(levels):
+        sc.add_instance(Mesh.star(lv, 25.0, 8, 0.04, 5 + k), 2.0 + k, offset=[70.0 * k, 3.0 * k, 0.0])
+    return sc.build().arrays()
+
+
+def device(a, far="auto", kappa=0.125, near="precompute", precs=("fp64", "fp32")):
+    d = Device(0)
+    d.set_far_field(far, 5, 40)
+    d.set_geometry(a)
+    d.set_tree(a)
+    d.set_near_mode(near)
+    for p in precs:
+        d.precompute(kappa, p)
+    return d
+
+
+# 42 .. 3,204 patches: one to thirteen super-tiles, odd and even rings, last
+# tiles of 2 .. 42 patches, one leaf and many
+@pytest.mark.parametrize("levels,nbsize", [((1,), 1500), ((2,), 30), ((1, 2, 1), 1500), ((2, 2, 2, 1), 50),
+                                           ((3,), 1500), ((3, 2), 100), ((3, 3, 2), 60), ((4, 3), 200),
+                                           ((4,), 1500)])
+@pytest.mark.parametrize("kappa", [0.125, 0.0])
+def test_direct_matvec_against_oracle(levels, nbsize, kappa):
+    a = scene(levels, nbsize, kappa)
+    n = a["area"].shape[0]
+    x = np.random.default_rng(n).normal(size=2 * n)
+    orc = oracle.Oracle(a, kappa, 80.0)
+    ref = orc.matvec(x)
+    d = device(a, kappa=kappa)
+    for p, tol in bounds(orc, x, ref).items():
+        y = d.matvec(x, p)
+        print(n, nbsize, kappa, p, rel(y, ref), tol, flush=True)
+        assert rel(y, ref) < tol
+        d.set_overlap(False)
+        assert np.array_equal(d.matvec(x, p), y)
+        d.set_overlap(True)
+    # sets made for either form of the direct far field serve both modes
+    d.set_far_field("direct", 5, 40)
+    assert rel(d.matvec(x, "fp64"), ref) < 1e-12
+    d.close()
+
+
+@pytest.mark.parametrize("levels,nbsize", [((3,), 1500), ((3, 2), 100)])
+def test_direct_matvec_on_the_fly(levels, nbsize):
+    a = scene(levels, nbsize)
+    n = a["area"].shape[0]
+    x = np.random.default_rng(n).normal(size=2 * n)
+    orc = oracle.Oracle(a, 0.125, 80.0)
+    ref = orc.matvec(x)
+    d = device(a, near="on_the_fly")
+    for p, tol in bounds(orc, x, ref).items():
+        assert rel(d.matvec(x, p), ref) < tol
+    d.close()
+
+
+def test_shared_near_field_of_a_one_leaf_mesh():
+    """A context whose FP64 set has no far field, then shared: the pose over
+    two copies of it matches the oracle of the scene with the same pairs."""
+    one = scene((3,), 1500)
+    n = one["area"].shape[0]
+    src = device(one)
+    x1 = np.random.default_rng(1).normal(size=2 * n)
+    y1 = src.matvec(x1, "fp64")
+    sc = Scene(80.0, 0.125, 6, 0, 1500)
+    m = Mesh.star(3, 25.0, 8, 0.04, 5)
+    two = sc.add_instance(m, 2.0).add_instance(m, 2.0, offset=[80.0, 0.0, 0.0]).build().arrays()
+    x = np.random.default_rng(2).normal(size=4 * n)
+    pose = Device(0)
+    pose.set_far_field("direct", 5, 40)
+    pose.set_geometry(two)
+    pose.share_near(src, [0, n])
+    lists = dict(two)
+    lists["leaf_ptr"] = np.array([0, n, 2 * n], np.int32)
+    lists["leaf_idx"] = np.arange(2 * n, dtype=np.int32)
+    lists["nb_ptr"] = lists["leaf_ptr"]
+    lists["nb_idx"] = lists["leaf_idx"]
+    orc = oracle.Oracle(lists, 0.125, 80.0)
+    ref = orc.matvec(x)
+    for p, tol in bounds(orc, x, ref).items():
+        pose.precompute(0.125, p)
+        assert rel(pose.matvec(x, p), ref) < tol
+    assert rel(src.matvec(x1, "fp64"), y1) < 1e-12
+    pose.close()
+    src.close()
