@@ -138,6 +138,7 @@ struct beep_hip_ctx {
     DevBuf<int4> spmv_work, spmv_groups;
     DevBuf<int> spmv_group_nblk;
     DevBuf<double> spmv_part;
+    DevBuf<unsigned> spmv_next;  // next free work item of a capped SpMV, zero between launches
     SpmvPlan spmv;
     // the on-the-fly near field: its plan (row groups of <= FLY_RB rows),
     // the mode, and whether its FP32 pass integrates near-singular pairs in
@@ -439,6 +440,20 @@ void far_buffers(beep_hip_ctx* c) {
     if (ns > 1) c->far_part.alloc(size_t(2) * c->N * ns);
 }
 
+// The stream of the FMM's leaf pass (20 to 80 us): the shorter of the two.
+// Estimates from runs of each alone: the SpMV streams 6 TB/s; the Chebyshev far
+// field takes 1.9 (FP64) or 1.1 ns (FP32) per M2L pair at order 5, about as
+// the cube of the order, and half of that again around it.  Not beside the
+// plane waves (longer than their SpMV at every size) or a near field on the
+// fly.  163,842 patches, FP64: the last kernels after the SpMV 100 -> 25 us.
+bool leaf_pass_on_far(const beep_hip_ctx* c, int mode) {
+    if (c->share || c->near_mode != BEEP_NEAR_PRECOMPUTE || c->fmm->engine != 0) return false;
+    const double near_us = double(c->nnz) * (mode == 0 ? 32.0 : 16.0) / 6e6;
+    const double p = c->fmm->P / 5.0;
+    const double far_us = double(c->fmm->n_pairs) * (mode == 1 ? 1.1e-3 : 1.9e-3) * p * p * p * 1.5;
+    return near_us > far_us;
+}
+
 // near-SpMV coefficient mode of a mat-vec precision
 int spmv_mode(int precision) {
     return precision == BEEP_FP64 ? 0 : (precision == BEEP_FP32 ? 1 : 2);
@@ -471,6 +486,7 @@ void matvec_dev(beep_hip_ctx* c, const double* dx, double* dy, int precision) {
     const int far32 = precision == BEEP_FP32 ? 1 : 0;
     const bool fold = folded(c, precision);
     const bool sym = far_is_sym(c);
+    const bool p2p_far = c->use_fmm && leaf_pass_on_far(c, mode);
     if (!c->capturing && !fold) far_buffers(c);
     if (timed) hip_check(hipEventRecord(ev[0], s), "hipEventRecord");
     auto matvec_timed = [&](bool with_m2l) {
@@ -509,7 +525,7 @@ void matvec_dev(beep_hip_ctx* c, const double* dx, double* dy, int precision) {
         for (int k = 0; k < nco; k += 2)
             launch_near_spmv(s, mode, c->N, h->spmv, h->leaf_ptr.p, h->leaf_idx.p, h->nb_ptr.p,
                              h->nb_idx.p, h->coef_off.p, h->coef32.p, h->coef64.p, h->diag.p, dx,
-                             c->spmv_part.p, dy, spmv_blocks(c, mode), c->spmv_depth[mode],
+                             c->spmv_part.p, dy, spmv_blocks(c, mode), c->spmv_depth[mode], c->spmv_next.p,
                              std::min(2, nco - k), c->share_off.data() + k);
         launch_pair_spmv(s, mode, c->N, c->n_pair_rows, c->pair_rows.p, c->pair_ptr.p, c->pair_col.p,
                          c->pcoef32.p, c->pcoef64.p, dx, dy);
@@ -521,7 +537,7 @@ void matvec_dev(beep_hip_ctx* c, const double* dx, double* dy, int precision) {
     } else {
         launch_near_spmv(s, mode, c->N, c->spmv, c->leaf_ptr.p, c->leaf_idx.p, c->nb_ptr.p,
                          c->nb_idx.p, c->coef_off.p, c->coef32.p, c->coef64.p, c->diag.p, dx,
-                         c->spmv_part.p, dy, spmv_blocks(c, mode), c->spmv_depth[mode]);
+                         c->spmv_part.p, dy, spmv_blocks(c, mode), c->spmv_depth[mode], c->spmv_next.p);
     }
     if (timed) hip_check(hipEventRecord(ev[1], s), "hipEventRecord");
     if (fold) {
@@ -535,11 +551,12 @@ void matvec_dev(beep_hip_ctx* c, const double* dx, double* dy, int precision) {
     if (sym) {
         launch_far_sym(sf, far32, c->N, c->leaf_idx.p, c->patches.p, dx, c->kappa, c->far_part.p);
     } else {
-        launch_fill(sf, n2, 0.0, c->yfar.p);
         if (c->use_fmm) {
             fmm_evaluate(c->fmm, sf, far32, c->patches.p, dx, c->kappa, c->yfar.p, timed ? &ev[4] : nullptr,
                          c->ev_pack);
+            if (p2p_far) fmm_p2p(c->fmm, sf, far32, c->patches.p, c->kappa, c->yfar.p);
         } else {
+            launch_fill(sf, n2, 0.0, c->yfar.p);
             launch_far_pack(sf, c->N, c->patches.p, c->leaf_idx.p, dx, c->src.p);
             launch_far_direct(sf, far32, c->N, far_direct_splits(c->N, c->n_cu), c->leaf_idx.p, c->patches.p,
                               c->src.p, c->kappa, c->yfar.p, c->far_part.p);
@@ -547,7 +564,7 @@ void matvec_dev(beep_hip_ctx* c, const double* dx, double* dy, int precision) {
     }
     if (timed) hip_check(hipEventRecord(ev[3], sf), "hipEventRecord");
     if (c->overlap) hip_check(hipEventRecord(c->ev_join, sf), "hipEventRecord");
-    if (c->use_fmm) {
+    if (c->use_fmm && !p2p_far) {
         // the P2P part (VALU) follows the SpMV on this stream, beside the
         // MFMA-bound M2L of the far stream; it needs the packed sources
         if (c->overlap) hip_check(hipStreamWaitEvent(s, c->ev_pack, 0), "hipStreamWaitEvent");
@@ -774,6 +791,8 @@ int beep_hip_create(int device, beep_hip_ctx** out) {
         hip_check(hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, device),
                   "hipDeviceGetAttribute");
         c->scratch = scratch_address(device);
+        c->spmv_next.alloc(1);
+        launch_set_int(c->stream, reinterpret_cast<int*>(c->spmv_next.p), 0);
         hip_check(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming), "hipEventCreate");
         hip_check(hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming), "hipEventCreate");
         hip_check(hipEventCreateWithFlags(&c->ev_pack, hipEventDisableTiming), "hipEventCreate");
@@ -1311,11 +1330,11 @@ void precompute_impl(beep_hip_ctx* ctx, double kappa, int precision) {
     size_t freeb = 0, totalb = 0;
     hip_check(hipMemGetInfo(&freeb, &totalb), "hipMemGetInfo");
     if (precision == BEEP_FP64) {
-        const size_t need = size_t(ctx->nnz) * 2 * sizeof(double2);
+        const size_t need = coef64_size(ctx->nnz) * sizeof(double2);
         const size_t have = ctx->coef64.n * sizeof(double2);
         require(need <= have || need + (size_t(1) << 30) < freeb + have,
                 "not enough device memory for FP64 coefficients");
-        ctx->coef64.alloc(size_t(ctx->nnz) * 2);
+        ctx->coef64.alloc(coef64_size(ctx->nnz));
         launch_set_int(s, reinterpret_cast<int*>(gcnt + 1), 0);
         launch_near_coeffs_fp64(s, ctx->n_coef_blocks, ctx->L, ctx->coef_blk.p, ctx->leaf_ptr.p,
                                 ctx->leaf_idx.p, ctx->nb_ptr.p, ctx->nb_idx.p, ctx->coef_off.p,
@@ -1501,7 +1520,7 @@ int beep_hip_share_near(beep_hip_ctx* ctx, beep_hip_ctx* src, int n_copies, cons
         ctx->pair_col.upload(col.data(), col.size(), s);
         ctx->pair_i.upload(pi.data(), pi.size(), s);
         ctx->pcoef32.alloc(np);
-        ctx->pcoef64.alloc(2 * np);
+        ctx->pcoef64.alloc(coef64_size((long long)np));
         hip_check(hipStreamSynchronize(s), "sync pairs");  // host arrays die here
         // no residual leaf pass: the explicit pairs store full - 1 point
         far_setup(ctx);
@@ -1561,7 +1580,7 @@ int beep_hip_share_near_cutoff(beep_hip_ctx* ctx, beep_hip_ctx* src, int n_copie
         ctx->pair_col.alloc(np);
         ctx->pair_i.alloc(np);
         ctx->pcoef32.alloc(np);
-        ctx->pcoef64.alloc(2 * np);
+        ctx->pcoef64.alloc(coef64_size((long long)np));
         ctx->pair_rows.alloc(size_t(N));
         if (total > 0)
             launch_cut_pairs(s, N, n_copies, Ns, ctx->cut_off_d.p, ctx->cut_sph_d.p, ctx->cut_chunk_d.p,
@@ -1693,8 +1712,9 @@ int beep_hip_debug_poke(beep_hip_ctx* ctx, int which, long long entry, const dou
         if (which == 0) {
             require(ctx->have64 && entry >= 0 && entry < ctx->nnz, "no such FP64 coefficient");
             const double2 h[2] = {make_double2(v4[0], v4[1]), make_double2(v4[2], v4[3])};
-            hip_check(hipMemcpyAsync(ctx->coef64.p + 2 * entry, h, sizeof(h), hipMemcpyHostToDevice, s),
-                      "H2D poke");
+            for (int k = 0; k < 2; ++k)
+                hip_check(hipMemcpyAsync(ctx->coef64.p + coef64_at(entry) + k * COEF64_CD, h + k, sizeof(double2),
+                                         hipMemcpyHostToDevice, s), "H2D poke");
         } else if (which == 1) {
             require(ctx->have32 && entry >= 0 && entry < ctx->nnz, "no such FP32 coefficient");
             const float4 h = make_float4(float(v4[0]), float(v4[1]), float(v4[2]), float(v4[3]));
@@ -1817,7 +1837,8 @@ int beep_hip_matvec_device_noalloc(beep_hip_ctx* ctx, const double* dx, double* 
         else
             launch_near_spmv(s, mode, N, ctx->spmv, ctx->leaf_ptr.p, ctx->leaf_idx.p, ctx->nb_ptr.p,
                              ctx->nb_idx.p, ctx->coef_off.p, ctx->coef32.p, ctx->coef64.p, ctx->diag.p,
-                             dx, spart, dy, spmv_blocks(ctx, mode), ctx->spmv_depth[mode]);
+                             dx, spart, dy, spmv_blocks(ctx, mode), ctx->spmv_depth[mode],
+                             ctx->spmv_next.p);
         if (fold) return;
         if (sym) {
             launch_far_sym(s, far32, N, ctx->leaf_idx.p, ctx->patches.p, dx, ctx->kappa, far);

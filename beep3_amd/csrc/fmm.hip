@@ -205,10 +205,11 @@ __global__ __launch_bounds__(256) void k_m2m(const FmmDev d, int first, T* __res
 // of the axes and t_c one of 16 canonical offsets (t_c0 >= t_c1 >= t_c2 >= 0)
 //   K_t[m][n] = K_c[phi(m)][phi(n)],
 // phi = the same signed permutation acting on node indices.  The plan groups
-// the pairs of a level by canonical offset into chunks of 64; a block stages
-// the source expansions of its chunk through LDS with each pair's node
-// permutation applied (B operands), multiplies by the one canonical table
-// (A operands, 16 tables per level: they stay in L2) with 16x16x4 MFMA tiles.
+// the pairs of a level by canonical offset into chunks of 32; a block stages
+// the source expansions of its chunk in LDS with each pair's node permutation
+// applied (B operands), multiplies by the one canonical table, block diagonal
+// for 15 of the 16 offsets (A operands, 16 tables per level: they stay in L2),
+// with 16x16x4 MFMA tiles.
 // Pairs of a class are listed target by target, so a chunk holds runs of one
 // target's pairs (segments, 3.3 pairs on average): the block sums each
 // segment's results, permuted back to the target's node order, through LDS
@@ -254,174 +255,350 @@ inline int node_of(int mc, int sym) {
     return (a[0] * P + a[1]) * P + a[2];
 }
 
-constexpr int M2L_G = 64;     // pairs per block (4 MFMA column tiles)
-constexpr int M2L_WAVES = 8;  // waves per block, each owning output row tiles
-// K-dimension slab staged in LDS per barrier: 32 (FP64) or 64 (FP32)
-// K-indices, measured fastest; rows padded by 4 (spreads the B reads over the
-// banks, keeps 16-byte alignment)
-template <typename T>
-constexpr int m2l_slab() { return sizeof(T) == 8 ? 32 : 64; }
+inline int node_at(int mc, int sym, int P) {
+    switch (P) {
+        case 3: return node_of<3>(mc, sym);
+        case 4: return node_of<4>(mc, sym);
+        case 5: return node_of<5>(mc, sym);
+        case 6: return node_of<6>(mc, sym);
+        default: throw std::runtime_error("FMM order must be 3..6");
+    }
+}
+
+// A block of 4 waves takes 32 pairs (2 MFMA column tiles): 36 KB of LDS in
+// FP64, so four blocks run on a CU, each in another phase (staging is LDS and
+// VALU work, the products MFMA, and one block's phases do not overlap).
+// Bound by issue: MFMA and VALU time add up (49 and 35 % of the cycles in
+// FP64, by counters).  163,842 patches, order 5, 267,810 pairs x 3: 476 us FP64
+// and 281 us FP32 against 746 and 396 us with full 125 x 125 blocks, sources
+// gathered node by node and results permuted on the way out.
+constexpr int M2L_G = 32;
+constexpr int M2L_WAVES = 4;
+
+// All canonical offsets but (3, 2, 1) are fixed by a reflection or a swap of
+// two axes; the table of such an offset is unchanged when source and target
+// nodes are both mapped by it.  In sums and differences over the node pairs
+// the involution exchanges it is block diagonal: a block of the sums (and the
+// fixed nodes) and one of the differences, 75^2 + 50^2 instead of 125^2
+// products at P = 5.  The involution of an offset (t0 >= t1 >= t2 >= 0):
+constexpr int M2L_NONE = 0;      // no symmetry: one full block
+constexpr int M2L_REFLECT2 = 1;  // t2 = 0: axis 2 reflected
+constexpr int M2L_SWAP01 = 2;    // t0 = t1
+constexpr int M2L_SWAP12 = 3;    // t1 = t2
+constexpr int M2L_TYPES = 4;
+inline int m2l_type(const std::array<int, 3>& t) {
+    if (t[2] == 0) return M2L_REFLECT2;
+    if (t[0] == t[1]) return M2L_SWAP01;
+    if (t[1] == t[2]) return M2L_SWAP12;
+    return M2L_NONE;
+}
+
+// Blocks of one type: ns sums (nfix of them fixed nodes), na differences;
+// their row tiles and k-steps of four
+struct M2lBlocks {
+    int nfix, ns, na, ts, ta, ks, ka;
+};
+__host__ __device__ constexpr M2lBlocks m2l_blocks(int P, int type) {
+    const int NP = P * P * P;
+    const int nfix = type == M2L_NONE ? NP : (type == M2L_REFLECT2 && P % 2 == 0 ? 0 : P * P);
+    const int ns = (NP + nfix) / 2, na = NP - ns;
+    return M2lBlocks{nfix, ns, na, (ns + 15) / 16, (na + 15) / 16, (ns + 3) / 4, (na + 3) / 4};
+}
+// values of one offset's table: both blocks as [4 k-steps][16 row tiles], zero
+// padded; the same room for every offset
+__host__ __device__ constexpr int m2l_table(int P) {
+    int most = 0;
+    for (int t = 0; t < M2L_TYPES; ++t) {
+        const M2lBlocks b = m2l_blocks(P, t);
+        const int n = 64 * (b.ks * b.ts + b.ka * b.ta);
+        most = n > most ? n : most;
+    }
+    return most;
+}
+// k-step slots of a staged source row: both blocks, each rounded up to the rv
+// steps of a 16-byte read
+__host__ __device__ constexpr int m2l_slots(int P, int rv) {
+    int most = 0;
+    for (int t = 0; t < M2L_TYPES; ++t) {
+        const M2lBlocks b = m2l_blocks(P, t);
+        const int n = (b.ks + rv - 1) / rv * rv + (b.ka + rv - 1) / rv * rv;
+        most = n > most ? n : most;
+    }
+    return most;
+}
+
+// passes of a wave over the nodes of an expansion (and the zero after them),
+// 64 entries of the node lists each
+__host__ __device__ constexpr int m2l_passes(int P) { return (P * P * P + 63) / 64; }
+
+// What a wave multiplies: whole row tiles w, w + 4, ... and its share of the
+// last tiles % 4 row tiles, cut by columns and given to the last waves first
+// (the first waves' tiles are the longer sum tiles).
+struct M2lJob {
+    int tile, c0, nc;
+};
+__host__ __device__ constexpr int m2l_jobs(int P) {
+    int most = 0;
+    for (int t = 0; t < M2L_TYPES; ++t) {
+        const int n = (m2l_blocks(P, t).ts + m2l_blocks(P, t).ta + M2L_WAVES - 1) / M2L_WAVES;
+        most = n > most ? n : most;
+    }
+    return most;
+}
+__device__ __forceinline__ M2lJob m2l_job(int w, int j, int tiles) {
+    const int whole = tiles / M2L_WAVES, rest = tiles % M2L_WAVES;
+    if (j < whole) return M2lJob{w + M2L_WAVES * j, 0, 2};
+    if (j > whole || rest == 0) return M2lJob{0, 0, 0};
+    const int t0 = M2L_WAVES * whole, u = M2L_WAVES - 1 - w;  // u: place from the last wave
+    if (rest == 1) return M2lJob{t0, u & 1, u < 2 ? 1 : 0};
+    if (rest == 2) return M2lJob{t0 + (u >> 1), u & 1, 1};
+    return u < 2 ? M2lJob{t0 + u, 0, 2} : M2lJob{t0 + 2, u & 1, 1};
+}
+
+// acc[c] += A B over `steps` k-steps for NC column tiles.  The table operands
+// come from L2 (A: the wave's tile, uniform; lane: the lane's element; 4 ld
+// values per step), PF steps of them in flight: a step's register is loaded
+// again for the next group as soon as its products are issued (a group may
+// read up to PF steps past the last: the table buffer is padded).  The staged
+// sources come from LDS, RV steps per read.
+constexpr int M2L_PF = 4;
+template <typename T, int NC, int BST>
+__device__ __forceinline__ void m2l_multiply(const T* __restrict__ A, unsigned lane, int ld, const T* B, int steps,
+                                             typename Mfma<T>::acc_t* acc) {
+    constexpr int RV = 16 / int(sizeof(T)), PF = M2L_PF;
+    typedef T vec_t __attribute__((ext_vector_type(RV)));
+    T a[PF];
+#pragma unroll
+    for (int r = 0; r < PF; ++r) a[r] = (A + 4 * r * ld)[lane];
+    A += 4 * PF * ld;
+    int sg = 0;
+#pragma unroll 1
+    for (; sg + PF <= steps; sg += PF, A += 4 * PF * ld, B += PF) {
+        vec_t bv[PF / RV][NC];
+#pragma unroll
+        for (int h = 0; h < PF / RV; ++h)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) bv[h][c] = *reinterpret_cast<const vec_t*>(B + c * 16 * BST + h * RV);
+#pragma unroll
+        for (int r = 0; r < PF; ++r) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c) acc[c] = Mfma<T>::op(a[r], bv[r / RV][c][r % RV], acc[c]);
+            a[r] = (A + 4 * r * ld)[lane];
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < PF / RV; ++h) {
+        if (sg + h * RV >= steps) break;
+        vec_t bv[NC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) bv[c] = *reinterpret_cast<const vec_t*>(B + c * 16 * BST + h * RV);
+#pragma unroll
+        for (int r = 0; r < RV; ++r) {
+            if (sg + h * RV + r >= steps) break;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) acc[c] = Mfma<T>::op(a[h * RV + r], bv[c][r], acc[c]);
+        }
+    }
+}
 
 template <typename T, int P>
-__global__ __launch_bounds__(512) void k_m2l(const FmmDev d, const int4* __restrict__ chunks,
-                                             const T* __restrict__ kl,
-                                             const T* const* __restrict__ ytabs,
-                                             const T* __restrict__ M, T* __restrict__ Cout) {
+__global__ __launch_bounds__(64 * M2L_WAVES, sizeof(T) == 4 ? 6 : 4) void k_m2l(const FmmDev d, const int4* __restrict__ chunks,
+                                                                     const T* __restrict__ tabs,
+                                                                     const T* __restrict__ M, T* __restrict__ Cout) {
     constexpr int NP = P * P * P;
-    constexpr int NPP = (NP + 15) / 16 * 16;
-    constexpr int NTILE = NPP / 16;
-    constexpr int NTW = (NTILE + M2L_WAVES - 1) / M2L_WAVES;  // row tiles per wave
-    constexpr int G = M2L_G, CT = G / 16, MS = m2l_slab<T>(), MSP = MS + 4;
-    constexpr int NQ = (G * MS + 511) / 512;  // slab entries per thread
-    constexpr int NSLAB = (NPP + MS - 1) / MS;
-    constexpr int NSTEP = NPP / 4, SPS = MS / 4;  // k-steps, k-steps per slab
-    constexpr int RV = 16 / int(sizeof(T));       // k-steps per 16-byte LDS read
-    static_assert(SPS % RV == 0 && NSTEP % RV == 0, "slab / vector shape");
+    constexpr int G = M2L_G;
+    constexpr int RV = 16 / int(sizeof(T));  // k-steps per 16-byte LDS read
+    constexpr int SPT = m2l_slots(P, RV);
+    // a staged source row: K index 4 s + k at k * SPT + s, so a lane finds the
+    // operands of RV consecutive k-steps side by side; rows 4 odd dwords apart
+    // modulo the 64 banks (conflict-free 16-byte reads of 16 lanes)
+    constexpr int VD = int(sizeof(T)) / 4;
+    // with a zero at NP beside the raw expansion and a spare place at the end
+    constexpr int SPARE = 4 * SPT > NP + 1 ? 4 * SPT : NP + 1;
+    constexpr int BST0 = (SPARE + 1 + 4 / VD - 1) / (4 / VD) * (4 / VD);
+    constexpr int BST = BST0 * VD / 4 % 2 == 1 ? BST0 : BST0 + 4 / VD;
+    constexpr int YS = NP + 1;
+    constexpr int SMEM = G * BST > G * YS ? G * BST : G * YS;
     using acc_t = typename Mfma<T>::acc_t;
-    typedef T vec_t __attribute__((ext_vector_type(RV)));
-    // two B slab buffers [g][position of m] (slab s + 1 is stored while slab
-    // s feeds the matrix cores), then the results Y[g][canonical node] of
-    // the block's pairs, rows padded by one (conflict-free column writes)
-    constexpr int SLAB_BUF = G * MSP, YS = NPP + 1;
-    constexpr int SMEM = 2 * SLAB_BUF > G * YS ? 2 * SLAB_BUF : G * YS;
+    // the staged sources of the block's pairs, then their results Y[g][row]
     __shared__ alignas(16) T smem[SMEM];
-    __shared__ int psrc[G];
-    __shared__ const unsigned short* pperm[G];
-    __shared__ const unsigned short* pphi[G];
     __shared__ int sstart[G + 1];  // first pair of each segment of the chunk (+ end)
     // block = (chunk, potential): potential 0 uses the Laplace table,
     // potentials 1 and 2 the Yukawa table of the level
     const int bid = xcd_remap(blockIdx.x, gridDim.x);
     const int cid = bid / 3, e = bid - 3 * cid;
-    const int4 ch = chunks[cid];  // canonical offset, pairs, level
-    const int off = ch.x, p0 = ch.y, np = ch.z - ch.y, level = ch.w;
+    const int4 ch = chunks[cid];  // canonical offset + type << 8, pairs, level
+    const int off = ch.x & 255, type = ch.x >> 8, p0 = ch.y, np = ch.z - ch.y, level = ch.w;
+    const M2lBlocks bk = m2l_blocks(P, type);
     const int t = threadIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6), l = t & 63;
     const int seg0 = d.chunk_seg[cid], nseg = d.chunk_seg[cid + 1] - seg0;
     if (t < G) {
-        const size_t sym = size_t(t < np ? d.pair_sym[p0 + t] : 0) * NP;
-        psrc[t] = t < np ? d.pair_src[p0 + t] : 0;
-        pperm[t] = d.psi + sym;
-        pphi[t] = d.phi + sym;
         if (t < np) {
             const int sg = d.pair_seg[p0 + t];
             if (t == 0 || d.pair_seg[p0 + t - 1] != sg) sstart[sg - seg0] = t;
         }
         if (t == 0) sstart[nseg] = np;
     }
-    const int w = t >> 6, l = t & 63;
+    const int ka0 = (bk.ks + RV - 1) / RV * RV;  // first slot of the differences
+    // Staging: wave w brings in pairs 8 w .. 8 w + 7, GB of them at a time (all
+    // their loads in flight): the source expansion in one coalesced read to the
+    // pair's LDS row, from there the sums and differences over the exchanged
+    // nodes in the pair's canonical order (list: places of the two actual nodes
+    // in the row, that of a zero for a fixed node's second) to the operand
+    // places of the same row.  Only this wave touches the row until the
+    // barrier, and its LDS accesses complete in order.  Nothing is conditional:
+    // pairs past the chunk's end are others' (their results are not added),
+    // lanes past the lists write to the row's spare place.
+    constexpr int GW = G / M2L_WAVES, NQ = m2l_passes(P), GB = NQ <= 2 ? GW : GW / 2, LST = 64 * NQ;
+    unsigned lists[GW];
+#pragma unroll
+    for (int i = 0; i < GW; ++i) lists[i] = unsigned(type * 48 + d.pair_sym[p0 + w * GW + i]) * LST;
+    auto place = [&](int slot0, int k) { return (k & 3) * SPT + slot0 + (k >> 2); };
+    int at_raw[NQ], at_sum[NQ], at_diff[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const int m = l + 64 * q;
+        at_raw[q] = m < NP ? m : SPARE;
+        at_sum[q] = m < bk.ns ? place(0, m) : SPARE;
+        at_diff[q] = m >= bk.nfix && m < bk.ns ? place(ka0, m - bk.nfix) : SPARE;
+    }
+    // the last k-steps' missing K indices
+    const int ps = 4 * bk.ks - bk.ns, pa = 4 * bk.ka - bk.na;
+    const int at_pad = l < ps ? place(0, bk.ns + l) : (l < ps + pa ? place(ka0, bk.na + l - ps) : SPARE);
+#pragma unroll
+    for (int i0 = 0; i0 < GW; i0 += GB) {
+        T raw[GB][NQ];
+        unsigned ab[GB][NQ];
+#pragma unroll
+        for (int i = 0; i < GB; ++i) {
+            const T* src = M + (size_t(d.pair_src[p0 + w * GW + i0 + i]) * 3 + e) * NP;
+            const unsigned* list = d.m2l_src + lists[i0 + i];
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                raw[i][q] = src[unsigned(l) + 64 * q];
+                ab[i][q] = list[unsigned(l) + 64 * q];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < GB; ++i) {
+            T* row = smem + (w * GW + i0 + i) * BST;
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) row[at_raw[q]] = raw[i][q];
+            if (l == 0) row[NP] = T(0);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int i = 0; i < GB; ++i) {
+            T* row = smem + (w * GW + i0 + i) * BST;
+            T a[NQ], b[NQ];
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                a[q] = row[ab[i][q] & 0xffffu];
+                b[q] = row[ab[i][q] >> 16];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                row[at_sum[q]] = a[q] + b[q];
+                row[at_diff[q]] = a[q] - b[q];
+            }
+            row[at_pad] = T(0);
+        }
+    }
     const int kl16 = l / 16, il = l % 16;
-    const T* KT = (e == 0 ? kl : ytabs[level]) + size_t(off) * NP * NP;
-    acc_t acc[NTW][CT];
+    const T* KT = tabs + (size_t(e == 0 ? d.D + 1 : level) * FmmPlan::NCANON + off) * m2l_table(P);
+    constexpr int NJ = m2l_jobs(P);
+    acc_t acc[NJ][2];
 #pragma unroll
-    for (int k = 0; k < NTW; ++k)
+    for (int j = 0; j < NJ; ++j)
 #pragma unroll
-        for (int c = 0; c < CT; ++c) acc[k][c] = acc_t{0, 0, 0, 0};
-    // B slabs: B[g][mm] = M_src(g)[e][psi_g(m0 + mm)], the source expansions
-    // in the canonical node order of their pairs.  Thread t owns the same
-    // (g, mm) entries of every slab (consecutive threads walk mm of one g, a
-    // run inside one expansion).  In each g row, m = 4 s + k (k-step s of the
-    // slab, K index k of the MFMA operand) sits at k * SPS + s, so a lane
-    // finds the operands of RV consecutive k-steps side by side.
-    __syncthreads();  // pair lists written
-    int qsrc[NQ], qmm[NQ];
-    const unsigned short* qperm[NQ];
+        for (int c = 0; c < 2; ++c) acc[j][c] = acc_t{0, 0, 0, 0};
+    __syncthreads();
 #pragma unroll
-    for (int i = 0; i < NQ; ++i) {
-        const int q = t + 512 * i;
-        const int g = q / MS, mm = q - g * MS;
-        const bool ok = q < G * MS && g < np;
-        qsrc[i] = ok ? psrc[g] * 3 * NP + e * NP : -1;
-        qperm[i] = ok ? pperm[g] : nullptr;
-        qmm[i] = q < G * MS ? g * MSP + (mm & 3) * SPS + (mm >> 2) : -1;
+    for (int j = 0; j < NJ; ++j) {
+        const M2lJob job = m2l_job(w, j, bk.ts + bk.ta);
+        if (job.nc <= 0) continue;
+        const bool diff = job.tile >= bk.ts;
+        const int ld = 16 * (diff ? bk.ta : bk.ts), steps = diff ? bk.ka : bk.ks;
+        const T* A = KT + (diff ? 64 * bk.ks * bk.ts : 0) + 16 * (diff ? job.tile - bk.ts : job.tile);
+        const unsigned lane = unsigned(kl16 * ld + il);
+        const T* B = smem + (job.c0 * 16 + il) * BST + kl16 * SPT + (diff ? ka0 : 0);
+        if (job.nc == 2) m2l_multiply<T, 2, BST>(A, lane, ld, B, steps, acc[j]);
+        else m2l_multiply<T, 1, BST>(A, lane, ld, B, steps, acc[j]);
     }
-    auto fetch = [&](int m0, T* v) {
-#pragma unroll
-        for (int i = 0; i < NQ; ++i) {
-            const int m = m0 + (t + 512 * i) % MS;
-            v[i] = (qsrc[i] >= 0 && m < NP) ? M[size_t(qsrc[i]) + qperm[i][m]] : T(0);
-        }
-    };
-    T nxt[NQ];
-    fetch(0, nxt);
-#pragma unroll
-    for (int i = 0; i < NQ; ++i)
-        if (qmm[i] >= 0) smem[qmm[i]] = nxt[i];
-    if (NSLAB > 1) fetch(MS, nxt);  // in flight during the first slab
-    // A operands (kernel table values) one k-step ahead: the loads of step
-    // k+1 are in flight while the MFMAs of step k run
-    T xa_n[NTW];
-    auto load_a = [&](int step, T* xa) {
-        const int m = 4 * step + kl16;  // K-dimension index (canonical source node)
-#pragma unroll
-        for (int k = 0; k < NTW; ++k) {
-            const int n = (w + M2L_WAVES * k) * 16 + il;  // output row (canonical target node)
-            xa[k] = (m < NP && n < NP) ? KT[m * NP + n] : T(0);
-        }
-    };
-    load_a(0, xa_n);
-#pragma unroll 1
-    for (int sg = 0; sg < NSTEP; sg += RV) {
-        const int ss = sg % SPS, slab = sg / SPS;  // first k-step of the group in its slab
-        if (ss == 0) {
-            // slab `slab` is complete in its buffer, and every read of the
-            // previous slab (the other buffer) is done
-            __syncthreads();
-            if (slab + 1 < NSLAB) {
-#pragma unroll
-                for (int i = 0; i < NQ; ++i)
-                    if (qmm[i] >= 0) smem[((slab + 1) & 1) * SLAB_BUF + qmm[i]] = nxt[i];
-                if (slab + 2 < NSLAB) fetch((slab + 2) * MS, nxt);
-            }
-        }
-        const T* sbuf = smem + (slab & 1) * SLAB_BUF;
-        vec_t bv[CT];
-#pragma unroll
-        for (int c = 0; c < CT; ++c)
-            bv[c] = *reinterpret_cast<const vec_t*>(&sbuf[(c * 16 + il) * MSP + kl16 * SPS + ss]);
-#pragma unroll
-        for (int r = 0; r < RV; ++r) {
-            const int step = sg + r;
-            T xa[NTW];
-#pragma unroll
-            for (int k = 0; k < NTW; ++k) xa[k] = xa_n[k];
-            if (step + 1 < NSTEP) load_a(step + 1, xa_n);
-#pragma unroll
-            for (int k = 0; k < NTW; ++k) {
-                if (w + M2L_WAVES * k >= NTILE) continue;
-#pragma unroll
-                for (int c = 0; c < CT; ++c) acc[k][c] = Mfma<T>::op(xa[k], bv[c][r], acc[k][c]);
-            }
-        }
-    }
-    // the results through LDS: Y[g][n] of pair g at canonical target node n
+    // the results through LDS: Y[g][row] of pair g, sums then differences
     // (accumulator element r of lane l holds row Mfma<T>::row(l, r) of the
     // tile, column l % 16)
     const T scale = e == 0 ? T(1.0 / d.box_h[level]) : T(1);  // Laplace tables are built at h = 1
-    __syncthreads();  // every read of the last slab done: the slab buffers become Y
+    // block rows of every actual target node of this wave's pairs: sum row |
+    // difference row (that of a zero for a fixed node) << 12 | sign << 31
+    unsigned rows_of[GW][NQ];
 #pragma unroll
-    for (int k = 0; k < NTW; ++k) {
-        const int nt = w + M2L_WAVES * k;
-        if (nt >= NTILE) continue;
+    for (int i = 0; i < GW; ++i)
 #pragma unroll
-        for (int c = 0; c < CT; ++c) {
-            const acc_t v = acc[k][c];
-            T* col = smem + (c * 16 + il) * YS + nt * 16;
+        for (int q = 0; q < NQ; ++q) rows_of[i][q] = (d.m2l_dst + lists[i])[unsigned(l) + 64 * q];
+    __syncthreads();  // every read of the staged sources done: they become Y
 #pragma unroll
-            for (int r = 0; r < 4; ++r) col[Mfma<T>::row(l, r)] = v[r] * scale;
+    for (int j = 0; j < NJ; ++j) {
+        const M2lJob job = m2l_job(w, j, bk.ts + bk.ta);
+        if (job.nc <= 0) continue;
+        const bool diff = job.tile >= bk.ts;
+        const int row0 = 16 * (diff ? job.tile - bk.ts : job.tile), rows = diff ? bk.na : bk.ns;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            if (c >= job.nc) continue;
+            T* col = smem + ((job.c0 + c) * 16 + il) * YS + (diff ? bk.ns : 0);
+            const int spare = NP - (diff ? bk.ns : 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = row0 + Mfma<T>::row(l, r);
+                col[row < rows ? row : spare] = acc[j][c][r] * scale;
+            }
         }
     }
     __syncthreads();
-    // one slot per segment: its pairs' results at each actual target node m
-    // (canonical node phi_g(m) of pair g), added in pair order
-    for (int o = t; o < nseg * NP; o += 512) {
-        const int sl = o / NP, m = o - sl * NP;
-        T sum = 0;
-        for (int g = sstart[sl]; g < sstart[sl + 1]; ++g) sum += smem[g * YS + pphi[g][m]];
-        Cout[(size_t(seg0 + sl) * 3 + e) * NP + m] = sum;
+    // to the actual target nodes, sum row +- difference row, in place (a wave
+    // owns its pairs' rows)
+#pragma unroll
+    for (int i = 0; i < GW; ++i) {
+        T* y = smem + (w * GW + i) * YS;
+        if (l == 0) y[NP] = T(0);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        T v[NQ];
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            const unsigned r = rows_of[i][q];
+            const T dv = y[(r >> 12) & 0xfffu];
+            v[q] = y[r & 0xfffu] + (int(r) < 0 ? -dv : dv);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) y[min(l + 64 * q, NP)] = v[q];
+    }
+    __syncthreads();
+    // one slot per segment: its pairs' results added in pair order (a wave per
+    // segment, its bounds uniform)
+    for (int sl = w; sl < nseg; sl += M2L_WAVES) {
+        const int ga = __builtin_amdgcn_readfirstlane(sstart[sl]), gb = __builtin_amdgcn_readfirstlane(sstart[sl + 1]);
+        const T* y = smem + ga * YS;
+        T sum[NQ];
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) sum[q] = y[min(l + 64 * q, NP)];
+        for (int g = ga + 1; g < gb; ++g) {
+            y += YS;
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) sum[q] += y[min(l + 64 * q, NP)];
+        }
+        T* out = Cout + (size_t(seg0 + sl) * 3 + e) * NP;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q)
+            if (l + 64 * q < NP) out[l + 64 * q] = sum[q];
     }
 }
 
-// Sum the M2L segment slots of every target box into its local expansion
+// Sum the M2L segment slots of every target box to its local expansion (zero
+// without any: every box of the levels >= 2 is written)
 // (one block per box at levels >= 2; a box's segments listed in increasing
 // order in tgt_ptr / tgt_seg).  Each thread owns outputs (e, n) and adds the
 // slots in list order, so the sum is deterministic.
@@ -432,7 +609,6 @@ __global__ __launch_bounds__(256) void k_m2l_sum(const FmmDev d, int first_box,
     constexpr int NQ = (3 * NP + 255) / 256;
     const int box = first_box + blockIdx.x;
     const int k0 = d.tgt_ptr[box], k1 = d.tgt_ptr[box + 1];
-    if (k0 == k1) return;
     const int t = threadIdx.x;
     T acc[NQ];
 #pragma unroll
@@ -446,7 +622,7 @@ __global__ __launch_bounds__(256) void k_m2l_sum(const FmmDev d, int first_box,
     }
 #pragma unroll
     for (int i = 0; i < NQ; ++i)
-        if (t + 256 * i < 3 * NP) L[size_t(box) * 3 * NP + t + 256 * i] += acc[i];
+        if (t + 256 * i < 3 * NP) L[size_t(box) * 3 * NP + t + 256 * i] = acc[i];
 }
 
 // L2L: one block per child box at level l+1 (boxes [first, first+count)).
@@ -535,9 +711,9 @@ __global__ __launch_bounds__(64) void k_l2p(const FmmDev d, const Patch64* __res
                 }
             }
         const T nx = T(p.nx), ny = T(p.ny), nz = T(p.nz);
-        y[i] += double(pL + p1) * FOUR_PI_INV;
-        y[n + i] += double(ih * (nx * (gLx + g2x) + ny * (gLy + g2y) + nz * (gLz + g2z))) *
-                    FOUR_PI_INV;
+        y[i] = double(pL + p1) * FOUR_PI_INV;
+        y[n + i] = double(ih * (nx * (gLx + g2x) + ny * (gLy + g2y) + nz * (gLz + g2z))) *
+                   FOUR_PI_INV;
     }
 }
 
@@ -642,36 +818,43 @@ __global__ __launch_bounds__(256) void k_p2p(const FmmDev d, const Src64* __rest
     }
 }
 
-template <typename T>
-__global__ void k_zero(size_t n, T* __restrict__ p) {
-    const size_t k = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (k < n) p[k] = T(0);
-}
-
-// Kernel tables between node sets: out[c][m][n] = G(|t_c + (xi_m - xi_n)/2| * h)
+// Kernel tables between node sets, K[m][n] = G(|t_c + (xi_m - xi_n)/2| * h)
 // (m = source node, n = target node) for the canonical offsets t_c (box
-// units, t_c0 >= t_c1 >= t_c2 >= 0, t_c0 in {2, 3}); laplace: 1/r with h = 1
-// (scaled by 1/h at use), else e^{-kappa r}/r at box size h.
+// units, t_c0 >= t_c1 >= t_c2 >= 0, t_c0 in {2, 3}), as the two blocks of
+// m2l_blocks: over the sums of exchanged pairs (a, b) = nodes[type][q] (equal
+// for a fixed node) 1/2 (K[a_q][a_r] + K[b_q][a_r]), over the differences
+// 1/2 (K[a_q][a_r] - K[b_q][a_r]).  laplace: 1/r with h = 1 (scaled by 1/h at
+// use), else e^{-kappa r}/r at box size h.
 template <typename T, int P>
 __global__ void k_ktab(const double* __restrict__ xi, const int4* __restrict__ canon, int ncanon,
-                       double h, double kappa, int laplace, T* __restrict__ out) {
-    constexpr int NP = P * P * P;
+                       const unsigned* __restrict__ nodes, double h, double kappa, int laplace,
+                       T* __restrict__ out) {
+    constexpr int NP = P * P * P, TBL = m2l_table(P);
     const size_t idx = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (idx >= size_t(ncanon) * NP * NP) return;
-    const int off = int(idx / (size_t(NP) * NP));
-    const int rem = int(idx - size_t(off) * NP * NP);
-    const int m = rem / NP, nn = rem - m * NP;
-    const int tx = canon[off].x, ty = canon[off].y, tz = canon[off].z;
-    const int ma = m / (P * P), mb = (m / P) % P, mc = m % P;
-    const int na = nn / (P * P), nb = (nn / P) % P, nc = nn % P;
-    const double vx = tx + 0.5 * (xi[ma] - xi[na]);
-    const double vy = ty + 0.5 * (xi[mb] - xi[nb]);
-    const double vz = tz + 0.5 * (xi[mc] - xi[nc]);
-    const double r = sqrt(vx * vx + vy * vy + vz * vz);
+    if (idx >= size_t(ncanon) * TBL) return;
+    const int off = int(idx / TBL), rem = int(idx - size_t(off) * TBL);
+    const int4 tc = canon[off];  // offset, type
+    const M2lBlocks bk = m2l_blocks(P, tc.w);
+    const int sums = 64 * bk.ks * bk.ts, all = sums + 64 * bk.ka * bk.ta;
     double v = 0;
-    if (max(abs(tx), max(abs(ty), abs(tz))) > 1) {
-        if (laplace) v = 1.0 / r;
-        else v = exp(-kappa * h * r) / (h * r);
+    const bool diff = rem >= sums;
+    const int at = diff ? rem - sums : rem, ld = 16 * (diff ? bk.ta : bk.ts), rows = diff ? bk.na : bk.ns;
+    if (rem < all) {
+        const int k = at / ld, r = at - k * ld;
+        if (k < rows && r < rows) {
+            const int q0 = diff ? bk.nfix : 0;
+            const unsigned src = nodes[tc.w * NP + q0 + k];
+            const int nn = int(nodes[tc.w * NP + q0 + r] & 0xffffu);
+            auto G = [&](int m) {
+                const double vx = tc.x + 0.5 * (xi[m / (P * P)] - xi[nn / (P * P)]);
+                const double vy = tc.y + 0.5 * (xi[(m / P) % P] - xi[(nn / P) % P]);
+                const double vz = tc.z + 0.5 * (xi[m % P] - xi[nn % P]);
+                const double rr = sqrt(vx * vx + vy * vy + vz * vz);
+                return laplace ? 1.0 / rr : exp(-kappa * h * rr) / (h * rr);
+            };
+            const int a = int(src & 0xffffu), b = int(src >> 16);
+            v = a == b ? G(a) : 0.5 * (diff ? G(a) - G(b) : G(a) + G(b));
+        }
     }
     out[idx] = T(v);
 }
@@ -1040,7 +1223,7 @@ void fmm_plan_finish(FmmPlan* pl, hipStream_t s) {
                     pair_sym.push_back(v[j][2]);
                     pair_seg.push_back(n_segs - 1);
                 }
-                chunks.push_back(make_int4(off, b0, int(pair_src.size()), l));
+                chunks.push_back(make_int4(off | m2l_type(canonical_list()[off]) << 8, b0, int(pair_src.size()), l));
             }
         }
     }
@@ -1048,6 +1231,9 @@ void fmm_plan_finish(FmmPlan* pl, hipStream_t s) {
     chunk_seg.push_back(n_segs);
     if (D >= 2 && pl->lvl_chunk[2] != 0) throw std::runtime_error("M2L chunks must start at level 2");
     pl->n_pairs = int(pair_src.size());
+    // a block reads a full chunk of pairs: past the last, box 0 unpermuted
+    pair_src.resize(pair_src.size() + G, 0);
+    pair_sym.resize(pair_sym.size() + G, 0);
     pl->n_segs = n_segs;
     // per target box its segments, in increasing order (the order k_m2l_sum
     // adds them in)
@@ -1187,32 +1373,56 @@ void fmm_plan_finish(FmmPlan* pl, hipStream_t s) {
     upload(arena, "pair_sym", pl->dv.pair_sym, pair_sym, s);
     upload(arena, "pair_seg", pl->dv.pair_seg, pair_seg, s);
     upload(arena, "chunk_seg", pl->dv.chunk_seg, chunk_seg, s);
-    // node maps of the 48 symmetries: psi (canonical -> actual) and phi
-    // (actual -> canonical), order^3 entries each (host copies live until the
-    // stream is synchronised below)
+    // the node pairs each involution exchanges (canonical nodes, the fixed
+    // ones first), and under each of the 48 symmetries the actual source nodes
+    // of every pair and the block rows every actual target node is made of
+    // (host copies live until the stream is synchronised below)
     const int NPn = order * order * order;
-    std::vector<unsigned short> psi(size_t(48) * NPn), phi(size_t(48) * NPn);
+    std::vector<unsigned> m2l_nodes, m2l_src, m2l_dst;
     if (pl->engine == 0) {
-        for (int k = 0; k < 48; ++k)
+        m2l_nodes.resize(size_t(M2L_TYPES) * NPn, 0u);
+        const int LST = 64 * m2l_passes(order);
+        const unsigned zero = unsigned(NPn);  // place of a zero in a staged or result row
+        m2l_src.resize(size_t(M2L_TYPES) * 48 * LST, zero | zero << 16);
+        m2l_dst.resize(size_t(M2L_TYPES) * 48 * LST, zero | zero << 12);
+        for (int ty = 0; ty < M2L_TYPES; ++ty) {
+            const M2lBlocks bk = m2l_blocks(order, ty);
+            std::vector<std::pair<int, int>> fixed, pairs;
             for (int m = 0; m < NPn; ++m) {
-                int a = 0;
-                switch (order) {
-                    case 3: a = node_of<3>(m, symmetry_codes()[k]); break;
-                    case 4: a = node_of<4>(m, symmetry_codes()[k]); break;
-                    case 5: a = node_of<5>(m, symmetry_codes()[k]); break;
-                    default: a = node_of<6>(m, symmetry_codes()[k]); break;
-                }
-                psi[size_t(k) * NPn + m] = (unsigned short)a;
-                phi[size_t(k) * NPn + a] = (unsigned short)m;
+                int c[3] = {m / (order * order), (m / order) % order, m % order};
+                if (ty == M2L_REFLECT2) c[2] = order - 1 - c[2];
+                if (ty == M2L_SWAP01) std::swap(c[0], c[1]);
+                if (ty == M2L_SWAP12) std::swap(c[1], c[2]);
+                const int im = (c[0] * order + c[1]) * order + c[2];
+                if (im == m) fixed.push_back({m, m});
+                if (im > m) pairs.push_back({m, im});
             }
-        upload(arena, "psi", pl->dv.psi, psi, s);
-        upload(arena, "phi", pl->dv.phi, phi, s);
+            if (int(fixed.size()) != bk.nfix || int(pairs.size()) != bk.na)
+                throw std::runtime_error("M2L symmetry blocks");
+            fixed.insert(fixed.end(), pairs.begin(), pairs.end());
+            for (int q = 0; q < bk.ns; ++q) {
+                const auto [a, b] = fixed[q];
+                m2l_nodes[size_t(ty) * NPn + q] = unsigned(a) | unsigned(b) << 16;
+                for (int k = 0; k < 48; ++k) {
+                    const size_t at = (size_t(ty) * 48 + k) * LST;
+                    const unsigned ra = unsigned(node_at(a, symmetry_codes()[k], order));
+                    const unsigned rb = unsigned(node_at(b, symmetry_codes()[k], order));
+                    m2l_src[at + q] = ra | (a == b ? zero : rb) << 16;
+                    const unsigned dr = a == b ? zero : unsigned(bk.ns + q - bk.nfix);
+                    m2l_dst[at + ra] = unsigned(q) | dr << 12;
+                    if (a != b) m2l_dst[at + rb] = unsigned(q) | dr << 12 | 1u << 31;
+                }
+            }
+        }
+        upload(arena, "m2l_nodes", pl->d_m2l_nodes, m2l_nodes, s);
+        upload(arena, "m2l_src", pl->dv.m2l_src, m2l_src, s);
+        upload(arena, "m2l_dst", pl->dv.m2l_dst, m2l_dst, s);
     }
     std::vector<int4> canon(FmmPlan::NCANON);
     {
         for (int c = 0; c < FmmPlan::NCANON; ++c) {
             const auto t = canonical_list()[c];
-            canon[c] = make_int4(t[0], t[1], t[2], 0);
+            canon[c] = make_int4(t[0], t[1], t[2], m2l_type(t));
         }
         upload(arena, "canon", pl->d_canon, canon, s);
     }
@@ -1222,8 +1432,6 @@ void fmm_plan_finish(FmmPlan* pl, hipStream_t s) {
     upload(arena, "t_oct", pl->dv.t_oct, t_oct, s);
     upload(arena, "chunks", pl->d_chunks, chunks, s);
     upload(arena, "xi", pl->d_xi, xi, s);
-    pl->ktab64.assign(D + 2, nullptr);
-    pl->ktab32.assign(D + 2, nullptr);
     pl->src = arena.get<Src64>("src", size_t(std::max(N, 1)));
     const size_t ne = size_t(nbox) * 3 * NP;
     pl->n_exp = ne;
@@ -1269,27 +1477,21 @@ void fmm_plan_destroy(FmmPlan* p) {
     delete p;
 }
 
+// the kernel tables of every level in one buffer: slot l Yukawa at level l,
+// slot D+1 Laplace (level independent, h = 1)
 template <typename T, int P>
-static void make_tables(FmmPlan* pl, double kappa, std::vector<T*>& tabs, T**& ytab,
-                        hipStream_t s) {
-    constexpr int NP = P * P * P;
-    const size_t n = size_t(FmmPlan::NCANON) * NP * NP;
+static void make_tables(FmmPlan* pl, double kappa, T*& tabs, hipStream_t s) {
+    const size_t n = size_t(FmmPlan::NCANON) * m2l_table(P);
     const int blocks = int((n + 255) / 256);
-    const std::string pre = sizeof(T) == 8 ? "ktab64_" : "ktab32_";
-    tabs.assign(pl->D + 2, nullptr);
-    // slot D+1: Laplace (level independent, h = 1); slot l: Yukawa at level l
-    tabs[pl->D + 1] = pl->arena->get<T>(pre + "laplace", n);
-    hipLaunchKernelGGL((k_ktab<T, P>), dim3(blocks), dim3(256), 0, s, pl->d_xi, pl->d_canon,
-                       FmmPlan::NCANON, 1.0, 0.0, 1, tabs[pl->D + 1]);
-    for (int l = 2; l <= pl->D; ++l) {
-        tabs[l] = pl->arena->get<T>(pre + std::to_string(l), n);
-        hipLaunchKernelGGL((k_ktab<T, P>), dim3(blocks), dim3(256), 0, s, pl->d_xi, pl->d_canon,
-                           FmmPlan::NCANON, pl->box_h[l], kappa, 0, tabs[l]);
+    const size_t pad = size_t(M2L_PF) * 4 * 16 * ((P * P * P + 15) / 16);  // m2l_multiply reads ahead
+    tabs = pl->arena->get<T>(sizeof(T) == 8 ? "ktab64" : "ktab32", n * (pl->D + 2) + pad);
+    for (int l = 2; l <= pl->D + 1; ++l) {
+        const bool laplace = l == pl->D + 1;
+        hipLaunchKernelGGL((k_ktab<T, P>), dim3(blocks), dim3(256), 0, s, pl->d_xi, pl->d_canon, FmmPlan::NCANON,
+                           pl->d_m2l_nodes, laplace ? 1.0 : pl->box_h[l], laplace ? 0.0 : kappa, laplace ? 1 : 0,
+                           tabs + n * l);
     }
     hip_check(hipGetLastError(), "k_ktab launch");
-    ytab = pl->arena->get<T*>(pre + "ptrs", tabs.size());
-    hip_check(hipMemcpyAsync(ytab, tabs.data(), tabs.size() * sizeof(T*), hipMemcpyHostToDevice, s),
-              "H2D ytab");
 }
 
 // M2L result slots: 3 x P^3 values per target segment
@@ -1311,25 +1513,25 @@ void fmm_prepare(FmmPlan* pl, double kappa, bool fp64, bool fp32, hipStream_t s)
     }
     if (fp64 && !pl->have64) {
         switch (pl->P) {
-            case 3: make_tables<double, 3>(pl, kappa, pl->ktab64, pl->ytab64, s); break;
-            case 4: make_tables<double, 4>(pl, kappa, pl->ktab64, pl->ytab64, s); break;
-            case 5: make_tables<double, 5>(pl, kappa, pl->ktab64, pl->ytab64, s); break;
-            case 6: make_tables<double, 6>(pl, kappa, pl->ktab64, pl->ytab64, s); break;
+            case 3: make_tables<double, 3>(pl, kappa, pl->ktab64, s); break;
+            case 4: make_tables<double, 4>(pl, kappa, pl->ktab64, s); break;
+            case 5: make_tables<double, 5>(pl, kappa, pl->ktab64, s); break;
+            case 6: make_tables<double, 6>(pl, kappa, pl->ktab64, s); break;
         }
         const size_t ns = slot_count(pl);
-        pl->exp64 = pl->arena->get<double>("exp64", 2 * pl->n_exp);
+        pl->exp64 = pl->arena->get<double>("exp64", 2 * pl->n_exp + 64);  // M2L reads whole passes
         pl->slots64 = pl->arena->get<double>("slots64", ns);
         pl->have64 = true;
     }
     if (fp32 && !pl->have32) {
         switch (pl->P) {
-            case 3: make_tables<float, 3>(pl, kappa, pl->ktab32, pl->ytab32, s); break;
-            case 4: make_tables<float, 4>(pl, kappa, pl->ktab32, pl->ytab32, s); break;
-            case 5: make_tables<float, 5>(pl, kappa, pl->ktab32, pl->ytab32, s); break;
-            case 6: make_tables<float, 6>(pl, kappa, pl->ktab32, pl->ytab32, s); break;
+            case 3: make_tables<float, 3>(pl, kappa, pl->ktab32, s); break;
+            case 4: make_tables<float, 4>(pl, kappa, pl->ktab32, s); break;
+            case 5: make_tables<float, 5>(pl, kappa, pl->ktab32, s); break;
+            case 6: make_tables<float, 6>(pl, kappa, pl->ktab32, s); break;
         }
         const size_t ns = slot_count(pl);
-        pl->exp32 = pl->arena->get<float>("exp32", 2 * pl->n_exp);
+        pl->exp32 = pl->arena->get<float>("exp32", 2 * pl->n_exp + 64);
         pl->slots32 = pl->arena->get<float>("slots32", ns);
         pl->have32 = true;
     }
@@ -1338,17 +1540,12 @@ void fmm_prepare(FmmPlan* pl, double kappa, bool fp64, bool fp32, hipStream_t s)
 
 template <typename T, int P>
 static void evaluate(FmmPlan* pl, hipStream_t s, const Patch64* patches, const double* x,
-                     double kappa, T* M, T* L, const std::vector<T*>& tabs, T* const* ytab,
-                     T* slots, double* y, hipEvent_t* m2l_ev, hipEvent_t pack_ev) {
+                     double kappa, T* M, T* L, const T* tabs, T* slots, double* y, hipEvent_t* m2l_ev, hipEvent_t pack_ev) {
     constexpr int NP = P * P * P;
     constexpr int NT = ((NP + 63) / 64) * 64;
     const FmmDev& d = pl->dv;
     launch_far_pack(s, pl->N, patches, d.perm, x, pl->src);
     if (pack_ev) hip_check(hipEventRecord(pack_ev, s), "hipEventRecord");
-    {
-        const size_t n = pl->n_exp;
-        hipLaunchKernelGGL((k_zero<T>), dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, n, L);
-    }
     const int D = pl->D;
     hipLaunchKernelGGL((k_p2m<T, P>), dim3(pl->nleaf), dim3(NT), 0, s, d, pl->src, M);
     // parents at levels D-1 .. 2 (level-1 multipoles are never translated)
@@ -1361,9 +1558,10 @@ static void evaluate(FmmPlan* pl, hipStream_t s, const Patch64* patches, const d
         // segments (slots) are numbered in chunk order
         const int nch = D >= 2 ? pl->lvl_chunk[D + 1] : 0;
         if (m2l_ev) hip_check(hipEventRecord(m2l_ev[0], s), "hipEventRecord");
-        if (nch > 0) {
-            hipLaunchKernelGGL((k_m2l<T, P>), dim3(3 * nch), dim3(512), 0, s, d, pl->d_chunks,
-                               tabs[D + 1], ytab, M, slots);
+        if (nch > 0)
+            hipLaunchKernelGGL((k_m2l<T, P>), dim3(3 * nch), dim3(64 * M2L_WAVES), 0, s, d, pl->d_chunks,
+                               tabs, M, slots);
+        if (D >= 2) {
             const int b0 = pl->lvl_first[2], nb = pl->lvl_first[D + 1] - b0;
             hipLaunchKernelGGL((k_m2l_sum<T, P>), dim3(nb), dim3(256), 0, s, d, b0, slots, L);
         }
@@ -1385,15 +1583,7 @@ int fmm_canonical(int tx, int ty, int tz, int order, int* canon_xyz, int* node_m
     const auto t = canonical_list()[c];
     for (int k = 0; k < 3; ++k) canon_xyz[k] = t[k];
     const int NP = order * order * order;
-    for (int m = 0; m < NP; ++m) {
-        switch (order) {
-            case 3: node_map[m] = node_of<3>(m, sym); break;
-            case 4: node_map[m] = node_of<4>(m, sym); break;
-            case 5: node_map[m] = node_of<5>(m, sym); break;
-            case 6: node_map[m] = node_of<6>(m, sym); break;
-            default: throw std::runtime_error("FMM order must be 3..6");
-        }
-    }
+    for (int m = 0; m < NP; ++m) node_map[m] = node_at(m, sym, order);
     return c;
 }
 
@@ -1415,6 +1605,7 @@ void fmm_p2p(FmmPlan* pl, hipStream_t s, int fp32, const Patch64* patches, doubl
 
 void fmm_evaluate(FmmPlan* pl, hipStream_t s, int fp32, const Patch64* patches, const double* x,
                   double kappa, double* y, hipEvent_t* m2l_ev, hipEvent_t pack_ev) {
+    if (pl->D < 2) launch_fill(s, 2 * pl->N, 0.0, y);  // no L2P: the leaf pass covers every pair
     if (pl->engine == 1) {
         launch_far_pack(s, pl->N, patches, pl->dv.perm, x, pl->src);
         if (pack_ev) hip_check(hipEventRecord(pack_ev, s), "hipEventRecord");
@@ -1426,20 +1617,20 @@ void fmm_evaluate(FmmPlan* pl, hipStream_t s, int fp32, const Patch64* patches, 
         float* M = pl->exp32;
         float* L = pl->exp32 + pl->n_exp;
         switch (pl->P) {
-            case 3: evaluate<float, 3>(pl, s, patches, x, kappa, M, L, pl->ktab32, pl->ytab32, pl->slots32, y, m2l_ev, pack_ev); break;
-            case 4: evaluate<float, 4>(pl, s, patches, x, kappa, M, L, pl->ktab32, pl->ytab32, pl->slots32, y, m2l_ev, pack_ev); break;
-            case 5: evaluate<float, 5>(pl, s, patches, x, kappa, M, L, pl->ktab32, pl->ytab32, pl->slots32, y, m2l_ev, pack_ev); break;
-            case 6: evaluate<float, 6>(pl, s, patches, x, kappa, M, L, pl->ktab32, pl->ytab32, pl->slots32, y, m2l_ev, pack_ev); break;
+            case 3: evaluate<float, 3>(pl, s, patches, x, kappa, M, L, pl->ktab32, pl->slots32, y, m2l_ev, pack_ev); break;
+            case 4: evaluate<float, 4>(pl, s, patches, x, kappa, M, L, pl->ktab32, pl->slots32, y, m2l_ev, pack_ev); break;
+            case 5: evaluate<float, 5>(pl, s, patches, x, kappa, M, L, pl->ktab32, pl->slots32, y, m2l_ev, pack_ev); break;
+            case 6: evaluate<float, 6>(pl, s, patches, x, kappa, M, L, pl->ktab32, pl->slots32, y, m2l_ev, pack_ev); break;
         }
     } else {
         if (!pl->have64) throw std::runtime_error("FMM FP64 tables not prepared");
         double* M = pl->exp64;
         double* L = pl->exp64 + pl->n_exp;
         switch (pl->P) {
-            case 3: evaluate<double, 3>(pl, s, patches, x, kappa, M, L, pl->ktab64, pl->ytab64, pl->slots64, y, m2l_ev, pack_ev); break;
-            case 4: evaluate<double, 4>(pl, s, patches, x, kappa, M, L, pl->ktab64, pl->ytab64, pl->slots64, y, m2l_ev, pack_ev); break;
-            case 5: evaluate<double, 5>(pl, s, patches, x, kappa, M, L, pl->ktab64, pl->ytab64, pl->slots64, y, m2l_ev, pack_ev); break;
-            case 6: evaluate<double, 6>(pl, s, patches, x, kappa, M, L, pl->ktab64, pl->ytab64, pl->slots64, y, m2l_ev, pack_ev); break;
+            case 3: evaluate<double, 3>(pl, s, patches, x, kappa, M, L, pl->ktab64, pl->slots64, y, m2l_ev, pack_ev); break;
+            case 4: evaluate<double, 4>(pl, s, patches, x, kappa, M, L, pl->ktab64, pl->slots64, y, m2l_ev, pack_ev); break;
+            case 5: evaluate<double, 5>(pl, s, patches, x, kappa, M, L, pl->ktab64, pl->slots64, y, m2l_ev, pack_ev); break;
+            case 6: evaluate<double, 6>(pl, s, patches, x, kappa, M, L, pl->ktab64, pl->slots64, y, m2l_ev, pack_ev); break;
         }
     }
 }

@@ -28,8 +28,11 @@ struct FmmDev {
     int* pair_sym = nullptr;    // symmetry (0..47) taking each pair to its canonical offset
     int* pair_seg = nullptr;    // target segment of each pair (runs of one target in a chunk)
     int* chunk_seg = nullptr;   // per chunk: its first segment (+ end)
-    unsigned short* psi = nullptr;  // [48][P^3] canonical node -> actual node
-    unsigned short* phi = nullptr;  // [48][P^3] actual node -> canonical node
+    // M2L blocks ([4 involutions][48 symmetries][P^3], see fmm.hip): actual
+    // source nodes a | b << 16 of each sum row; block rows of each actual
+    // target node
+    unsigned* m2l_src = nullptr;
+    unsigned* m2l_dst = nullptr;
     int* tgt_ptr = nullptr;     // per box: its M2L segments, increasing
     int* tgt_seg = nullptr;
     double* tn = nullptr;       // T_j(xi_k), P x P
@@ -124,7 +127,7 @@ struct PwDevTables {
 };
 
 struct FmmPlan {
-    static constexpr int CHUNK = 64;  // M2L pairs per block
+    static constexpr int CHUNK = 32;  // M2L pairs per block
     static constexpr int NCANON = 16; // canonical M2L offsets
     unsigned long long uid = 0;       // unique per plan built in the process
     int N = 0, P = 4, D = 0, nbox = 0, nleaf = 0, n_pairs = 0, n_segs = 0;
@@ -141,14 +144,13 @@ struct FmmPlan {
     std::vector<double> box_h;
     FmmDev dv;
     int4* d_chunks = nullptr;
-    int4* d_canon = nullptr;          // canonical offsets (x, y, z, 0)
+    int4* d_canon = nullptr;          // canonical offsets (x, y, z, involution)
+    unsigned* d_m2l_nodes = nullptr;  // canonical node pairs of each involution
     double* d_xi = nullptr;
-    std::vector<double*> ktab64;      // [l] Yukawa at level l, [D+1] Laplace
-    std::vector<float*> ktab32;
+    double* ktab64 = nullptr;         // M2L tables: [l] Yukawa at level l, [D+1] Laplace
+    float* ktab32 = nullptr;
     double* exp64 = nullptr;          // M then L
     float* exp32 = nullptr;
-    double** ytab64 = nullptr;        // device copies of the table pointers
-    float** ytab32 = nullptr;
     double* slots64 = nullptr;        // M2L results per target segment (n_segs x 3 x P^3)
     float* slots32 = nullptr;
     Src64* src = nullptr;
@@ -207,10 +209,10 @@ inline bool fmm_tables_ready(const FmmPlan* p, double kappa, bool fp64, bool fp3
 // canonical offset of the M2L offset t (index returned, components in
 // canon_xyz) and the map canonical node -> actual node (order^3 entries)
 int fmm_canonical(int tx, int ty, int tz, int order, int* canon_xyz, int* node_map);
-// y += far field (1-point interaction of every pair) of x
-// y += the far field of x without its P2P part (pack, upward pass, M2L,
-// downward pass, L2P); m2l_ev: optional pair of events recorded around the
-// M2L launches; pack_ev: optional event recorded once the sources are packed
+// y = the far field (1-point interaction of every pair) of x without its P2P
+// part (pack, upward pass, M2L, downward pass, L2P); m2l_ev: optional pair of
+// events recorded around the M2L launches; pack_ev: optional event recorded
+// once the sources are packed
 void fmm_evaluate(FmmPlan* p, hipStream_t s, int fp32, const Patch64* patches, const double* x,
                   double kappa, double* y, hipEvent_t* m2l_ev = nullptr,
                   hipEvent_t pack_ev = nullptr);

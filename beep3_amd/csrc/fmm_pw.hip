@@ -300,9 +300,9 @@ __global__ __launch_bounds__(64) void k_pw_l2p(const FmmDev d, const Patch64* __
             });
         }
         const T nx = T(p.nx), ny = T(p.ny), nz = T(p.nz);
-        y[i] += double(pL + p1) * FOUR_PI_INV;
-        y[n_patch + i] += double(T(ih) * (nx * (gL[0] + g2v[0]) + ny * (gL[1] + g2v[1]) +
-                                           nz * (gL[2] + g2v[2]))) * FOUR_PI_INV;
+        y[i] = double(pL + p1) * FOUR_PI_INV;
+        y[n_patch + i] = double(T(ih) * (nx * (gL[0] + g2v[0]) + ny * (gL[1] + g2v[1]) +
+                                          nz * (gL[2] + g2v[2]))) * FOUR_PI_INV;
     }
 }
 

@@ -284,8 +284,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 5) void k_near_coeffs(
         reinterpret_cast<float4*>(coef)[idx] = make_float4(out[0], out[1], out[2], out[3]);
     } else {
         double2* c2 = reinterpret_cast<double2*>(coef);
-        c2[2 * idx] = make_double2(out[0], out[1]);
-        c2[2 * idx + 1] = make_double2(out[2], out[3]);
+        c2[coef64_at(idx)] = make_double2(out[0], out[1]);
+        c2[coef64_at(idx) + COEF64_CD] = make_double2(out[2], out[3]);
     }
 }
 
@@ -372,7 +372,7 @@ __global__ __launch_bounds__(256) void k_coef_scan(
         v[0] = c.x; v[1] = c.y; v[2] = c.z; v[3] = c.w;
     } else {
         const double2* c2 = reinterpret_cast<const double2*>(coef);
-        const double2 a = c2[2 * idx], c = c2[2 * idx + 1];
+        const double2 a = c2[coef64_at(idx)], c = c2[coef64_at(idx) + COEF64_CD];
         v[0] = a.x; v[1] = a.y; v[2] = c.x; v[3] = c.y;
     }
     if (!coef4_bad(v, maxv)) return;
@@ -415,8 +415,8 @@ __global__ __launch_bounds__(256) void k_coef_repair(NsList list, const Patch64*
                 make_float4(float(out[0]), float(out[1]), float(out[2]), float(out[3]));
         } else {
             double2* c2 = reinterpret_cast<double2*>(coef);
-            c2[2 * r.idx] = make_double2(out[0], out[1]);
-            c2[2 * r.idx + 1] = make_double2(out[2], out[3]);
+            c2[coef64_at(r.idx)] = make_double2(out[0], out[1]);
+            c2[coef64_at(r.idx) + COEF64_CD] = make_double2(out[2], out[3]);
         }
         atomicAdd(repaired, 1u);
     }
@@ -487,18 +487,18 @@ struct Coef4 {
 };
 
 typedef float f32x4_nt __attribute__((ext_vector_type(4)));
+typedef double f64x2_nt __attribute__((ext_vector_type(2)));
 
-// Coefficients are read once per mat-vec and exceed every cache.  FP32
-// blocks use streaming (non-temporal) loads, measured 3 % faster; for FP64
-// blocks they measured 14 % slower, so those use ordinary loads.
+// Coefficients are read once per mat-vec and exceed every cache: streaming
+// (non-temporal) loads.
 template <typename TC>
 __device__ __forceinline__ Coef4<TC> load_coef(const void* __restrict__ coef, int64_t idx) {
     if constexpr (sizeof(TC) == 4) {
         const f32x4_nt v = __builtin_nontemporal_load(reinterpret_cast<const f32x4_nt*>(coef) + idx);
         return Coef4<TC>{v.x, v.y, v.z, v.w};
     } else {
-        const double2* c2 = reinterpret_cast<const double2*>(coef);
-        const double2 v0 = c2[2 * idx], v1 = c2[2 * idx + 1];
+        const f64x2_nt* c2 = reinterpret_cast<const f64x2_nt*>(coef) + coef64_at(idx);
+        const f64x2_nt v0 = __builtin_nontemporal_load(c2), v1 = __builtin_nontemporal_load(c2 + COEF64_CD);
         return Coef4<TC>{v0.x, v0.y, v1.x, v1.y};
     }
 }
@@ -602,15 +602,26 @@ __global__ __launch_bounds__(256) void k_near_spmv_part(
     const int4* __restrict__ work, int n_work, const int* __restrict__ leaf_ptr,
     const int* __restrict__ nb_ptr, const int* __restrict__ nb_idx,
     const int64_t* __restrict__ coef_off, const void* __restrict__ coef,
-    const double* __restrict__ x, CopyOffsets co, int n, int pstride, TA* __restrict__ part) {
+    const double* __restrict__ x, CopyOffsets co, int n, int pstride, unsigned* __restrict__ next,
+    TA* __restrict__ part) {
     __shared__ SpmvLds<TA, NC> sm;
+    __shared__ int taken;
     // with fewer blocks than work items (a residency cap that leaves room on
-    // every CU for the far-field kernels of the other stream) a block walks
-    // the work items with a grid stride
-    for (int wi = blockIdx.x; wi < n_work; wi += gridDim.x) {
-        __syncthreads();  // LDS of the previous item consumed
+    // every CU for the far-field kernels of the other stream) a block takes
+    // the next free item from a counter (the sum kernel sets it back to zero):
+    // items differ in size and blocks in speed beside the far field, and a
+    // fixed stride left a tenth of the time to the slowest blocks.  Which
+    // block sums an item does not change its sums.  163,842 patches, one block
+    // per CU, alone: 1,218 us FP64 (6.5 TB/s; 1,491 with a fixed stride, 1,347
+    // uncapped), 651 us FP32 (791, 685).
+    int wi = blockIdx.x;
+    while (wi < n_work) {
+        if (threadIdx.x == 0) taken = gridDim.x < unsigned(n_work) ? int(gridDim.x + atomicAdd(next, 1u)) : n_work;
         spmv_item<TC, TA, U, NC>(sm, wi, work, n_work, leaf_ptr, nb_ptr, nb_idx, coef_off, coef, x, co, n,
                                  pstride, part);
+        __syncthreads();  // LDS of this item consumed
+        wi = taken;
+        __syncthreads();
     }
 }
 
@@ -661,9 +672,10 @@ __global__ __launch_bounds__(256) void k_near_spmv_sum(
     const int4* __restrict__ groups, const int* __restrict__ group_nblk,
     const int* __restrict__ leaf_ptr, const int* __restrict__ leaf_idx,
     const double* __restrict__ diag4, const double* __restrict__ x, CopyOffsets co, int n, int n_work,
-    int pstride, const TA* __restrict__ part, double* __restrict__ y) {
+    int pstride, const TA* __restrict__ part, unsigned* __restrict__ next, double* __restrict__ y) {
     const int4 g = groups[blockIdx.x];  // leaf, first row, rows, first work block
     const int cq = blockIdx.y, off = co.off[cq];
+    if (next && blockIdx.x == 0 && cq == 0 && threadIdx.x == 0) *next = 0u;
     double vf, vh;
     const int i = near_row_sum(g, group_nblk[blockIdx.x], leaf_ptr, leaf_idx, diag4, x, off, n, pstride,
                                part + size_t(cq) * n_work * 2 * pstride, vf, vh);
@@ -679,20 +691,20 @@ template <typename TC, typename TA, int U>
 static void spmv_part(hipStream_t s, int grid, const SpmvPlan& p, const int* leaf_ptr,
                       const int* nb_ptr, const int* nb_idx, const int64_t* coef_off,
                       const void* coef, const double* x, int ncopies, CopyOffsets co, int n,
-                      TA* part) {
+                      unsigned* next, TA* part) {
     if (ncopies == 2)
         hipLaunchKernelGGL((k_near_spmv_part<TC, TA, U, 2>), dim3(grid), dim3(256), 0, s, p.work,
-                           p.n_work, leaf_ptr, nb_ptr, nb_idx, coef_off, coef, x, co, n, p.pstride, part);
+                           p.n_work, leaf_ptr, nb_ptr, nb_idx, coef_off, coef, x, co, n, p.pstride, next, part);
     else
         hipLaunchKernelGGL((k_near_spmv_part<TC, TA, U, 1>), dim3(grid), dim3(256), 0, s, p.work,
-                           p.n_work, leaf_ptr, nb_ptr, nb_idx, coef_off, coef, x, co, n, p.pstride, part);
+                           p.n_work, leaf_ptr, nb_ptr, nb_idx, coef_off, coef, x, co, n, p.pstride, next, part);
 }
 
 void launch_near_spmv(hipStream_t s, int mode, int n, const SpmvPlan& p, const int* leaf_ptr,
                       const int* leaf_idx, const int* nb_ptr, const int* nb_idx,
                       const int64_t* coef_off, const float4* coef32, const double2* coef64,
                       const double* diag4, const double* x, void* part, double* y,
-                      int max_blocks, int depth, int ncopies, const int* copy_offset) {
+                      int max_blocks, int depth, unsigned* next, int ncopies, const int* copy_offset) {
     if (p.n_work <= 0) return;
     if (depth != 1 && depth != 2 && depth != 4) throw std::runtime_error("SpMV depth must be 1, 2 or 4");
     if (ncopies != 1 && ncopies != 2) throw std::runtime_error("the SpMV takes 1 or 2 copies");
@@ -703,28 +715,28 @@ void launch_near_spmv(hipStream_t s, int mode, int n, const SpmvPlan& p, const i
     const dim3 sgrid(unsigned(p.n_groups), unsigned(ncopies));
     if (mode == 0) {
         using F = void (*)(hipStream_t, int, const SpmvPlan&, const int*, const int*, const int*,
-                           const int64_t*, const void*, const double*, int, CopyOffsets, int, double*);
+                           const int64_t*, const void*, const double*, int, CopyOffsets, int, unsigned*, double*);
         constexpr F f[3] = {spmv_part<double, double, 4>, spmv_part<double, double, 8>,
                             spmv_part<double, double, 16>};
-        f[d](s, grid, p, leaf_ptr, nb_ptr, nb_idx, coef_off, coef64, x, ncopies, co, n, (double*)part);
+        f[d](s, grid, p, leaf_ptr, nb_ptr, nb_idx, coef_off, coef64, x, ncopies, co, n, next, (double*)part);
         hipLaunchKernelGGL((k_near_spmv_sum<double>), sgrid, dim3(256), 0, s, p.groups, p.group_nblk,
-                           leaf_ptr, leaf_idx, diag4, x, co, n, p.n_work, p.pstride, (const double*)part, y);
+                           leaf_ptr, leaf_idx, diag4, x, co, n, p.n_work, p.pstride, (const double*)part, next, y);
     } else if (mode == 1) {
         using F = void (*)(hipStream_t, int, const SpmvPlan&, const int*, const int*, const int*,
-                           const int64_t*, const void*, const double*, int, CopyOffsets, int, float*);
+                           const int64_t*, const void*, const double*, int, CopyOffsets, int, unsigned*, float*);
         constexpr F f[3] = {spmv_part<float, float, 8>, spmv_part<float, float, 16>,
                             spmv_part<float, float, 32>};
-        f[d](s, grid, p, leaf_ptr, nb_ptr, nb_idx, coef_off, coef32, x, ncopies, co, n, (float*)part);
+        f[d](s, grid, p, leaf_ptr, nb_ptr, nb_idx, coef_off, coef32, x, ncopies, co, n, next, (float*)part);
         hipLaunchKernelGGL((k_near_spmv_sum<float>), sgrid, dim3(256), 0, s, p.groups, p.group_nblk,
-                           leaf_ptr, leaf_idx, diag4, x, co, n, p.n_work, p.pstride, (const float*)part, y);
+                           leaf_ptr, leaf_idx, diag4, x, co, n, p.n_work, p.pstride, (const float*)part, next, y);
     } else {
         using F = void (*)(hipStream_t, int, const SpmvPlan&, const int*, const int*, const int*,
-                           const int64_t*, const void*, const double*, int, CopyOffsets, int, double*);
+                           const int64_t*, const void*, const double*, int, CopyOffsets, int, unsigned*, double*);
         constexpr F f[3] = {spmv_part<float, double, 8>, spmv_part<float, double, 16>,
                             spmv_part<float, double, 32>};
-        f[d](s, grid, p, leaf_ptr, nb_ptr, nb_idx, coef_off, coef32, x, ncopies, co, n, (double*)part);
+        f[d](s, grid, p, leaf_ptr, nb_ptr, nb_idx, coef_off, coef32, x, ncopies, co, n, next, (double*)part);
         hipLaunchKernelGGL((k_near_spmv_sum<double>), sgrid, dim3(256), 0, s, p.groups, p.group_nblk,
-                           leaf_ptr, leaf_idx, diag4, x, co, n, p.n_work, p.pstride, (const double*)part, y);
+                           leaf_ptr, leaf_idx, diag4, x, co, n, p.n_work, p.pstride, (const double*)part, next, y);
     }
     hip_check(hipGetLastError(), "k_near_spmv launch");
 }
@@ -989,7 +1001,7 @@ static void fly_launch(hipStream_t s, const SpmvPlan& p, const int* leaf_ptr, co
     const CopyOffsets co{{0, 0}};
     hipLaunchKernelGGL((k_near_spmv_sum<TA>), dim3(unsigned(p.n_groups), 1u), dim3(256), 0, s, p.groups,
                        p.group_nblk, leaf_ptr, leaf_idx, diag4, x, co, n, p.n_work, FLY_RB,
-                       (const TA*)part, y);
+                       (const TA*)part, static_cast<unsigned*>(nullptr), y);
     hip_check(hipGetLastError(), "k_near_spmv_sum launch");
 }
 
@@ -1043,8 +1055,8 @@ __global__ __launch_bounds__(256) void k_pair_coeffs(long long n_pairs, const in
             atomicAdd(repaired, 1u);
         }
     }
-    c64[2 * k] = make_double2(out[0], out[1]);
-    c64[2 * k + 1] = make_double2(out[2], out[3]);
+    c64[coef64_at(k)] = make_double2(out[0], out[1]);
+    c64[coef64_at(k) + COEF64_CD] = make_double2(out[2], out[3]);
     c32[k] = make_float4(float(out[0]), float(out[1]), float(out[2]), float(out[3]));
 }
 

@@ -62,7 +62,9 @@ def test_direct_matvec_against_oracle(levels, nbsize, kappa):
         print(n, nbsize, kappa, p, rel(y, ref), tol, flush=True)
         assert rel(y, ref) < tol
         d.set_overlap(False)
-        assert np.array_equal(d.matvec(x, p), y)
+        for cap in (0, 1):  # one block per work item; blocks that take the next free one
+            d.set_spmv_residency(cap)
+            assert np.array_equal(d.matvec(x, p), y)
         d.set_overlap(True)
     # sets made for either form of the direct far field serve both modes
     d.set_far_field("direct", 5, 40)

@@ -5,7 +5,7 @@ import pytest
 
 from beep3_amd import configs
 from beep3_amd.device import Device
-from beep3_amd.scene import Scene
+from beep3_amd.scene import Mesh, Scene
 
 pytestmark = pytest.mark.gpu
 
@@ -164,3 +164,35 @@ def test_leaf_pass_folded_into_near_coefficients(off_centre_arrays):
     assert rel(y64, y_dir) < 4e-5
     assert rel(y32, y_dir) < 4e-5
     d.close()
+
+
+# relative interpolation error of a well-separated box pair at kappa h = 1.6
+# (the coarsest translated boxes of this scene), orders 3..6, computed from the
+# node interpolation itself; the far field is part of the mat-vec, so its
+# error relative to the whole stays below
+SMALL = {3: 4.0e-2, 4: 5.2e-3, 5: 9.5e-4, 6: 1.2e-4}
+
+
+@pytest.mark.parametrize("order", [3, 4, 5, 6])
+@pytest.mark.parametrize("leaf", [2000, 250, 40, 5])
+def test_fmm_small_scenes(order, leaf):
+    """Every order's M2L blocks at chunk remainders, on trees of 0 to 5 levels
+    (without translated levels the FMM is the direct sum)."""
+    sc = Scene(80.0, 0.125, 6, 0, 100)
+    for k, lv in enumerate((3, 2)):
+        sc.add_instance(Mesh.star(lv, 25.0, 8, 0.04, 9 + k), 2.0, offset=[60.0 * k, 0.0, 5.0 * k])
+    a = sc.build().arrays()
+    x = np.random.default_rng(order).normal(size=2 * a["area"].shape[0])
+    dd = _device(a, 0.125, "direct", precs=("fp64", "fp32"))
+    df = _device(a, 0.125, "fmm", order, leaf, precs=("fp64", "fp32"))
+    levels = df.far_info()["leaf_level"]
+    for p, fp32 in (("fp64", 0.0), ("fp32", 5e-6), ("fp32_resid", 0.0)):
+        y, ref = df.matvec(x, p), dd.matvec(x, p)
+        print(order, leaf, levels, p, rel(y, ref), flush=True)
+        assert np.all(np.isfinite(y))
+        assert rel(y, ref) < (SMALL[order] if levels >= 2 else 1e-6) + fp32
+        df.set_overlap(False)
+        assert np.array_equal(df.matvec(x, p), y)
+        df.set_overlap(True)
+    dd.close()
+    df.close()
