@@ -115,6 +115,12 @@ struct beep_hip_ctx {
     DevBuf<int> qual_ptr, quad_ptr, gal_ptr;
     DevBuf<Pt64> qual64, quad64, gal64;
     DevBuf<Pt32> qual32, quad32;
+    // planar runs of the quadrature and galerkin points (PointPlanes; gs 0: none)
+    DevBuf<double4> quad_plane, gal_plane;
+    DevBuf<float> quad_radius, gal_radius;
+    DevBuf<float4> quad_xyzw;
+    DevBuf<int> plane_bad;
+    PointPlanes quad_planes, gal_planes;
     DevBuf<double> stage;  // raw point upload staging (7 doubles per point)
     DevBuf<double> sverts; // surface for point generation
     DevBuf<int> stris, svt_ptr, svt_tri, svt_corner;
@@ -532,7 +538,7 @@ void matvec_dev(beep_hip_ctx* c, const double* dx, double* dy, int precision) {
     } else if (c->near_mode == BEEP_NEAR_ON_THE_FLY) {
         launch_near_fly(s, mode, c->N, c->fly, c->leaf_ptr.p, c->leaf_idx.p, c->nb_ptr.p, c->nb_idx.p,
                         c->patches.p, c->qual_ptr.p, c->qual32.p, c->qual64.p, c->quad_ptr.p, c->quad32.p,
-                        c->quad64.p, c->kappa, fold ? 0 : 1, c->use_fmm ? c->fmm->cellkey : nullptr, c->fly_ns64 ? 1 : 0,
+                        c->quad64.p, c->quad_planes, c->kappa, fold ? 0 : 1, c->use_fmm ? c->fmm->cellkey : nullptr, c->fly_ns64 ? 1 : 0,
                         c->guard_max, c->diag.p, dx, c->spmv_part.p, dy);
     } else {
         launch_near_spmv(s, mode, c->N, c->spmv, c->leaf_ptr.p, c->leaf_idx.p, c->nb_ptr.p,
@@ -836,6 +842,25 @@ int beep_hip_destroy(beep_hip_ctx* ctx) {
     return 0;
 }
 
+// The planar runs of gs points of a point set (gs 0: none), or none where any
+// patch's points are not such runs.
+static void point_planes(beep_hip_ctx* ctx, int N, const DevBuf<int>& ptr, const DevBuf<Pt64>& pts, int total, int gs,
+                         DevBuf<double4>& plane, DevBuf<float>& radius, DevBuf<float4>* xyzw, PointPlanes& out) {
+    out = PointPlanes{};
+    if (gs < MIN_RUN || total % gs != 0) return;
+    hipStream_t s = ctx->stream;
+    plane.alloc(size_t(total) / gs);
+    radius.alloc(size_t(N));
+    if (xyzw) xyzw->alloc(size_t(total) + 1);
+    ctx->plane_bad.alloc(1);
+    launch_set_int(s, ctx->plane_bad.p, 0);
+    launch_point_planes(s, N, ptr.p, pts.p, gs, plane.p, radius.p, xyzw ? xyzw->p : nullptr, ctx->plane_bad.p);
+    int bad = 0;
+    hip_check(hipMemcpyAsync(&bad, ctx->plane_bad.p, sizeof(int), hipMemcpyDeviceToHost, s), "D2H point planes");
+    hip_check(hipStreamSynchronize(s), "sync point planes");
+    if (bad == 0) out = PointPlanes{plane.p, radius.p, xyzw ? xyzw->p : nullptr, gs};
+}
+
 int beep_hip_set_geometry(beep_hip_ctx* ctx, const beep_hip_geometry* g) {
     return guarded(ctx, [&] {
         require(g && g->n_patches > 0, "empty geometry");
@@ -871,7 +896,7 @@ int beep_hip_set_geometry(beep_hip_ctx* ctx, const beep_hip_geometry* g) {
         auto points = [&](const int* hptr, const int* dptr, const double* raw, DevBuf<Pt64>& o64,
                           DevBuf<Pt32>* o32) {
             const int total = hptr[N];
-            o64.alloc(size_t(total));
+            o64.alloc(size_t(total) + 1);  // one behind the last: PointPlanes
             if (o32) o32->alloc(size_t(total));
             for (int k0 = 0; k0 < total; k0 += CHUNK) {
                 const int n = std::min(CHUNK, total - k0);
@@ -884,6 +909,19 @@ int beep_hip_set_geometry(beep_hip_ctx* ctx, const beep_hip_geometry* g) {
         points(g->qual_ptr, ctx->qual_ptr.p, g->qual_pts, ctx->qual64, &ctx->qual32);
         points(g->quad_ptr, ctx->quad_ptr.p, g->quad_pts, ctx->quad64, &ctx->quad32);
         points(g->gal_ptr, ctx->gal_ptr.p, g->gal_pts, ctx->gal64, nullptr);
+        // points of planar triangles: the shortest run of equal normals over the
+        // first patches gives the length, the device checks every patch
+        auto shortest_run = [&](const int* ptr, const double* pts) {
+            int run = 0x7fffffff, k = 1;
+            for (int p = 0, a = ptr[0]; p < std::min(N, 64); ++p)
+                for (k = a; k < ptr[p + 1]; run = std::min(run, k - a), a = k)
+                    while (k < ptr[p + 1] && std::equal(pts + 7 * k + 3, pts + 7 * k + 6, pts + 7 * a + 3)) ++k;
+            return run;
+        };
+        point_planes(ctx, N, ctx->quad_ptr, ctx->quad64, g->quad_ptr[N], shortest_run(g->quad_ptr, g->quad_pts),
+                     ctx->quad_plane, ctx->quad_radius, &ctx->quad_xyzw, ctx->quad_planes);
+        point_planes(ctx, N, ctx->gal_ptr, ctx->gal64, g->gal_ptr[N], shortest_run(g->gal_ptr, g->gal_pts),
+                     ctx->gal_plane, ctx->gal_radius, nullptr, ctx->gal_planes);
         hip_check(hipStreamSynchronize(s), "sync geometry upload");
         geometry_done(ctx, N, g->centroid);
     });
@@ -953,7 +991,7 @@ int beep_hip_set_surface(beep_hip_ctx* ctx, const beep_hip_surface* g) {
                 ptr[p + 1] = ptr[p] + int(c);
             }
             dptr.upload(ptr.data(), N + 1, s);
-            o64.alloc(size_t(ptr[N]));
+            o64.alloc(size_t(ptr[N]) + 1);  // one behind the last: PointPlanes
             if (o32) o32->alloc(size_t(ptr[N]));
             launch_gen_points(s, N, ctx->sverts.p, ctx->stris.p, ctx->svt_ptr.p, ctx->svt_tri.p,
                               ctx->svt_corner.p, g->ctl_idx ? ctx->sctl_idx.p : nullptr,
@@ -963,7 +1001,18 @@ int beep_hip_set_surface(beep_hip_ctx* ctx, const beep_hip_surface* g) {
         };
         make(g->qual_rule, ctx->qual_ptr, ctx->qual64, &ctx->qual32, 1);
         make(g->quad_rule, ctx->quad_ptr, ctx->quad64, &ctx->quad32, 0);
+        const int nq_quad = ptr[N];
         make(4, ctx->gal_ptr, ctx->gal64, nullptr, 0);
+        const int nq_gal = ptr[N];
+        // a planar triangle's two sub-triangles share its plane
+        const bool planar = NC == 0;
+        auto runs = [&](int order) {
+            return planar && order != 0 ? 2 * int(beep::rule_for_order(order).w.size()) : 0;
+        };
+        point_planes(ctx, N, ctx->quad_ptr, ctx->quad64, nq_quad, runs(g->quad_rule), ctx->quad_plane,
+                     ctx->quad_radius, &ctx->quad_xyzw, ctx->quad_planes);
+        point_planes(ctx, N, ctx->gal_ptr, ctx->gal64, nq_gal, runs(4), ctx->gal_plane, ctx->gal_radius,
+                     nullptr, ctx->gal_planes);
         geometry_done(ctx, N, g->centroid);
     });
 }
@@ -1256,7 +1305,7 @@ void precompute_shared(beep_hip_ctx* ctx, double kappa, int precision) {
     launch_set_int(s, reinterpret_cast<int*>(gcnt + 1), 0);
     launch_set_int(s, reinterpret_cast<int*>(gcnt + 2), 0);
     launch_pair_coeffs(s, ctx->n_pairs, ctx->pair_i.p, ctx->pair_col.p, ctx->patches.p, ctx->qual_ptr.p,
-                       ctx->qual64.p, ctx->quad_ptr.p, ctx->quad64.p, kappa, ctx->guard_max, gcnt + 1,
+                       ctx->qual64.p, ctx->quad_ptr.p, ctx->quad64.p, ctx->quad_planes, kappa, ctx->guard_max, gcnt + 1,
                        ctx->pcoef32.p, ctx->pcoef64.p);
     ctx->have_diag = true;
     ctx->have64 = h->have64;
@@ -1339,10 +1388,10 @@ void precompute_impl(beep_hip_ctx* ctx, double kappa, int precision) {
         launch_near_coeffs_fp64(s, ctx->n_coef_blocks, ctx->L, ctx->coef_blk.p, ctx->leaf_ptr.p,
                                 ctx->leaf_idx.p, ctx->nb_ptr.p, ctx->nb_idx.p, ctx->coef_off.p,
                                 ctx->patches.p, ctx->qual_ptr.p, ctx->qual64.p, ctx->quad_ptr.p,
-                                ctx->quad64.p, kappa, sub_1pt, cellkey, guard, ctx->guard_max,
+                                ctx->quad64.p, ctx->quad_planes, kappa, sub_1pt, cellkey, guard, ctx->guard_max,
                                 ctx->coef64.p);
         launch_coef_repair(s, 0, guard, ctx->patches.p, ctx->qual_ptr.p, ctx->qual64.p,
-                           ctx->quad_ptr.p, ctx->quad64.p, kappa, ctx->guard_max, gcnt + 1,
+                           ctx->quad_ptr.p, ctx->quad64.p, ctx->quad_planes, kappa, ctx->guard_max, gcnt + 1,
                            ctx->coef64.p);
         ctx->have64 = true;
         ctx->uid64 = uid;
@@ -1366,12 +1415,12 @@ void precompute_impl(beep_hip_ctx* ctx, double kappa, int precision) {
         launch_near_coeffs_fp32(s, ctx->n_coef_blocks, ctx->L, ctx->coef_blk.p, ctx->leaf_ptr.p,
                                 ctx->leaf_idx.p, ctx->nb_ptr.p, ctx->nb_idx.p, ctx->coef_off.p,
                                 ctx->patches.p, ctx->qual_ptr.p, ctx->qual32.p, ctx->quad_ptr.p,
-                                ctx->quad32.p, float(kappa), sub_1pt, cellkey, ns, guard,
+                                ctx->quad32.p, ctx->quad_planes, float(kappa), sub_1pt, cellkey, ns, guard,
                                 ctx->guard_max, ctx->coef32.p);
         launch_near_fix64(s, ns, ctx->patches.p, ctx->qual_ptr.p, ctx->qual64.p, ctx->quad_ptr.p,
-                          ctx->quad64.p, kappa, ctx->guard_max, gcnt + 2, ctx->coef32.p);
+                          ctx->quad64.p, ctx->quad_planes, kappa, ctx->guard_max, gcnt + 2, ctx->coef32.p);
         launch_coef_repair(s, 1, guard, ctx->patches.p, ctx->qual_ptr.p, ctx->qual64.p,
-                           ctx->quad_ptr.p, ctx->quad64.p, kappa, ctx->guard_max, gcnt + 2,
+                           ctx->quad_ptr.p, ctx->quad64.p, ctx->quad_planes, kappa, ctx->guard_max, gcnt + 2,
                            ctx->coef32.p);
         ctx->ns_listed = ctx->ns_fp64;
         ctx->have32 = true;
@@ -1689,7 +1738,7 @@ int beep_hip_sanity_check(beep_hip_ctx* ctx, long long* repaired) {
                              ctx->leaf_idx.p, ctx->nb_ptr.p, ctx->nb_idx.p, ctx->coef_off.p, cellkey,
                              folded(ctx, fp32 ? BEEP_FP32 : BEEP_FP64) ? 0 : 1, coef, ctx->guard_max, guard);
             launch_coef_repair(s, fp32, guard, ctx->patches.p, ctx->qual_ptr.p, ctx->qual64.p,
-                               ctx->quad_ptr.p, ctx->quad64.p, ctx->kappa, ctx->guard_max, gcnt + 4,
+                               ctx->quad_ptr.p, ctx->quad64.p, ctx->quad_planes, ctx->kappa, ctx->guard_max, gcnt + 4,
                                coef);
         }
         unsigned h = 0;
@@ -1832,7 +1881,7 @@ int beep_hip_matvec_device_noalloc(beep_hip_ctx* ctx, const double* dx, double* 
         if (fly)
             launch_near_fly(s, mode, N, ctx->fly, ctx->leaf_ptr.p, ctx->leaf_idx.p, ctx->nb_ptr.p,
                             ctx->nb_idx.p, ctx->patches.p, ctx->qual_ptr.p, ctx->qual32.p, ctx->qual64.p,
-                            ctx->quad_ptr.p, ctx->quad32.p, ctx->quad64.p, ctx->kappa, fold ? 0 : 1, nullptr,
+                            ctx->quad_ptr.p, ctx->quad32.p, ctx->quad64.p, ctx->quad_planes, ctx->kappa, fold ? 0 : 1, nullptr,
                             ctx->fly_ns64 ? 1 : 0, ctx->guard_max, ctx->diag.p, dx, spart, dy);
         else
             launch_near_spmv(s, mode, N, ctx->spmv, ctx->leaf_ptr.p, ctx->leaf_idx.p, ctx->nb_ptr.p,
@@ -2095,7 +2144,7 @@ int beep_hip_energy_coefficients(beep_hip_ctx* ctx, int n_inst, const int* ipp, 
         cp.upload(icp, n_inst + 1, ctx->stream);
         ef.alloc(N);
         eh.alloc(N);
-        launch_energy_coeffs(ctx->stream, N, ctx->gal_ptr.p, ctx->gal64.p, ctx->patches.p, pi.p,
+        launch_energy_coeffs(ctx->stream, N, ctx->gal_ptr.p, ctx->gal64.p, ctx->patches.p, ctx->gal_planes, pi.p,
                              cp.p, q.p, ef.p, eh.p);
         hip_check(hipMemcpyAsync(ec_f, ef.p, sizeof(double) * N, hipMemcpyDeviceToHost,
                                  ctx->stream), "D2H ec_f");
@@ -2338,6 +2387,7 @@ int beep_hip_memory_held(beep_hip_ctx* ctx, size_t* bytes) {
         auto add = [&](const auto& buf) { b += buf.n * sizeof(*buf.p); };
         add(ctx->patches); add(ctx->gc); add(ctx->qual_ptr); add(ctx->quad_ptr); add(ctx->gal_ptr);
         add(ctx->qual64); add(ctx->quad64); add(ctx->gal64); add(ctx->qual32); add(ctx->quad32);
+        add(ctx->quad_plane); add(ctx->gal_plane); add(ctx->quad_radius); add(ctx->gal_radius); add(ctx->quad_xyzw);
         add(ctx->stage); add(ctx->sverts); add(ctx->stris); add(ctx->svt_ptr); add(ctx->svt_tri);
         add(ctx->svt_corner);
         add(ctx->leaf_ptr); add(ctx->leaf_idx); add(ctx->nb_ptr); add(ctx->nb_idx);

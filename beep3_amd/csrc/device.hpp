@@ -48,14 +48,16 @@ __device__ __forceinline__ int xcd_remap(int b, int n) {
     return x * q + min(x, r) + k;
 }
 
-// 1/sqrt(v) in FP64: the hardware estimate refined by two Newton steps
-// y <- y + y (1/2 - (v/2) y^2), within an ulp or two of the correctly
-// rounded value and several times cheaper than 1.0 / sqrt(v)
+// 1/sqrt(v) in FP64: the hardware estimate y (relative error below 2^-24)
+// refined by the series of (1 - e)^(-1/2) to second order in e = 1 - v y^2,
+// whose third-order remainder is below 2^-70.  Five operations, where two
+// Newton steps take seven, and the same error: within 1.25 x 2^-53 of the exact
+// value, 0.475 x 2^-53 in the mean square (4 million values each around 1, small,
+// large and near either end of the range).
 __device__ __forceinline__ double rsqrt_nr(double v) {
-    double y = __builtin_amdgcn_rsq(v);
-    const double h = 0.5 * v;
-    y = fma(y, fma(-h * y, y, 0.5), y);
-    return fma(y, fma(-h * y, y, 0.5), y);
+    const double y = __builtin_amdgcn_rsq(v);
+    const double e = fma(-(v * y), y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
 }
 
 // FMM leaf cell of a patch packed as x | y << 10 | z << 20 (leaf level
@@ -121,6 +123,23 @@ struct DevArena {
     }
 };
 
+// A point set whose points come in runs of gs that lie in one plane and share
+// its unit normal (a planar triangle's points): per run the normal n and n.p
+// (local frame, FP64), and per patch an upper bound of |p|; for FP32 kernels the
+// points again as position and weight alone.  Both point arrays have one unused
+// entry behind the last (the kernels load one point ahead).  gs = 0: no such structure (curved triangles).  Run of a patch's first
+// point k: k / gs.
+struct PointPlanes {
+    const double4* plane = nullptr;
+    const float* radius = nullptr;
+    const float4* xyzw = nullptr;
+    int gs = 0;
+};
+// Shorter runs keep a normal per point: the FP32 precompute of 4,002 patches with
+// one point per sub-triangle (runs of 2) took 241 us so and 257 us by runs.  8 is
+// the next length a rule gives: 483 us and 384 us by runs (FP64: 935 and 699).
+constexpr int MIN_RUN = 4;
+
 // ---- launchers (defined in the .hip files) ----
 // singular self terms; a bad one (|v| > maxv or not finite) is zeroed and
 // counted in *repaired; guard_only: check the stored terms and recompute only
@@ -156,14 +175,14 @@ void launch_near_coeffs_fp32(hipStream_t s, int n_blocks, int n_leaves, const in
                              const int* leaf_ptr, const int* leaf_idx, const int* nb_ptr,
                              const int* nb_idx, const int64_t* coef_off, const Patch64* patches,
                              const int* qual_ptr, const Pt32* qual, const int* quad_ptr,
-                             const Pt32* quad, float kappa, int subtract_1pt,
+                             const Pt32* quad, const PointPlanes& planes, float kappa, int subtract_1pt,
                              const unsigned* cellkey, const NsList& ns, const NsList& guard,
                              double maxv, float4* coef);
 // the FP64 pass over the near-singular entries the FP32 kernel listed (a bad
 // result is zeroed and counted in *repaired)
 void launch_near_fix64(hipStream_t s, const NsList& ns, const Patch64* patches, const int* qual_ptr,
-                       const Pt64* qual, const int* quad_ptr, const Pt64* quad, double kappa,
-                       double maxv, unsigned* repaired, float4* coef);
+                       const Pt64* qual, const int* quad_ptr, const Pt64* quad, const PointPlanes& planes,
+                       double kappa, double maxv, unsigned* repaired, float4* coef);
 // coefficient guard: list the entries of a stored set with a value |v| >
 // maxv or not finite (the coefficient kernels list theirs as they go), then
 // recompute the listed ones in FP64 (zero if still bad, or a self pair)
@@ -173,12 +192,12 @@ void launch_coef_scan(hipStream_t s, int fp32, int n_blocks, int n_leaves, const
                       const void* coef, double maxv, const NsList& out);
 void launch_coef_repair(hipStream_t s, int fp32, const NsList& list, const Patch64* patches,
                         const int* qual_ptr, const Pt64* qual, const int* quad_ptr, const Pt64* quad,
-                        double kappa, double maxv, unsigned* repaired, void* coef);
+                        const PointPlanes& planes, double kappa, double maxv, unsigned* repaired, void* coef);
 void launch_near_coeffs_fp64(hipStream_t s, int n_blocks, int n_leaves, const int* blk_ptr,
                              const int* leaf_ptr, const int* leaf_idx, const int* nb_ptr,
                              const int* nb_idx, const int64_t* coef_off, const Patch64* patches,
                              const int* qual_ptr, const Pt64* qual, const int* quad_ptr,
-                             const Pt64* quad, double kappa, int subtract_1pt,
+                             const Pt64* quad, const PointPlanes& planes, double kappa, int subtract_1pt,
                              const unsigned* cellkey, const NsList& guard, double maxv,
                              double2* coef);
 
@@ -220,7 +239,8 @@ void launch_near_spmv(hipStream_t s, int mode, int n, const SpmvPlan& p, const i
 void launch_near_fly(hipStream_t s, int mode, int n, const SpmvPlan& p, const int* leaf_ptr,
                      const int* leaf_idx, const int* nb_ptr, const int* nb_idx, const Patch64* patches,
                      const int* qual_ptr, const Pt32* qual32, const Pt64* qual64, const int* quad_ptr,
-                     const Pt32* quad32, const Pt64* quad64, double kappa, int subtract_1pt, const unsigned* cellkey,
+                     const Pt32* quad32, const Pt64* quad64, const PointPlanes& planes, double kappa, int subtract_1pt,
+                     const unsigned* cellkey,
                      int ns64, double maxv, const double* diag4, const double* x, void* part, double* y);
 
 // explicit pairs listed one by one: coefficients (FP64, rounded to FP32 as
@@ -228,8 +248,8 @@ void launch_near_fly(hipStream_t s, int mode, int n, const SpmvPlan& p, const in
 // rows that have pairs (CSR: rows, ptr, col; mode as launch_near_spmv)
 void launch_pair_coeffs(hipStream_t s, long long n_pairs, const int* pi, const int* pj,
                         const Patch64* patches, const int* qual_ptr, const Pt64* qual, const int* quad_ptr,
-                        const Pt64* quad, double kappa, double maxv, unsigned* repaired, float4* c32,
-                        double2* c64);
+                        const Pt64* quad, const PointPlanes& planes, double kappa, double maxv,
+                        unsigned* repaired, float4* c32, double2* c64);
 void launch_pair_spmv(hipStream_t s, int mode, int n, int n_rows, const int* rows, const int* ptr,
                       const int* col, const float4* c32, const double2* c64, const double* x, double* y);
 // pairs between copies (contiguous ranges of ns patches at copy_off) closer
@@ -283,7 +303,7 @@ void launch_rhs(hipStream_t s, int n, const int* qual_ptr, const Pt64* qual,
                 const Patch64* patches, int n_charges, const double* xyzq, double scale,
                 double* b);
 void launch_energy_coeffs(hipStream_t s, int n, const int* gal_ptr, const Pt64* gal,
-                          const Patch64* patches, const int* patch_inst,
+                          const Patch64* patches, const PointPlanes& planes, const int* patch_inst,
                           const int* inst_charge_ptr, const double* xyzq, double* ec_f,
                           double* ec_h);
 
@@ -330,6 +350,10 @@ void launch_gen_points(hipStream_t s, int n, const double* verts, const int* tri
                        const int* ctl_idx, const double* ctl, const Patch64* patches,
                        const int* ptr, const RuleDev& rule, int per_area, Pt64* out64,
                        Pt32* out32);
+// planes and radii of a point set in runs of gs; *bad counts the patches whose
+// points are not (the outputs then hold nothing usable); xyzw may be null
+void launch_point_planes(hipStream_t s, int n, const int* ptr, const Pt64* pts, int gs, double4* plane,
+                         float* radius, float4* xyzw, int* bad);
 // raw CSR points k0 .. k0+n-1 (7 doubles each) -> local-frame records
 void launch_to_local(hipStream_t s, int n, int k0, const double* raw, const int* ptr, int N,
                      const Patch64* patches, Pt64* out64, Pt32* out32);

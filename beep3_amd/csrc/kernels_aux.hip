@@ -162,13 +162,93 @@ __global__ __launch_bounds__(64) void k_energy_coeffs(int n, const int* __restri
     }
 }
 
+// The same for points in planar runs (PointPlanes).  n.r is one number per run
+// and charge, so a point adds only w/r and w/r^3: 16 FP64 operations, the
+// reciprocal root's among them, against 28 with a normal per point.  The points are read
+// through scalar loads (every lane the same one), with no LDS and no barrier;
+// the coincidence test is run only where a charge is within the patch's reach
+// (rare, so per wave).  Charges two per lane, as above.
+template <bool GUARD>
+__device__ __forceinline__ void energy_run(const Pt64* __restrict__ pts, int gs, double x, double y, double z,
+                                           double& sh, double& sf) {
+    sh = sf = 0.0;
+#pragma unroll 4
+    for (int k = 0; k < gs; ++k) {
+        const double rx = x + pts[k].x, ry = y + pts[k].y, rz = z + pts[k].z;
+        const double d2 = rx * rx + ry * ry + rz * rz;
+        double id = rsqrt_nr(d2);
+        if constexpr (GUARD) id = d2 <= 2.220446049250313e-16 ? 0.0 : id;
+        const double wid = pts[k].w * id;
+        sh += wid;
+        sf = fma(wid, id * id, sf);
+    }
+}
+
+__global__ __launch_bounds__(64) void k_energy_planes(int n, const int* __restrict__ gal_ptr,
+                                                      const Pt64* __restrict__ gal,
+                                                      const Patch64* __restrict__ patches, PointPlanes planes,
+                                                      const int* __restrict__ patch_inst,
+                                                      const int* __restrict__ inst_charge_ptr,
+                                                      const double* __restrict__ xyzq,
+                                                      double* __restrict__ ec_f,
+                                                      double* __restrict__ ec_h) {
+    const int i = blockIdx.x;
+    if (i >= n) return;
+    const int t = threadIdx.x;
+    const int g0 = gal_ptr[i], runs = (gal_ptr[i + 1] - g0) / planes.gs;
+    const int inst = patch_inst[i];
+    const int c0 = inst_charge_ptr[inst], c1 = inst_charge_ptr[inst + 1];
+    const Patch64 p = patches[i];
+    const double4* plane = planes.plane + g0 / planes.gs;
+    const double reach = double(planes.radius[i]) + 1e-7;  // > 1e-7 from every point beyond it
+    double ef = 0, eh = 0;
+    for (int c = c0 + 2 * t; c < c1; c += 128) {
+        // two charges (the second may be past the end: zero charge); positions
+        // of the centroid as seen from them
+        const bool two = c + 1 < c1;
+        const double ax = p.cx - xyzq[4 * c], ay = p.cy - xyzq[4 * c + 1], az = p.cz - xyzq[4 * c + 2];
+        const double aq = xyzq[4 * c + 3];
+        const double bx = two ? p.cx - xyzq[4 * c + 4] : ax, by = two ? p.cy - xyzq[4 * c + 5] : ay;
+        const double bz = two ? p.cz - xyzq[4 * c + 6] : az, bq = two ? xyzq[4 * c + 7] : 0.0;
+        const double nearest = fmin(ax * ax + ay * ay + az * az, bx * bx + by * by + bz * bz);
+        const bool guard = __any(nearest <= reach * reach);
+        for (int g = 0; g < runs; ++g) {
+            const double4 pl = plane[g];
+            const Pt64* pts = gal + g0 + g * planes.gs;
+            double ha, fa, hb, fb;
+            if (guard) {
+                energy_run<true>(pts, planes.gs, ax, ay, az, ha, fa);
+                energy_run<true>(pts, planes.gs, bx, by, bz, hb, fb);
+            } else {
+                energy_run<false>(pts, planes.gs, ax, ay, az, ha, fa);
+                energy_run<false>(pts, planes.gs, bx, by, bz, hb, fb);
+            }
+            eh = fma(aq, ha, fma(bq, hb, eh));
+            ef = fma(-aq * fa, pl.x * ax + pl.y * ay + pl.z * az + pl.w, ef);
+            ef = fma(-bq * fb, pl.x * bx + pl.y * by + pl.z * bz + pl.w, ef);
+        }
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        ef += __shfl_down(ef, off, 64);
+        eh += __shfl_down(eh, off, 64);
+    }
+    if (t == 0) {
+        ec_f[i] = ef * FOUR_PI_INV;
+        ec_h[i] = eh * FOUR_PI_INV;
+    }
+}
+
 void launch_energy_coeffs(hipStream_t s, int n, const int* gal_ptr, const Pt64* gal,
-                          const Patch64* patches, const int* patch_inst,
+                          const Patch64* patches, const PointPlanes& planes, const int* patch_inst,
                           const int* inst_charge_ptr, const double* xyzq, double* ec_f,
                           double* ec_h) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_energy_coeffs, dim3(n), dim3(64), 0, s, n, gal_ptr, gal, patches,
-                       patch_inst, inst_charge_ptr, xyzq, ec_f, ec_h);
+    if (planes.gs)
+        hipLaunchKernelGGL(k_energy_planes, dim3(n), dim3(64), 0, s, n, gal_ptr, gal, patches, planes,
+                           patch_inst, inst_charge_ptr, xyzq, ec_f, ec_h);
+    else
+        hipLaunchKernelGGL(k_energy_coeffs, dim3(n), dim3(64), 0, s, n, gal_ptr, gal, patches,
+                           patch_inst, inst_charge_ptr, xyzq, ec_f, ec_h);
     hip_check(hipGetLastError(), "k_energy_coeffs launch");
 }
 
@@ -554,6 +634,52 @@ void launch_gen_points(hipStream_t s, int n, const double* verts, const int* tri
                        vt_ptr, vt_tri, vt_corner, ctl_idx, ctl, patches, ptr, rule, per_area,
                        out64, out32);
     hip_check(hipGetLastError(), "k_gen_points launch");
+}
+
+// Planes of the runs of gs points of every patch, and its points' largest
+// distance from the centroid (rounded up).  A wave per patch, lanes over its
+// points; a patch whose points are not whole runs with one normal in one plane
+// is counted in *bad (a point may be off its run's plane by rounding only: 1e-12
+// of the patch's size).
+__global__ __launch_bounds__(256) void k_point_planes(int n, const int* __restrict__ ptr,
+                                                      const Pt64* __restrict__ pts, int gs,
+                                                      double4* __restrict__ plane, float* __restrict__ radius,
+                                                      float4* __restrict__ xyzw, int* __restrict__ bad) {
+    const int p = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+    if (p >= n) return;  // the whole wave
+    const int k0 = ptr[p], m = ptr[p + 1] - k0;
+    if (m % gs != 0 || k0 % gs != 0) {
+        if (l == 0) atomicAdd(bad, 1);
+        return;
+    }
+    double r2 = 0;
+    for (int k = l; k < m; k += 64) {
+        const Pt64 q = pts[k0 + k];
+        r2 = fmax(r2, q.x * q.x + q.y * q.y + q.z * q.z);
+    }
+    for (int off = 32; off > 0; off >>= 1) r2 = fmax(r2, __shfl_xor(r2, off, 64));
+    const double tol = 1e-12 * sqrt(r2) + 1e-300;
+    bool ok = true;
+    for (int k = l; k < m; k += 64) {
+        const Pt64 q = pts[k0 + k], f = pts[k0 + k - k % gs];
+        const double fp = f.nx * f.x + f.ny * f.y + f.nz * f.z;
+        ok = ok && q.nx == f.nx && q.ny == f.ny && q.nz == f.nz &&
+             fabs(f.nx * q.x + f.ny * q.y + f.nz * q.z - fp) <= tol;
+        if (k % gs == 0) plane[(k0 + k) / gs] = make_double4(f.nx, f.ny, f.nz, fp);
+        if (xyzw) xyzw[k0 + k] = make_float4(float(q.x), float(q.y), float(q.z), float(q.w));
+    }
+    if (!__all(ok)) {
+        if (l == 0) atomicAdd(bad, 1);
+    } else if (l == 0) {
+        radius[p] = float(sqrt(r2)) * 1.000001f;
+    }
+}
+
+void launch_point_planes(hipStream_t s, int n, const int* ptr, const Pt64* pts, int gs, double4* plane,
+                         float* radius, float4* xyzw, int* bad) {
+    if (n <= 0) return;
+    hipLaunchKernelGGL(k_point_planes, dim3((n + 3) / 4), dim3(256), 0, s, n, ptr, pts, gs, plane, radius, xyzw, bad);
+    hip_check(hipGetLastError(), "k_point_planes launch");
 }
 
 // Points k0 .. k0+n-1 of a CSR point set (raw: 7 doubles x, y, z, nx, ny,

@@ -53,13 +53,7 @@ struct FarMath<float> {
 };
 template <>
 struct FarMath<double> {
-    // hardware estimate refined by two Newton steps y <- y + y (1/2 - (v/2) y^2)
-    static __device__ __forceinline__ double rsqrt_(double v) {
-        double y = __builtin_amdgcn_rsq(v);
-        const double h = 0.5 * v;
-        y = fma(y, fma(-h * y, y, 0.5), y);
-        return fma(y, fma(-h * y, y, 0.5), y);
-    }
+    static __device__ __forceinline__ double rsqrt_(double v) { return rsqrt_nr(v); }
     static __device__ __forceinline__ double exp_(double v) { return exp(v); }
 };
 

@@ -24,6 +24,7 @@ namespace beepdev {
 template <typename T>
 struct Math;
 // e^{-kappa r} = expk(ek * r) with ek = ek_of(kappa) formed once per kernel
+// (kappa >= 0)
 template <>
 struct Math<float> {
     // hardware reciprocal square root (1 ulp)
@@ -36,10 +37,9 @@ struct Math<float> {
 };
 template <>
 struct Math<double> {
-    // hardware estimate refined by two Newton steps y <- y + y (1/2 - (v/2) y^2)
     static __device__ __forceinline__ double rsqrt_(double v) { return rsqrt_nr(v); }
-    static __host__ __device__ __forceinline__ double ek_of(double kappa) { return -kappa; }
-    static __device__ __forceinline__ double expk(double v) { return exp(v); }
+    static __host__ __device__ __forceinline__ double ek_of(double kappa) { return kappa; }
+    static __device__ __forceinline__ double expk(double v) { return exp_neg64(v); }
 };
 
 // Accumulate A..D of one (qual point, quad point) pair into the per-qual-point
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(64) void k_singular(int n, const Patch64* __restric
         double a = 0, b = 0, c = 0, d = 0;
         for (int t = 0; t < np; ++t) {
             const Pt64 p = gal[p0 + t];
-            integrand<double, KAPPA>(kappa, -kappa, inv_eps, p.x - q.x, p.y - q.y, p.z - q.z,
+            integrand<double, KAPPA>(kappa, Math<double>::ek_of(kappa), inv_eps, p.x - q.x, p.y - q.y, p.z - q.z,
                                      q.nx, q.ny, q.nz, p.nx, p.ny, p.nz, p.w, a, b, c, d);
         }
         A += a * q.w;
@@ -188,40 +188,133 @@ __device__ __forceinline__ int find_leaf(const int* __restrict__ blk_ptr, int n_
     return lo;
 }
 
+
+// The points of one planar run share their normal n and n.d = n.(o + p), so B
+// and the second part of D need only sums over the run (o: column centroid
+// less the row's point, FP64; d = o + p):
+//   S0 = sum w/r^3, S1 = sum w c/r^3, S2 = sum w (n0.d) (3 - e h)/r^5,
+//   B -= n.d ((1/eps - 1) S0 + S1),  D -= n.d S2 - n.n0 S1,
+// with c = 1 - e (1 + kr), h = (1 + kr)(2 + kr) + 1 (integrand's terms); C is
+// sum w (n0.d)/r^3 ((1 - 1/eps) + c/eps), its two parts summed apart, and 1 - 1/eps
+// is held as two numbers: rounded to one, its error would be the same in every
+// pair and add up.  n.d comes from the FP64 plane, once per run.  GUARD:
+// coincident points may occur (integrand).
+//
+// Vector operations per point and exponential: 32 in FP32 and 55 in FP64 against
+// 46 and 71 with a normal per point.  The next point is loaded while this one is
+// worked on: without that the FP32 loop waits for the L1 at every point and
+// gains nothing (setup below: 23.8 ms).  Before and after, 72 points a patch:
+// whole setup with a mat-vec, FP32, 163,842 patches, 22.4 -> 17.3 ms; precompute
+// alone, FP64, 4,002 patches, 1.30 -> 0.95 ms.
+template <typename T>
+struct PlanePoint {
+    T x, y, z, w;
+    __device__ __forceinline__ PlanePoint(const float4* xyzw, const Pt<T>* pts) { load(xyzw, pts); }
+    __device__ __forceinline__ void load(const float4* xyzw, const Pt<T>* pts) {
+        if constexpr (sizeof(T) == 4) {
+            const float4 p = *xyzw;
+            x = p.x, y = p.y, z = p.z, w = p.w;
+        } else {
+            x = pts->x, y = pts->y, z = pts->z, w = pts->w;
+        }
+    }
+};
+
+template <typename T, bool KAPPA, bool GUARD>
+__device__ __forceinline__ void pair_planes(double ox64, double oy64, double oz64, T n0x, T n0y, T n0z,
+                                            const double4* __restrict__ plane, int runs, int gs,
+                                            const float4* __restrict__ xyzw, const Pt<T>* __restrict__ pts, T kappa,
+                                            T ek, T ie, T& A, T& B, T& C, T& D) {
+    const T ox = T(ox64), oy = T(oy64), oz = T(oz64);
+    const double ie1d = 1.0 - double(ie);
+    const T ie1 = T(ie1d), ie1lo = T(ie1d - double(ie1));
+    T B0 = 0, B1 = 0, C0 = 0, C1 = 0;
+    PlanePoint<T> next(xyzw, pts);  // the point after this one, in flight
+    for (int g = 0; g < runs; ++g) {
+        const double4 pl = plane[g];
+        T S0 = 0, S1 = 0, S2 = 0;
+        constexpr int UNROLL = sizeof(T) == 4 ? 4 : 2;
+#pragma unroll UNROLL
+        for (int k = 0; k < gs; ++k) {
+            const T dx = ox + next.x, dy = oy + next.y, dz = oz + next.z, w = next.w;
+            next.load(++xyzw, ++pts);
+            const T r2 = dx * dx + dy * dy + dz * dz;
+            T ir = Math<T>::rsqrt_(r2);
+            if constexpr (GUARD) ir = r2 < T(1e-9) ? T(0) : ir;
+            const T ir2 = ir * ir, wir = w * ir, wi = wir * ir2;
+            const T v = wi * (n0x * dx + n0y * dy + n0z * dz);
+            S0 += wi;
+            if constexpr (KAPPA) {
+                const T r = r2 * ir, kr = kappa * r;
+                const T e = Math<T>::expk(ek * r);
+                const T s = T(1) + kr;
+                const T c = fma(-e, s, T(1));
+                A = fma(wir, T(1) - e, A);
+                S1 = fma(wi, c, S1);
+                C0 += v;
+                C1 = fma(v, c, C1);
+                S2 = fma(v * ir2, fma(-e, fma(s, kr + T(2), T(1)), T(3)), S2);
+            } else {
+                C0 += v;
+            }
+        }
+        const T nd = T(pl.x * ox64 + pl.y * oy64 + pl.z * oz64 + pl.w);
+        const T nn = T(pl.x) * n0x + T(pl.y) * n0y + T(pl.z) * n0z;
+        B0 = fma(nd, S0, B0);
+        if constexpr (KAPPA) {
+            B1 = fma(nd, S1, B1);
+            D = fma(nn, S1, fma(-nd, S2, D));
+        }
+    }
+    B += fma(ie1, B0, fma(ie1lo, B0, -B1));
+    C += fma(ie1, C0, fma(ie1lo, C0, ie * C1));
+}
+
 template <typename T, bool KAPPA>
-__device__ __forceinline__ void pair_coeffs(const Patch64& pi, const Patch64& pj, int qb, int qn,
+__device__ __forceinline__ void pair_coeffs(const Patch64& pi, const Patch64& pj, int j, int qb, int qn,
                                             const Pt<T>* __restrict__ qual, int pb, int pn,
-                                            const Pt<T>* __restrict__ quad, T kappa,
+                                            const Pt<T>* __restrict__ quad, const PointPlanes& planes, T kappa,
                                             int subtract_1pt, T out[4]) {
     // centroid difference in FP64, then the working precision
-    const T dcx = T(pj.cx - pi.cx), dcy = T(pj.cy - pi.cy), dcz = T(pj.cz - pi.cz);
+    const double dx64 = pj.cx - pi.cx, dy64 = pj.cy - pi.cy, dz64 = pj.cz - pi.cz;
+    const T dcx = T(dx64), dcy = T(dy64), dcz = T(dz64);
     const T inv_eps = T(pj.inv_eps);
     const T ek = Math<T>::ek_of(kappa);
     T A = 0, B = 0, C = 0, D = 0;
+    if (subtract_1pt) {  // first, so that the records' normals need no registers below
+        integrand<T, KAPPA>(kappa, ek, inv_eps, dcx, dcy, dcz, T(pi.nx), T(pi.ny), T(pi.nz),
+                            T(pj.nx), T(pj.ny), T(pj.nz), -T(pj.area), A, B, C, D);
+    }
     constexpr int UNROLL = sizeof(T) == 4 ? 4 : 2;  // source points per unrolled step
     for (int a = 0; a < qn; ++a) {
         const Pt<T> q = qual[qb + a];
         T a_ = 0, b_ = 0, c_ = 0, d_ = 0;
-        const T ox = dcx - q.x, oy = dcy - q.y, oz = dcz - q.z;
+        if (planes.gs) {
+            const double ox = dx64 - double(q.x), oy = dy64 - double(q.y), oz = dz64 - double(q.z);
+            const double reach = double(planes.radius[j]) + 1e-4;  // |d| > 1e-4 beyond it
+            const int runs = pn / planes.gs;
+            const double4* pl = planes.plane + pb / planes.gs;
+            if (!__any(ox * ox + oy * oy + oz * oz <= reach * reach))  // one form per wave
+                pair_planes<T, KAPPA, false>(ox, oy, oz, q.nx, q.ny, q.nz, pl, runs, planes.gs,
+                                             planes.xyzw + pb, quad + pb, kappa, ek,
+                                             inv_eps, a_, b_, c_, d_);
+            else
+                pair_planes<T, KAPPA, true>(ox, oy, oz, q.nx, q.ny, q.nz, pl, runs, planes.gs,
+                                             planes.xyzw + pb, quad + pb, kappa, ek,
+                                            inv_eps, a_, b_, c_, d_);
+        } else {
+            const T ox = dcx - q.x, oy = dcy - q.y, oz = dcz - q.z;
 #pragma unroll UNROLL
-        for (int k = 0; k < pn; ++k) {
-            const Pt<T> p = quad[pb + k];
-            integrand<T, KAPPA>(kappa, ek, inv_eps, ox + p.x, oy + p.y, oz + p.z, q.nx, q.ny,
-                                q.nz, p.nx, p.ny, p.nz, p.w, a_, b_, c_, d_);
+            for (int k = 0; k < pn; ++k) {
+                const Pt<T> p = quad[pb + k];
+                integrand<T, KAPPA>(kappa, ek, inv_eps, ox + p.x, oy + p.y, oz + p.z, q.nx, q.ny,
+                                    q.nz, p.nx, p.ny, p.nz, p.w, a_, b_, c_, d_);
+            }
         }
         A += a_ * q.w;
         B += b_ * q.w;
         C += c_ * q.w;
         D += d_ * q.w;
-    }
-    if (subtract_1pt) {
-        T a_ = 0, b_ = 0, c_ = 0, d_ = 0;
-        integrand<T, KAPPA>(kappa, ek, inv_eps, dcx, dcy, dcz, T(pi.nx), T(pi.ny), T(pi.nz),
-                            T(pj.nx), T(pj.ny), T(pj.nz), T(pj.area), a_, b_, c_, d_);
-        A -= a_;
-        B -= b_;
-        C -= c_;
-        D -= d_;
     }
     const T k4 = T(FOUR_PI_INV);
     out[0] = A * k4;
@@ -239,7 +332,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 5) void k_near_coeffs(
     const int* __restrict__ nb_idx, const int64_t* __restrict__ coef_off,
     const Patch64* __restrict__ patches, const int* __restrict__ qual_ptr,
     const Pt<T>* __restrict__ qual, const int* __restrict__ quad_ptr,
-    const Pt<T>* __restrict__ quad, T kappa, int subtract_1pt,
+    const Pt<T>* __restrict__ quad, PointPlanes planes, T kappa, int subtract_1pt,
     const unsigned* __restrict__ cellkey, NsList ns, NsList guard, double maxv,
     void* __restrict__ coef) {
     const int b = xcd_remap(blockIdx.x, gridDim.x);
@@ -270,7 +363,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 5) void k_near_coeffs(
                 return;
             }
         }
-        pair_coeffs<T, KAPPA>(pi, pj, qb, qn, qual, pb, pn, quad, kappa, sub, out);
+        pair_coeffs<T, KAPPA>(pi, pj, j, qb, qn, qual, pb, pn, quad, planes, kappa, sub, out);
         const double v[4] = {double(out[0]), double(out[1]), double(out[2]), double(out[3])};
         if (coef4_bad(v, maxv)) {
             // stored as zero; k_coef_repair recomputes it in FP64
@@ -293,7 +386,7 @@ void launch_near_coeffs_fp32(hipStream_t s, int n_blocks, int n_leaves, const in
                              const int* leaf_ptr, const int* leaf_idx, const int* nb_ptr,
                              const int* nb_idx, const int64_t* coef_off, const Patch64* patches,
                              const int* qual_ptr, const Pt32* qual, const int* quad_ptr,
-                             const Pt32* quad, float kappa, int subtract_1pt,
+                             const Pt32* quad, const PointPlanes& planes, float kappa, int subtract_1pt,
                              const unsigned* cellkey, const NsList& ns, const NsList& guard,
                              double maxv, float4* coef) {
     if (n_blocks <= 0) return;
@@ -301,7 +394,7 @@ void launch_near_coeffs_fp32(hipStream_t s, int n_blocks, int n_leaves, const in
     launch_set_int(s, reinterpret_cast<int*>(guard.count), 0);
     auto k = kappa != 0.0f ? k_near_coeffs<float, true> : k_near_coeffs<float, false>;
     hipLaunchKernelGGL(k, dim3(n_blocks), dim3(256), 0, s, n_leaves, blk_ptr, leaf_ptr, leaf_idx,
-                       nb_ptr, nb_idx, coef_off, patches, qual_ptr, qual, quad_ptr, quad, kappa,
+                       nb_ptr, nb_idx, coef_off, patches, qual_ptr, qual, quad_ptr, quad, planes, kappa,
                        subtract_1pt, cellkey, ns, guard, maxv, (void*)coef);
     hip_check(hipGetLastError(), "k_near_coeffs<float> launch");
 }
@@ -314,8 +407,9 @@ __global__ __launch_bounds__(256) void k_near_fix64(NsList ns, const Patch64* __
                                                    const int* __restrict__ qual_ptr,
                                                    const Pt64* __restrict__ qual,
                                                    const int* __restrict__ quad_ptr,
-                                                   const Pt64* __restrict__ quad, double kappa,
-                                                   double maxv, unsigned* __restrict__ repaired,
+                                                   const Pt64* __restrict__ quad, PointPlanes planes,
+                                                   double kappa, double maxv,
+                                                   unsigned* __restrict__ repaired,
                                                    float4* __restrict__ coef) {
     const unsigned n = min(*ns.count, ns.cap);
     for (unsigned k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
@@ -325,7 +419,7 @@ __global__ __launch_bounds__(256) void k_near_fix64(NsList ns, const Patch64* __
         const int qb = qual_ptr[i], qn = qual_ptr[i + 1] - qb;
         const int pb = quad_ptr[j], pn = quad_ptr[j + 1] - pb;
         double out[4];
-        pair_coeffs<double, KAPPA>(pi, pj, qb, qn, qual, pb, pn, quad, kappa, r.j2 & 1, out);
+        pair_coeffs<double, KAPPA>(pi, pj, j, qb, qn, qual, pb, pn, quad, planes, kappa, r.j2 & 1, out);
         const float4 o = make_float4(float(out[0]), float(out[1]), float(out[2]), float(out[3]));
         const double v[4] = {o.x, o.y, o.z, o.w};
         if (coef4_bad(v, maxv)) {
@@ -338,14 +432,14 @@ __global__ __launch_bounds__(256) void k_near_fix64(NsList ns, const Patch64* __
 }
 
 void launch_near_fix64(hipStream_t s, const NsList& ns, const Patch64* patches, const int* qual_ptr,
-                       const Pt64* qual, const int* quad_ptr, const Pt64* quad, double kappa,
-                       double maxv, unsigned* repaired, float4* coef) {
+                       const Pt64* qual, const int* quad_ptr, const Pt64* quad, const PointPlanes& planes,
+                       double kappa, double maxv, unsigned* repaired, float4* coef) {
     if (!ns.rec) return;
     // enough blocks for every CU several times over; each walks the list
     const unsigned blocks = std::max(1u, std::min(2048u, (ns.cap + 255) / 256));
     auto k = kappa != 0.0 ? k_near_fix64<true> : k_near_fix64<false>;
     hipLaunchKernelGGL(k, dim3(blocks), dim3(256), 0, s, ns, patches, qual_ptr, qual, quad_ptr, quad,
-                       kappa, maxv, repaired, coef);
+                       planes, kappa, maxv, repaired, coef);
     hip_check(hipGetLastError(), "k_near_fix64 launch");
 }
 
@@ -392,8 +486,9 @@ __global__ __launch_bounds__(256) void k_coef_repair(NsList list, const Patch64*
                                                      const int* __restrict__ qual_ptr,
                                                      const Pt64* __restrict__ qual,
                                                      const int* __restrict__ quad_ptr,
-                                                     const Pt64* __restrict__ quad, double kappa,
-                                                     double maxv, unsigned* __restrict__ repaired,
+                                                     const Pt64* __restrict__ quad, PointPlanes planes,
+                                                     double kappa, double maxv,
+                                                     unsigned* __restrict__ repaired,
                                                      void* __restrict__ coef) {
     const unsigned n = min(*list.count, list.cap);
     for (unsigned k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
@@ -404,7 +499,7 @@ __global__ __launch_bounds__(256) void k_coef_repair(NsList list, const Patch64*
             const Patch64 pi = patches[i], pj = patches[j];
             const int qb = qual_ptr[i], qn = qual_ptr[i + 1] - qb;
             const int pb = quad_ptr[j], pn = quad_ptr[j + 1] - pb;
-            pair_coeffs<double, KAPPA>(pi, pj, qb, qn, qual, pb, pn, quad, kappa, r.j2 & 1, out);
+            pair_coeffs<double, KAPPA>(pi, pj, j, qb, qn, qual, pb, pn, quad, planes, kappa, r.j2 & 1, out);
             double v[4] = {out[0], out[1], out[2], out[3]};
             if constexpr (sizeof(TC) == 4)
                 for (int q = 0; q < 4; ++q) v[q] = double(float(v[q]));
@@ -436,16 +531,16 @@ void launch_coef_scan(hipStream_t s, int fp32, int n_blocks, int n_leaves, const
 
 void launch_coef_repair(hipStream_t s, int fp32, const NsList& list, const Patch64* patches,
                         const int* qual_ptr, const Pt64* qual, const int* quad_ptr, const Pt64* quad,
-                        double kappa, double maxv, unsigned* repaired, void* coef) {
+                        const PointPlanes& planes, double kappa, double maxv, unsigned* repaired, void* coef) {
     const unsigned blocks = std::max(1u, std::min(256u, (list.cap + 255) / 256));
     if (fp32) {
         auto k = kappa != 0.0 ? k_coef_repair<float, true> : k_coef_repair<float, false>;
         hipLaunchKernelGGL(k, dim3(blocks), dim3(256), 0, s, list, patches, qual_ptr, qual, quad_ptr,
-                           quad, kappa, maxv, repaired, coef);
+                           quad, planes, kappa, maxv, repaired, coef);
     } else {
         auto k = kappa != 0.0 ? k_coef_repair<double, true> : k_coef_repair<double, false>;
         hipLaunchKernelGGL(k, dim3(blocks), dim3(256), 0, s, list, patches, qual_ptr, qual, quad_ptr,
-                           quad, kappa, maxv, repaired, coef);
+                           quad, planes, kappa, maxv, repaired, coef);
     }
     hip_check(hipGetLastError(), "k_coef_repair launch");
 }
@@ -454,14 +549,14 @@ void launch_near_coeffs_fp64(hipStream_t s, int n_blocks, int n_leaves, const in
                              const int* leaf_ptr, const int* leaf_idx, const int* nb_ptr,
                              const int* nb_idx, const int64_t* coef_off, const Patch64* patches,
                              const int* qual_ptr, const Pt64* qual, const int* quad_ptr,
-                             const Pt64* quad, double kappa, int subtract_1pt,
+                             const Pt64* quad, const PointPlanes& planes, double kappa, int subtract_1pt,
                              const unsigned* cellkey, const NsList& guard, double maxv,
                              double2* coef) {
     if (n_blocks <= 0) return;
     launch_set_int(s, reinterpret_cast<int*>(guard.count), 0);
     auto k = kappa != 0.0 ? k_near_coeffs<double, true> : k_near_coeffs<double, false>;
     hipLaunchKernelGGL(k, dim3(n_blocks), dim3(256), 0, s, n_leaves, blk_ptr, leaf_ptr, leaf_idx,
-                       nb_ptr, nb_idx, coef_off, patches, qual_ptr, qual, quad_ptr, quad, kappa,
+                       nb_ptr, nb_idx, coef_off, patches, qual_ptr, qual, quad_ptr, quad, planes, kappa,
                        subtract_1pt, cellkey, NsList{}, guard, maxv, (void*)coef);
     hip_check(hipGetLastError(), "k_near_coeffs<double> launch");
 }
@@ -847,39 +942,44 @@ void launch_direct_matvec(hipStream_t s, int mode, int n, const SpmvPlan& p, con
 // partials, the diagonal, and writes y): deterministic.
 // The FP64 integration of an FP32 pass's near-singular or bad entry, rounded
 // to FP32 (zero if still bad), out of line: rare, and inlined it would take
-// registers from the FP32 loop.
-// It takes indices, not patch records, so the caller keeps nothing on the
-// stack for the call.
+// registers from the FP32 loop.  It takes indices, not patch records, and the
+// planes by value, so the caller keeps nothing on the stack for the call (a
+// reference turns the caller's own loads through them into flat loads).
 template <bool KAPPA>
 __device__ __attribute__((noinline)) float4 fly_redo64(int i, int j, int sub, const Patch64* __restrict__ patches,
                                                        const int* __restrict__ qual_ptr,
                                                        const Pt64* __restrict__ qual64,
                                                        const int* __restrict__ quad_ptr,
-                                                       const Pt64* __restrict__ quad64, double kappa,
-                                                       double maxv) {
+                                                       const Pt64* __restrict__ quad64, PointPlanes planes,
+                                                       double kappa, double maxv) {
     const Patch64 pi = patches[i], pj = patches[j];
     const int qb = qual_ptr[i], qn = qual_ptr[i + 1] - qb;
     const int pb = quad_ptr[j], pn = quad_ptr[j + 1] - pb;
     double o[4];
-    pair_coeffs<double, KAPPA>(pi, pj, qb, qn, qual64, pb, pn, quad64, kappa, sub, o);
+    pair_coeffs<double, KAPPA>(pi, pj, j, qb, qn, qual64, pb, pn, quad64, planes, kappa, sub, o);
     const float4 v = make_float4(float(o[0]), float(o[1]), float(o[2]), float(o[3]));
     const double d[4] = {v.x, v.y, v.z, v.w};
     return coef4_bad(d, maxv) ? make_float4(0.f, 0.f, 0.f, 0.f) : v;
 }
 
 template <typename T, typename TA, bool KAPPA>
-__global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 5) void k_near_fly_part(
+__global__ __launch_bounds__(256, 4) void k_near_fly_part(
     const int4* __restrict__ work, int n_work, const int* __restrict__ leaf_ptr,
     const int* __restrict__ leaf_idx, const int* __restrict__ nb_ptr, const int* __restrict__ nb_idx,
     const Patch64* __restrict__ patches, const int* __restrict__ qual_ptr,
     const Pt<T>* __restrict__ qual, const int* __restrict__ quad_ptr, const Pt<T>* __restrict__ quad,
-    const Pt64* __restrict__ qual64, const Pt64* __restrict__ quad64, double kappa, int subtract_1pt,
-    const unsigned* __restrict__ cellkey, int ns64, double maxv, const double* __restrict__ x, int n,
+    const Pt64* __restrict__ qual64, const Pt64* __restrict__ quad64, PointPlanes planes, double kappa,
+    int subtract_1pt, const unsigned* __restrict__ cellkey, int ns64, double maxv, const double* __restrict__ x, int n,
     TA* __restrict__ part) {
-    // FP32 pass: the near-singular pairs of a thread (up to DEF of them) are
-    // set aside (column and leaf-pass bit) and integrated in FP64 by the
-    // whole block after the loop, so a wave does not run the FP64 path for a
-    // few of its lanes; each thread then adds its own in the order found.
+    // FP32 pass: the near-singular pairs and bad entries of a thread are set
+    // aside (column and leaf-pass bit) and integrated in FP64 by the whole
+    // block after the loop, so a wave does not run the FP64 path for a few of
+    // its lanes; each thread then adds its own in the order found.  A thread
+    // that has DEF of them stops there, and the block comes back to its
+    // columns afterwards (more than DEF of one thread's columns are rare).  At
+    // most 128 VGPRs in FP32 too: at 96 the point loop itself reloads spilled
+    // values.  Mat-vec of 40,962 patches: 11.6 ms at 96, 9.0 at 128 (9.6 before
+    // the planar runs).
     constexpr int DEF = sizeof(T) == 4 ? 4 : 1;
     __shared__ TA xs[2][SPMV_CW];
     __shared__ TA red[2][256];
@@ -901,69 +1001,69 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 5) void k_near_fly_part(
         xs[0][k] = TA(x[j]);
         xs[1][k] = TA(x[n + j]);
     }
+    // a thread has columns left (this round, the next): red is free until the end
+    int* again = reinterpret_cast<int*>(&red[0][0]);
+    int round = 0;
+    if (t == 0) again[0] = 0;
     __syncthreads();
     TA af = 0, ah = 0;
-    int nd = 0;  // pairs this thread set aside
-    if (active) {
-        const int i = leaf_idx[lp + row0 + r];
-        const Patch64 pi = patches[i];
-        const int qb = qual_ptr[i], qn = qual_ptr[i + 1] - qb;
-        const unsigned ki = cellkey ? cellkey[i] : 0u;
-        for (int c = s; c < nc; c += S) {
-            const int j = nb_idx[np + col0 + c];
-            if (j == i) continue;  // the self pair is the diagonal's (stored as zero)
-            const Patch64 pj = patches[j];
-            const int pb = quad_ptr[j], pn = quad_ptr[j + 1] - pb;
-            const int sub = subtract_1pt && !(cellkey && fmm_cells_adjacent(ki, cellkey[j]));
-            T v[4];
-            bool redo = false;
-            if constexpr (sizeof(T) == 4) {
-                redo = ns64 && near_singular(pi, pj);
-                if (redo && nd < DEF) {
-                    dcode[t * DEF + nd] = 2 * c + sub;
-                    ++nd;
-                    continue;
+    int c = active ? s : nc;  // next column of this thread
+    for (;;) {
+        int nd = 0;  // pairs this thread set aside
+        if (c < nc) {
+            const int i = leaf_idx[lp + row0 + r];
+            const Patch64 pi = patches[i];
+            const int qb = qual_ptr[i], qn = qual_ptr[i + 1] - qb;
+            const unsigned ki = cellkey ? cellkey[i] : 0u;
+            for (; c < nc; c += S) {
+                const int j = nb_idx[np + col0 + c];
+                if (j == i) continue;  // the self pair is the diagonal's (stored as zero)
+                const Patch64 pj = patches[j];
+                const int pb = quad_ptr[j], pn = quad_ptr[j + 1] - pb;
+                const int sub = subtract_1pt && !(cellkey && fmm_cells_adjacent(ki, cellkey[j]));
+                T v[4];
+                bool redo = sizeof(T) == 4 && ns64 && near_singular(pi, pj);
+                if (!redo) {
+                    pair_coeffs<T, KAPPA>(pi, pj, j, qb, qn, qual, pb, pn, quad, planes, T(kappa), sub, v);
+                    const double d[4] = {double(v[0]), double(v[1]), double(v[2]), double(v[3])};
+                    if (coef4_bad(d, maxv)) {
+                        // FP64 recomputes what FP64 already gave: zero at once
+                        if constexpr (sizeof(T) == 8) v[0] = v[1] = v[2] = v[3] = T(0);
+                        else redo = true;
+                    }
                 }
-            }
-            if (!redo) {
-                pair_coeffs<T, KAPPA>(pi, pj, qb, qn, qual, pb, pn, quad, T(kappa), sub, v);
-                const double d[4] = {double(v[0]), double(v[1]), double(v[2]), double(v[3])};
-                if (coef4_bad(d, maxv)) {
-                    // FP64 recomputes what FP64 already gave: zero at once
-                    if constexpr (sizeof(T) == 8) v[0] = v[1] = v[2] = v[3] = T(0);
-                    else redo = true;
+                if constexpr (sizeof(T) == 4) {
+                    if (redo) {
+                        if (nd == DEF) break;  // goes on here after the set-aside pairs
+                        dcode[t * DEF + nd] = 2 * c + sub;
+                        ++nd;
+                        continue;
+                    }
                 }
+                const TA xf = xs[0][c], xh = xs[1][c];
+                af += TA(v[1]) * xf - TA(v[0]) * xh;
+                ah += TA(v[3]) * xf - TA(v[2]) * xh;
             }
-            if constexpr (sizeof(T) == 4) {
-                if (redo) {
-                    const float4 o =
-                        fly_redo64<KAPPA>(i, j, sub, patches, qual_ptr, qual64, quad_ptr, quad64, kappa, maxv);
-                    v[0] = o.x;
-                    v[1] = o.y;
-                    v[2] = o.z;
-                    v[3] = o.w;
-                }
-            }
-            const TA xf = xs[0][c], xh = xs[1][c];
-            af += TA(v[1]) * xf - TA(v[0]) * xh;
-            ah += TA(v[3]) * xf - TA(v[2]) * xh;
         }
-    }
-    if constexpr (sizeof(T) == 4) {
+        if constexpr (sizeof(T) == 8) break;
         // the set-aside pairs, spread over the block: entry e belongs to
         // thread e / DEF
         for (int k = nd; k < DEF; ++k) dcode[t * DEF + k] = -1;
+        if (c < nc) again[round] = 1;
         __syncthreads();
+        const bool more = again[round];
+        round ^= 1;
+        if (t == 0) again[round] = 0;
         for (int e = t; e < 256 * DEF; e += 256) {
             const int code = dcode[e];
             if (code < 0) continue;
             const int owner = e / DEF;
-            const int c = code >> 1;
+            const int cc = code >> 1;
             const int i = leaf_idx[lp + row0 + owner % Rb];
-            const int j = nb_idx[np + col0 + c];
-            const float4 o =
-                fly_redo64<KAPPA>(i, j, code & 1, patches, qual_ptr, qual64, quad_ptr, quad64, kappa, maxv);
-            const TA xf = xs[0][c], xh = xs[1][c];
+            const int j = nb_idx[np + col0 + cc];
+            const float4 o = fly_redo64<KAPPA>(i, j, code & 1, patches, qual_ptr, qual64, quad_ptr, quad64, planes,
+                                               kappa, maxv);
+            const TA xf = xs[0][cc], xh = xs[1][cc];
             dprod[0][e] = TA(o.y) * xf - TA(o.x) * xh;
             dprod[1][e] = TA(o.w) * xf - TA(o.z) * xh;
         }
@@ -972,6 +1072,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 5) void k_near_fly_part(
             af += dprod[0][t * DEF + k];
             ah += dprod[1][t * DEF + k];
         }
+        if (!more) break;
     }
     red[0][t] = af;
     red[1][t] = ah;
@@ -991,11 +1092,11 @@ template <typename T, typename TA>
 static void fly_launch(hipStream_t s, const SpmvPlan& p, const int* leaf_ptr, const int* leaf_idx,
                        const int* nb_ptr, const int* nb_idx, const Patch64* patches, const int* qual_ptr,
                        const Pt<T>* qual, const int* quad_ptr, const Pt<T>* quad, const Pt64* qual64,
-                       const Pt64* quad64, double kappa, int subtract_1pt, const unsigned* cellkey, int ns64,
-                       double maxv, const double* diag4, const double* x, int n, TA* part, double* y) {
+                       const Pt64* quad64, const PointPlanes& planes, double kappa, int subtract_1pt,
+                       const unsigned* cellkey, int ns64, double maxv, const double* diag4, const double* x, int n, TA* part, double* y) {
     auto k = kappa != 0.0 ? k_near_fly_part<T, TA, true> : k_near_fly_part<T, TA, false>;
     hipLaunchKernelGGL(k, dim3(unsigned(p.n_work)), dim3(256), 0, s, p.work, p.n_work, leaf_ptr, leaf_idx,
-                       nb_ptr, nb_idx, patches, qual_ptr, qual, quad_ptr, quad, qual64, quad64, kappa,
+                       nb_ptr, nb_idx, patches, qual_ptr, qual, quad_ptr, quad, qual64, quad64, planes, kappa,
                        subtract_1pt, cellkey, ns64, maxv, x, n, part);
     hip_check(hipGetLastError(), "k_near_fly_part launch");
     const CopyOffsets co{{0, 0}};
@@ -1008,20 +1109,21 @@ static void fly_launch(hipStream_t s, const SpmvPlan& p, const int* leaf_ptr, co
 void launch_near_fly(hipStream_t s, int mode, int n, const SpmvPlan& p, const int* leaf_ptr,
                      const int* leaf_idx, const int* nb_ptr, const int* nb_idx, const Patch64* patches,
                      const int* qual_ptr, const Pt32* qual32, const Pt64* qual64, const int* quad_ptr,
-                     const Pt32* quad32, const Pt64* quad64, double kappa, int subtract_1pt, const unsigned* cellkey,
+                     const Pt32* quad32, const Pt64* quad64, const PointPlanes& planes, double kappa, int subtract_1pt,
+                     const unsigned* cellkey,
                      int ns64, double maxv, const double* diag4, const double* x, void* part, double* y) {
     if (p.n_work <= 0) return;
     if (mode == 0)
         fly_launch<double, double>(s, p, leaf_ptr, leaf_idx, nb_ptr, nb_idx, patches, qual_ptr, qual64,
-                                   quad_ptr, quad64, qual64, quad64, kappa, subtract_1pt, cellkey, 0, maxv, diag4, x, n,
+                                   quad_ptr, quad64, qual64, quad64, planes, kappa, subtract_1pt, cellkey, 0, maxv, diag4, x, n,
                                    (double*)part, y);
     else if (mode == 1)
         fly_launch<float, float>(s, p, leaf_ptr, leaf_idx, nb_ptr, nb_idx, patches, qual_ptr, qual32,
-                                 quad_ptr, quad32, qual64, quad64, kappa, subtract_1pt, cellkey, ns64, maxv, diag4, x,
+                                 quad_ptr, quad32, qual64, quad64, planes, kappa, subtract_1pt, cellkey, ns64, maxv, diag4, x,
                                  n, (float*)part, y);
     else
         fly_launch<float, double>(s, p, leaf_ptr, leaf_idx, nb_ptr, nb_idx, patches, qual_ptr, qual32,
-                                  quad_ptr, quad32, qual64, quad64, kappa, subtract_1pt, cellkey, ns64, maxv, diag4, x,
+                                  quad_ptr, quad32, qual64, quad64, planes, kappa, subtract_1pt, cellkey, ns64, maxv, diag4, x,
                                   n, (double*)part, y);
 }
 
@@ -1038,8 +1140,9 @@ __global__ __launch_bounds__(256) void k_pair_coeffs(long long n_pairs, const in
                                                     const int* __restrict__ qual_ptr,
                                                     const Pt64* __restrict__ qual,
                                                     const int* __restrict__ quad_ptr,
-                                                    const Pt64* __restrict__ quad, double kappa,
-                                                    double maxv, unsigned* __restrict__ repaired,
+                                                    const Pt64* __restrict__ quad, PointPlanes planes,
+                                                    double kappa, double maxv,
+                                                    unsigned* __restrict__ repaired,
                                                     float4* __restrict__ c32, double2* __restrict__ c64) {
     const long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x;
     if (k >= n_pairs) return;
@@ -1049,7 +1152,7 @@ __global__ __launch_bounds__(256) void k_pair_coeffs(long long n_pairs, const in
         const Patch64 a = patches[i], b = patches[j];
         const int qb = qual_ptr[i], qn = qual_ptr[i + 1] - qb;
         const int pb = quad_ptr[j], pn = quad_ptr[j + 1] - pb;
-        pair_coeffs<double, KAPPA>(a, b, qb, qn, qual, pb, pn, quad, kappa, 1, out);
+        pair_coeffs<double, KAPPA>(a, b, j, qb, qn, qual, pb, pn, quad, planes, kappa, 1, out);
         if (coef4_bad(out, maxv)) {
             out[0] = out[1] = out[2] = out[3] = 0.0;
             atomicAdd(repaired, 1u);
@@ -1062,12 +1165,12 @@ __global__ __launch_bounds__(256) void k_pair_coeffs(long long n_pairs, const in
 
 void launch_pair_coeffs(hipStream_t s, long long n_pairs, const int* pi, const int* pj,
                         const Patch64* patches, const int* qual_ptr, const Pt64* qual, const int* quad_ptr,
-                        const Pt64* quad, double kappa, double maxv, unsigned* repaired, float4* c32,
-                        double2* c64) {
+                        const Pt64* quad, const PointPlanes& planes, double kappa, double maxv,
+                        unsigned* repaired, float4* c32, double2* c64) {
     if (n_pairs <= 0) return;
     auto k = kappa != 0.0 ? k_pair_coeffs<true> : k_pair_coeffs<false>;
     hipLaunchKernelGGL(k, dim3(unsigned((n_pairs + 255) / 256)), dim3(256), 0, s, n_pairs, pi, pj, patches,
-                       qual_ptr, qual, quad_ptr, quad, kappa, maxv, repaired, c32, c64);
+                       qual_ptr, qual, quad_ptr, quad, planes, kappa, maxv, repaired, c32, c64);
     hip_check(hipGetLastError(), "k_pair_coeffs launch");
 }
 

@@ -1,0 +1,113 @@
+"""Points in planar runs (one plane per triangle of a patch) against the FP64
+CPU oracle: every rule, runs of several lengths, and sets that are not such
+runs, in near coefficients (stored and on the fly) and energy coefficients."""
+import numpy as np
+import pytest
+
+import oracle
+from beep3_amd.device import Device
+from beep3_amd.scene import Mesh, Scene
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    return float(np.linalg.norm(a - b) / np.linalg.norm(b))
+
+
+def renormalise(ef, a):
+    """The oracle's f coefficients are Gauss-renormalised: the gap between the
+    net charge and -sum(ef) is spread by area (one instance)."""
+    return ef - a["area"] / a["area"].sum() * (a["charges"][:, 3].sum() + ef.sum())
+
+
+def charges(n, seed, radius):
+    r = np.random.default_rng(seed)
+    d = r.normal(size=(n, 3))
+    d *= (0.6 * radius * r.uniform(size=n) ** (1 / 3) / np.linalg.norm(d, axis=1))[:, None]
+    return np.concatenate([d, r.normal(size=(n, 1))], axis=1)
+
+
+def arrays(quad, qual, kappa, nbsize=60, nc=37):
+    sc = Scene(80.0, kappa, quad, qual, nbsize)
+    m = Mesh.star(2, 8.0, 8, 0.08, 3)
+    sc.add_instance(m.set_charges(charges(nc, 4, 8.0)), 2.0)
+    sc.build()
+    return sc.arrays()
+
+
+def check(a, kappa):
+    n = a["area"].shape[0]
+    x = np.random.default_rng(n).normal(size=2 * n)
+    orc = oracle.Oracle(a, kappa, 80.0)
+    ref = orc.matvec(x)
+    # first-order rounding of the FP32 set: 16 roundings to form a coefficient,
+    # twice that with FP32 products and sums
+    u = 2.0 ** -24 * np.linalg.norm(np.abs(orc.assemble()) @ np.abs(x)) / np.linalg.norm(ref)
+    for near in ("precompute", "on_the_fly"):
+        d = Device(0)
+        d.set_far_field("direct", 5, 40)
+        d.set_geometry(a)
+        d.set_tree(a)
+        d.set_near_mode(near)
+        for p, tol in (("fp64", 1e-12), ("fp32", 32 * u)):
+            d.precompute(kappa, p)
+            err = rel(d.matvec(x, p), ref)
+            print(n, near, p, err, tol, flush=True)
+            assert err < tol
+        ef, eh = d.energy_coefficients(a["inst_patch_ptr"], a["inst_charge_ptr"], a["charges"])
+        ef = renormalise(ef, a)
+        rf, rh = orc.energy_coeffs()
+        assert rel(ef, rf) < 1e-12 and rel(eh, rh) < 1e-12
+        d.close()
+
+
+# runs of 2 (kept as points), 8, 12, 14 and 32; one and many row points
+@pytest.mark.parametrize("quad,qual", [(1, 0), (4, 0), (6, 0), (7, 1), (16, 0), (6, 4), (0, 0)])
+@pytest.mark.parametrize("kappa", [0.125, 0.0])
+def test_rules(quad, qual, kappa):
+    check(arrays(quad, qual, kappa), kappa)
+
+
+@pytest.mark.parametrize("case", ["bent", "shifted", "coplanar", "ragged"])
+def test_points_that_are_not_runs(case):
+    """One patch whose points have another normal, one whose points leave the
+    plane, a first patch with several triangles in one plane, and a last patch
+    one point short: all against the oracle on the same points."""
+    a = {k: (v.copy() if isinstance(v, np.ndarray) else v) for k, v in arrays(6, 0, 0.125).items()}
+    q = a["quad"]
+    k = a["quad_ptr"][70] + 5
+    if case == "bent":
+        q[k, 3:6] = q[k + 12, 3:6]
+    elif case == "shifted":
+        q[k, :3] += 1e-3 * q[k, 3:6]
+    elif case == "coplanar":
+        e = a["quad_ptr"][1]
+        q[:e, 2] = q[0, 2]
+        q[:e, 3:6] = (0.0, 0.0, 1.0)
+    else:
+        a["quad_ptr"][-1] -= 1
+        a["quad"] = q[:-1].copy()
+    check(a, 0.125)
+
+
+# no charge, one, odd numbers, and charges on and near the surface
+@pytest.mark.parametrize("nc", [1, 2, 129, 300])
+def test_energy_charges(nc):
+    a = arrays(4, 0, 0.1, nc=nc)
+    c = a["charges"]
+    g = a["gal"]
+    c[0, :3] = g[11, :3]          # on a point: contributes nothing there
+    if nc > 2:
+        c[2, :3] = g[40, :3] + 0.02 * g[40, 3:6]
+        c[nc - 1, :3] = a["centroid"][9]
+    d = Device(0)
+    d.set_far_field("direct", 5, 40)
+    d.set_geometry(a)
+    d.set_tree(a)
+    ef, eh = d.energy_coefficients(a["inst_patch_ptr"], a["inst_charge_ptr"], a["charges"])
+    ef = renormalise(ef, a)
+    rf, rh = oracle.Oracle(a, 0.1, 80.0).energy_coeffs()
+    print(nc, rel(ef, rf), rel(eh, rh), flush=True)
+    assert rel(ef, rf) < 1e-12 and rel(eh, rh) < 1e-12
+    d.close()
