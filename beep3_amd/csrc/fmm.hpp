@@ -119,6 +119,7 @@ struct PwDevTables {
     PwProb<T>* probs = nullptr;
     std::vector<int3> launch_m2m;  // one per level D-1 .. 2
     int3 launch_m2x{0, 0, 0}, launch_x2l{0, 0, 0};
+    int x2l_splits = 1;            // parts of X2L's K
     std::vector<int3> launch_l2l;  // one per level 3 .. D
     // X2X over every level >= 2 in one launch: per level the Laplace and
     // Yukawa wave counts and shift tables

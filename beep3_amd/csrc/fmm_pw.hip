@@ -11,7 +11,7 @@
 //   M2X   six-direction plane waves = M x m2x     MFMA   k_pw_gemm, every level at once
 //   X2X   diagonal translations, per target and   HBM    k_pw_x2x, every level at once
 //         direction in list order
-//   X2L   local = waves x x2l                     MFMA   k_pw_gemm, every level at once
+//   X2L   local = waves x x2l                     MFMA   k_pw_gemm + k_pw_x2l_sum, every level at once
 //   L2L   child local += parent local x A_o       MFMA   k_pw_gemm (grouped by octant), per level
 //   L2P   potential and gradient at the targets   VALU   k_pw_l2p
 // and the leaf pass (P2P) of fmm.hip / fmm_residual.hip.
@@ -465,10 +465,16 @@ __global__ __launch_bounds__(256) void k_pw_x2x(int base, int nwp, const int* __
     }
 }
 
+// X2L, second half: the locals of the boxes from base on are the sums of the
+// split products (split ps of n2 values, in order); the boxes above have none.
 template <typename T>
-__global__ void k_pw_zero(size_t n, T* __restrict__ p) {
-    for (size_t i = blockIdx.x * size_t(blockDim.x) + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x)
-        p[i] = T(0);
+__global__ void k_pw_x2l_sum(size_t n0, size_t n2, int splits, const T* __restrict__ ps, T* __restrict__ L) {
+    const size_t i = blockIdx.x * size_t(blockDim.x) + threadIdx.x;
+    if (i >= n0 + n2) return;
+    T v = T(0);
+    if (i >= n0)
+        for (int k = 0; k < splits; ++k) v += ps[k * n2 + (i - n0)];
+    L[i] = v;
 }
 
 // M2M, second half: the moments of every parent box at a level are the sum
@@ -613,16 +619,35 @@ void make_pw_launches(FmmPlan* pl, PwDevTables<T>& tb, T* M, T* L, T* W, T* Wacc
         tb.launch_m2x = launch(f);
     }
     {
-        // into zeroed locals: L = X2L, then L2L adds the parent's part
+        // K = 12 nw (about 900 to 2,200) against N = jp: the tiles of the output
+        // alone are a fraction of the chip at ordinary sizes, each a long
+        // serial product.  K is split so that there are about 1,024 blocks (four
+        // per CU, what their LDS lets in); the products of split q go to part q
+        // of W, whose waves X2X has consumed, and k_pw_x2l_sum adds the parts in
+        // order.  40,962 patches, order 12, FP64: 204 tiles; the product takes
+        // 0.27 ms with the sum in six parts and 0.64 ms in one (mat-vec 1.35 and
+        // 1.76 ms).
         const size_t f = probs.size();
+        const size_t n2 = size_t(pl->nbox - base) * 3 * jp;
+        int tiles = 0;
         for (int l = 2; l <= D; ++l)
             for (int k = 0; k < 2; ++k) {
-                PwProb<T> g = prob(0, k, 12 * tb.lev[l].nw[k], jp, nwp, jp, 1, Wacc, tb.lev[l].x2l[k], L, T(1),
-                                   base, 0);
-                g.first = pl->lvl_first[l];
-                g.nrows = pl->lvl_first[l + 1] - pl->lvl_first[l];
-                add(g);
+                const int rows = (pl->lvl_first[l + 1] - pl->lvl_first[l]) * (k == 0 ? 1 : 2);
+                tiles += ((rows + PW_BM - 1) / PW_BM) * ((jp + PW_BN - 1) / PW_BN);
             }
+        tb.x2l_splits = std::max(1, std::min({8, nwp / jp, (1024 + tiles - 1) / std::max(tiles, 1)}));
+        for (int q = 0; q < tb.x2l_splits; ++q)
+            for (int l = 2; l <= D; ++l)
+                for (int k = 0; k < 2; ++k) {
+                    const int K = 12 * tb.lev[l].nw[k];
+                    const int step = (K + PW_BK * tb.x2l_splits - 1) / (PW_BK * tb.x2l_splits) * PW_BK;
+                    const int k0 = std::min(K, q * step);  // a split may be empty: zeros
+                    PwProb<T> g = prob(0, k, std::min(step, K - k0), jp, nwp, jp, 0, Wacc + k0,
+                                       tb.lev[l].x2l[k] + size_t(k0) * jp, W + q * n2, T(1), base, base);
+                    g.first = pl->lvl_first[l];
+                    g.nrows = pl->lvl_first[l + 1] - pl->lvl_first[l];
+                    add(g);
+                }
         tb.launch_x2l = launch(f);
     }
     tb.launch_l2l.clear();
@@ -674,10 +699,6 @@ void pw_run(FmmPlan* pl, hipStream_t s, const Patch64* patches, double kappa, co
             T* M, T* L, T* W, T* Wacc, T* Tc, double* y, hipEvent_t* m2l_ev) {
     const FmmDev& d = pl->dv;
     const int D = pl->D, jp = pl->pw_jp, nwp = pl->pw_nwp;
-    {
-        const size_t n = size_t(pl->nbox) * 3 * jp;
-        hipLaunchKernelGGL(k_pw_zero<T>, dim3(unsigned(std::min<size_t>((n + 255) / 256, 65535))), dim3(256), 0, s, n, L);
-    }
     constexpr int ML = pw_mlanes<P>(), G = 256 / ML;
     hipLaunchKernelGGL((k_pw_p2m<T, P>), dim3(pl->nleaf), dim3(256), size_t(G) * 2 * jp * sizeof(T), s, d,
                        pl->src, kappa, jp, M);
@@ -701,6 +722,10 @@ void pw_run(FmmPlan* pl, hipStream_t s, const Patch64* patches, double kappa, co
                            pl->pw_xl_ptr, pl->pw_xl_src, pl->pw_xl_code, tb.x2x_nw, tb.x2x_sh, W, Wacc);
         hip_check(hipGetLastError(), "k_pw_x2x launch");
         gemm_launch(s, pl, tb, tb.launch_x2l);
+        const size_t n0 = size_t(base) * 3 * jp, n2 = size_t(nb) * 3 * jp;
+        hipLaunchKernelGGL(k_pw_x2l_sum<T>, dim3(unsigned((n0 + n2 + 255) / 256)), dim3(256), 0, s, n0, n2,
+                           tb.x2l_splits, W, L);
+        hip_check(hipGetLastError(), "k_pw_x2l_sum launch");
         // L2L from each level's parents, down the tree
         for (const int3& lc : tb.launch_l2l) gemm_launch(s, pl, tb, lc);
     }

@@ -7,7 +7,7 @@ import pytest
 import oracle
 from beep3_amd import configs
 from beep3_amd.device import Device
-from beep3_amd.scene import Scene
+from beep3_amd.scene import Mesh, Scene
 
 pytestmark = pytest.mark.gpu
 
@@ -136,3 +136,21 @@ def test_off_centre_solve_plane_wave_order12():
     for mode, (eE, ef, eh, its, conv) in out.items():
         assert conv == 1
         assert eE < 3e-7 and ef < 5e-6 and eh < 5e-6, mode
+
+
+# few and many boxes: the product of the waves with x2l in eight parts down to
+# one, some of them empty.  A lost part is an error of the order of the far
+# field (above 1e-2); the bounds are ten times those of the orders above.
+@pytest.mark.parametrize("level,leaf,order,bound", [(3, 10, 9, 3e-3), (4, 40, 9, 3e-3), (4, 10, 12, 1e-5),
+                                                    (4, 20, 18, 4e-6), (5, 40, 12, 1e-5), (5, 3, 12, 1e-5)])
+@pytest.mark.parametrize("kappa", [0.1, 0.0])
+def test_pw_small_scenes(level, leaf, order, bound, kappa):
+    sc = Scene(80.0, kappa, 4, 0, 60)
+    sc.add_instance(Mesh.star(level, 20.0, 8, 0.04, 7), 2.0)
+    a = sc.build().arrays()
+    x = np.random.default_rng(level).normal(size=2 * a["area"].shape[0])
+    ref = _device(a, kappa, "direct", 4).matvec(x, "fp64")
+    d = _device(a, kappa, "pw", order, leaf, ("fp64", "fp32"))
+    print(level, leaf, order, kappa, d.far_info(), rel(d.matvec(x, "fp64"), ref), flush=True)
+    assert rel(d.matvec(x, "fp64"), ref) < bound
+    assert rel(d.matvec(x, "fp32"), ref) < bound + 1e-6
