@@ -520,8 +520,9 @@ def main():
         "compulsory_GBs": cb64 / (near_alone * 1e-3) / 1e9}
     m2l = None
     if fi["mode"] == 1 and fi["m2l_pairs"] > 0:
-        # real GEMM flops of M2L: 3 products of the P^3 x P^3 table with a
-        # source expansion per box pair, over the k_m2l + k_m2l_sum time of a
+        # algorithmic GEMM flops of M2L: 3 products of the P^3 x P^3 table with
+        # a source expansion per box pair (the block-diagonal form executes a
+        # little over half of them), over the k_m2l + k_m2l_sum time of a
         # serialised mat-vec (and, beside it, of the overlapped one, where
         # the SpMV shares the chip)
         NP = fi["order"] ** 3
