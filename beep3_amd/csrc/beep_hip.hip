@@ -15,6 +15,7 @@
 #include "fmm.hpp"
 #include "pw.hpp"
 #include "host.hpp"
+#include "point_runs.hpp"
 #include "tree_key.hpp"
 
 using namespace beepdev;
@@ -911,17 +912,12 @@ int beep_hip_set_geometry(beep_hip_ctx* ctx, const beep_hip_geometry* g) {
         points(g->gal_ptr, ctx->gal_ptr.p, g->gal_pts, ctx->gal64, nullptr);
         // points of planar triangles: the shortest run of equal normals over the
         // first patches gives the length, the device checks every patch
-        auto shortest_run = [&](const int* ptr, const double* pts) {
-            int run = 0x7fffffff, k = 1;
-            for (int p = 0, a = ptr[0]; p < std::min(N, 64); ++p)
-                for (k = a; k < ptr[p + 1]; run = std::min(run, k - a), a = k)
-                    while (k < ptr[p + 1] && std::equal(pts + 7 * k + 3, pts + 7 * k + 6, pts + 7 * a + 3)) ++k;
-            return run;
-        };
-        point_planes(ctx, N, ctx->quad_ptr, ctx->quad64, g->quad_ptr[N], shortest_run(g->quad_ptr, g->quad_pts),
-                     ctx->quad_plane, ctx->quad_radius, &ctx->quad_xyzw, ctx->quad_planes);
-        point_planes(ctx, N, ctx->gal_ptr, ctx->gal64, g->gal_ptr[N], shortest_run(g->gal_ptr, g->gal_pts),
-                     ctx->gal_plane, ctx->gal_radius, nullptr, ctx->gal_planes);
+        point_planes(ctx, N, ctx->quad_ptr, ctx->quad64, g->quad_ptr[N],
+                     beep::shortest_normal_run(N, g->quad_ptr, g->quad_pts), ctx->quad_plane, ctx->quad_radius,
+                     &ctx->quad_xyzw, ctx->quad_planes);
+        point_planes(ctx, N, ctx->gal_ptr, ctx->gal64, g->gal_ptr[N],
+                     beep::shortest_normal_run(N, g->gal_ptr, g->gal_pts), ctx->gal_plane, ctx->gal_radius,
+                     nullptr, ctx->gal_planes);
         hip_check(hipStreamSynchronize(s), "sync geometry upload");
         geometry_done(ctx, N, g->centroid);
     });
