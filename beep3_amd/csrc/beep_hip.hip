@@ -1387,8 +1387,8 @@ void precompute_impl(beep_hip_ctx* ctx, double kappa, int precision) {
                                 ctx->quad64.p, ctx->quad_planes, kappa, sub_1pt, cellkey, guard, ctx->guard_max,
                                 ctx->coef64.p);
         launch_coef_repair(s, 0, guard, ctx->patches.p, ctx->qual_ptr.p, ctx->qual64.p,
-                           ctx->quad_ptr.p, ctx->quad64.p, ctx->quad_planes, kappa, ctx->guard_max, gcnt + 1,
-                           ctx->coef64.p);
+                           ctx->quad_ptr.p, ctx->quad64.p, ctx->quad_planes, kappa, sub_1pt, ctx->guard_max,
+                           gcnt + 1, ctx->coef64.p);
         ctx->have64 = true;
         ctx->uid64 = uid;
     } else {
@@ -1411,13 +1411,13 @@ void precompute_impl(beep_hip_ctx* ctx, double kappa, int precision) {
         launch_near_coeffs_fp32(s, ctx->n_coef_blocks, ctx->L, ctx->coef_blk.p, ctx->leaf_ptr.p,
                                 ctx->leaf_idx.p, ctx->nb_ptr.p, ctx->nb_idx.p, ctx->coef_off.p,
                                 ctx->patches.p, ctx->qual_ptr.p, ctx->qual32.p, ctx->quad_ptr.p,
-                                ctx->quad32.p, ctx->quad_planes, float(kappa), sub_1pt, cellkey, ns, guard,
+                                ctx->quad32.p, ctx->quad_planes, float(kappa), cellkey, ns, guard,
                                 ctx->guard_max, ctx->coef32.p);
         launch_near_fix64(s, ns, ctx->patches.p, ctx->qual_ptr.p, ctx->qual64.p, ctx->quad_ptr.p,
                           ctx->quad64.p, ctx->quad_planes, kappa, ctx->guard_max, gcnt + 2, ctx->coef32.p);
         launch_coef_repair(s, 1, guard, ctx->patches.p, ctx->qual_ptr.p, ctx->qual64.p,
-                           ctx->quad_ptr.p, ctx->quad64.p, ctx->quad_planes, kappa, ctx->guard_max, gcnt + 2,
-                           ctx->coef32.p);
+                           ctx->quad_ptr.p, ctx->quad64.p, ctx->quad_planes, kappa, 1, ctx->guard_max,
+                           gcnt + 2, ctx->coef32.p);
         ctx->ns_listed = ctx->ns_fp64;
         ctx->have32 = true;
         ctx->uid32 = uid;
@@ -1730,12 +1730,13 @@ int beep_hip_sanity_check(beep_hip_ctx* ctx, long long* repaired) {
                     "beep_hip_precompute again");
             const unsigned* cellkey = ctx->use_fmm ? ctx->fmm->cellkey : nullptr;
             void* coef = fp32 ? static_cast<void*>(ctx->coef32.p) : static_cast<void*>(ctx->coef64.p);
+            const int sub_1pt = folded(ctx, fp32 ? BEEP_FP32 : BEEP_FP64) ? 0 : 1;
             launch_coef_scan(s, fp32, ctx->n_coef_blocks, ctx->L, ctx->coef_blk.p, ctx->leaf_ptr.p,
                              ctx->leaf_idx.p, ctx->nb_ptr.p, ctx->nb_idx.p, ctx->coef_off.p, cellkey,
-                             folded(ctx, fp32 ? BEEP_FP32 : BEEP_FP64) ? 0 : 1, coef, ctx->guard_max, guard);
+                             sub_1pt, ctx->patches.p, ctx->kappa, coef, ctx->guard_max, guard);
             launch_coef_repair(s, fp32, guard, ctx->patches.p, ctx->qual_ptr.p, ctx->qual64.p,
-                               ctx->quad_ptr.p, ctx->quad64.p, ctx->quad_planes, ctx->kappa, ctx->guard_max, gcnt + 4,
-                               coef);
+                               ctx->quad_ptr.p, ctx->quad64.p, ctx->quad_planes, ctx->kappa, sub_1pt,
+                               ctx->guard_max, gcnt + 4, coef);
         }
         unsigned h = 0;
         hip_check(hipMemcpyAsync(&h, gcnt + 4, sizeof(h), hipMemcpyDeviceToHost, s), "D2H guard count");

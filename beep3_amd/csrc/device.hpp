@@ -175,8 +175,7 @@ void launch_near_coeffs_fp32(hipStream_t s, int n_blocks, int n_leaves, const in
                              const int* leaf_ptr, const int* leaf_idx, const int* nb_ptr,
                              const int* nb_idx, const int64_t* coef_off, const Patch64* patches,
                              const int* qual_ptr, const Pt32* qual, const int* quad_ptr,
-                             const Pt32* quad, const PointPlanes& planes, float kappa, int subtract_1pt,
-                             const unsigned* cellkey, const NsList& ns, const NsList& guard,
+                             const Pt32* quad, const PointPlanes& planes, float kappa, const unsigned* cellkey, const NsList& ns, const NsList& guard,
                              double maxv, float4* coef);
 // the FP64 pass over the near-singular entries the FP32 kernel listed (a bad
 // result is zeroed and counted in *repaired)
@@ -185,14 +184,17 @@ void launch_near_fix64(hipStream_t s, const NsList& ns, const Patch64* patches, 
                        double kappa, double maxv, unsigned* repaired, float4* coef);
 // coefficient guard: list the entries of a stored set with a value |v| >
 // maxv or not finite (the coefficient kernels list theirs as they go), then
-// recompute the listed ones in FP64 (zero if still bad, or a self pair)
+// recompute the listed ones in FP64 (zero if still bad, or a self pair).
+// subtract_1pt: as the set was computed; 0, a set of full rules with no far
+// field beside it, is judged by full - 1 point and falls back to the 1 point
 void launch_coef_scan(hipStream_t s, int fp32, int n_blocks, int n_leaves, const int* blk_ptr,
                       const int* leaf_ptr, const int* leaf_idx, const int* nb_ptr, const int* nb_idx,
                       const int64_t* coef_off, const unsigned* cellkey, int subtract_1pt,
-                      const void* coef, double maxv, const NsList& out);
+                      const Patch64* patches, double kappa, const void* coef, double maxv, const NsList& out);
 void launch_coef_repair(hipStream_t s, int fp32, const NsList& list, const Patch64* patches,
                         const int* qual_ptr, const Pt64* qual, const int* quad_ptr, const Pt64* quad,
-                        const PointPlanes& planes, double kappa, double maxv, unsigned* repaired, void* coef);
+                        const PointPlanes& planes, double kappa, int subtract_1pt, double maxv,
+                        unsigned* repaired, void* coef);
 void launch_near_coeffs_fp64(hipStream_t s, int n_blocks, int n_leaves, const int* blk_ptr,
                              const int* leaf_ptr, const int* leaf_idx, const int* nb_ptr,
                              const int* nb_idx, const int64_t* coef_off, const Patch64* patches,
@@ -235,7 +237,7 @@ void launch_near_spmv(hipStream_t s, int mode, int n, const SpmvPlan& p, const i
 // coefficients stored), over a plan of row groups of <= FLY_RB rows; part
 // holds 2 * FLY_RB values per work item.  subtract_1pt: pairs give full - 1
 // point, except those of adjacent FMM leaf cells (cellkey; null with the
-// direct far field); ns64: FP32 near-singular pairs in FP64.
+// direct far field); 0 (FP64 only): full rules, as a folded set's; ns64: FP32 near-singular pairs in FP64.
 void launch_near_fly(hipStream_t s, int mode, int n, const SpmvPlan& p, const int* leaf_ptr,
                      const int* leaf_idx, const int* nb_ptr, const int* nb_idx, const Patch64* patches,
                      const int* qual_ptr, const Pt32* qual32, const Pt64* qual64, const int* quad_ptr,

@@ -323,17 +323,41 @@ __device__ __forceinline__ void pair_coeffs(const Patch64& pi, const Patch64& pj
     out[3] = D * inv_eps * k4;
 }
 
+// The guard of a folded FP64 set (subtract_1pt = 0: every pair explicit, no far
+// field beside it).  Its entries hold the full rule, but they are judged by
+// full - 1 point, what the set stores beside a direct far field, and a bad one
+// becomes the 1-point interaction, which that far field would have added to
+// its zero: the same entries are bad, and the product is the same.
+template <bool KAPPA>
+__device__ __forceinline__ bool folded_bad(const Patch64* __restrict__ patches, int i, int j, double kappa,
+                                           double maxv, double out[4]) {
+    const Patch64 pi = patches[i], pj = patches[j];
+    double p[4] = {0, 0, 0, 0}, v[4];
+    integrand<double, KAPPA>(kappa, Math<double>::ek_of(kappa), pj.inv_eps, pj.cx - pi.cx, pj.cy - pi.cy,
+                             pj.cz - pi.cz, pi.nx, pi.ny, pi.nz, pj.nx, pj.ny, pj.nz, pj.area, p[0], p[1], p[2],
+                             p[3]);
+    p[3] *= pj.inv_eps;
+    for (int q = 0; q < 4; ++q) {
+        p[q] *= FOUR_PI_INV;
+        v[q] = out[q] - p[q];
+    }
+    if (!coef4_bad(v, maxv)) return false;
+    for (int q = 0; q < 4; ++q) out[q] = p[q];
+    return true;
+}
+
 // At most 128 VGPRs (FP64) or 102 (FP32): 4 or 5 waves per SIMD.  The FP64
 // kernel otherwise takes 136 and runs 3 waves per SIMD, 16 % slower.
-template <typename T, bool KAPPA>
+// FOLD: a folded set (folded_bad), FP64 only; a variant of its own, so that its
+// guard takes no registers from the other.
+template <typename T, bool KAPPA, bool FOLD = false>
 __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 5) void k_near_coeffs(
     int n_leaves, const int* __restrict__ blk_ptr, const int* __restrict__ leaf_ptr,
     const int* __restrict__ leaf_idx, const int* __restrict__ nb_ptr,
     const int* __restrict__ nb_idx, const int64_t* __restrict__ coef_off,
     const Patch64* __restrict__ patches, const int* __restrict__ qual_ptr,
     const Pt<T>* __restrict__ qual, const int* __restrict__ quad_ptr,
-    const Pt<T>* __restrict__ quad, PointPlanes planes, T kappa, int subtract_1pt,
-    const unsigned* __restrict__ cellkey, NsList ns, NsList guard, double maxv,
+    const Pt<T>* __restrict__ quad, PointPlanes planes, T kappa, const unsigned* __restrict__ cellkey, NsList ns, NsList guard, double maxv,
     void* __restrict__ coef) {
     const int b = xcd_remap(blockIdx.x, gridDim.x);
     const int L = find_leaf(blk_ptr, n_leaves, b);
@@ -353,7 +377,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 5) void k_near_coeffs(
         const int pb = quad_ptr[j], pn = quad_ptr[j + 1] - pb;
         // pairs the FMM leaf pass covers keep the full rule (that pass then
         // skips them)
-        const bool sub = subtract_1pt && !(cellkey && fmm_cells_adjacent(cellkey[i], cellkey[j]));
+        const bool sub = !FOLD && !(cellkey && fmm_cells_adjacent(cellkey[i], cellkey[j]));
         if (sizeof(T) == 4 && ns.rec && near_singular(pi, pj)) {
             // FP64 pass (k_near_fix64) for this entry; past the list's
             // capacity the entry stays in FP32
@@ -364,12 +388,18 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 5) void k_near_coeffs(
             }
         }
         pair_coeffs<T, KAPPA>(pi, pj, j, qb, qn, qual, pb, pn, quad, planes, kappa, sub, out);
-        const double v[4] = {double(out[0]), double(out[1]), double(out[2]), double(out[3])};
-        if (coef4_bad(v, maxv)) {
-            // stored as zero; k_coef_repair recomputes it in FP64
+        bool bad;
+        if constexpr (FOLD) {
+            bad = folded_bad<KAPPA>(patches, i, j, kappa, maxv, out);
+        } else {
+            const double v[4] = {double(out[0]), double(out[1]), double(out[2]), double(out[3])};
+            bad = coef4_bad(v, maxv);
+            if (bad) out[0] = out[1] = out[2] = out[3] = T(0);
+        }
+        if (bad) {
+            // stored as zero (1 point); k_coef_repair recomputes it in FP64
             const unsigned slot = atomicAdd(guard.count, 1u);
             if (slot < guard.cap) guard.rec[slot] = NsRec{coef_off[L] + e, i, 2 * j + (sub ? 1 : 0)};
-            out[0] = out[1] = out[2] = out[3] = T(0);
         }
     }
     const int64_t idx = coef_off[L] + e;
@@ -386,8 +416,7 @@ void launch_near_coeffs_fp32(hipStream_t s, int n_blocks, int n_leaves, const in
                              const int* leaf_ptr, const int* leaf_idx, const int* nb_ptr,
                              const int* nb_idx, const int64_t* coef_off, const Patch64* patches,
                              const int* qual_ptr, const Pt32* qual, const int* quad_ptr,
-                             const Pt32* quad, const PointPlanes& planes, float kappa, int subtract_1pt,
-                             const unsigned* cellkey, const NsList& ns, const NsList& guard,
+                             const Pt32* quad, const PointPlanes& planes, float kappa, const unsigned* cellkey, const NsList& ns, const NsList& guard,
                              double maxv, float4* coef) {
     if (n_blocks <= 0) return;
     if (ns.rec) launch_set_int(s, reinterpret_cast<int*>(ns.count), 0);
@@ -395,7 +424,7 @@ void launch_near_coeffs_fp32(hipStream_t s, int n_blocks, int n_leaves, const in
     auto k = kappa != 0.0f ? k_near_coeffs<float, true> : k_near_coeffs<float, false>;
     hipLaunchKernelGGL(k, dim3(n_blocks), dim3(256), 0, s, n_leaves, blk_ptr, leaf_ptr, leaf_idx,
                        nb_ptr, nb_idx, coef_off, patches, qual_ptr, qual, quad_ptr, quad, planes, kappa,
-                       subtract_1pt, cellkey, ns, guard, maxv, (void*)coef);
+                       cellkey, ns, guard, maxv, (void*)coef);
     hip_check(hipGetLastError(), "k_near_coeffs<float> launch");
 }
 
@@ -445,14 +474,15 @@ void launch_near_fix64(hipStream_t s, const NsList& ns, const Patch64* patches, 
 
 // Guard pass over a stored coefficient set (the sanity check on demand):
 // every entry is read once and the bad ones are listed for k_coef_repair.
-// Indexing as k_near_coeffs (one thread per entry).
+// Indexing as k_near_coeffs (one thread per entry).  A folded set's entries
+// are judged as k_near_coeffs does (kappa > 0 or 0: the same 1 point).
 template <typename TC>
 __global__ __launch_bounds__(256) void k_coef_scan(
     int n_leaves, const int* __restrict__ blk_ptr, const int* __restrict__ leaf_ptr,
     const int* __restrict__ leaf_idx, const int* __restrict__ nb_ptr,
     const int* __restrict__ nb_idx, const int64_t* __restrict__ coef_off,
-    const unsigned* __restrict__ cellkey, int subtract_1pt, const void* __restrict__ coef,
-    double maxv, NsList out) {
+    const unsigned* __restrict__ cellkey, int subtract_1pt, const Patch64* __restrict__ patches,
+    double kappa, const void* __restrict__ coef, double maxv, NsList out) {
     const int b = blockIdx.x;
     const int L = find_leaf(blk_ptr, n_leaves, b);
     const int lp = leaf_ptr[L], R = leaf_ptr[L + 1] - lp;
@@ -469,10 +499,12 @@ __global__ __launch_bounds__(256) void k_coef_scan(
         const double2 a = c2[coef64_at(idx)], c = c2[coef64_at(idx) + COEF64_CD];
         v[0] = a.x; v[1] = a.y; v[2] = c.x; v[3] = c.y;
     }
-    if (!coef4_bad(v, maxv)) return;
+    const bool fold = sizeof(TC) == 8 && !subtract_1pt;
+    if (!fold && !coef4_bad(v, maxv)) return;
     const int c = int(e / R);
     const int r = int(e - int64_t(c) * R);
     const int i = leaf_idx[lp + r], j = nb_idx[np + c];
+    if (fold && !(i == j ? coef4_bad(v, maxv) : folded_bad<true>(patches, i, j, kappa, maxv, v))) return;
     const bool sub = subtract_1pt && !(cellkey && fmm_cells_adjacent(cellkey[i], cellkey[j]));
     const unsigned slot = atomicAdd(out.count, 1u);
     if (slot < out.cap) out.rec[slot] = NsRec{idx, i, 2 * j + (sub ? 1 : 0)};
@@ -480,14 +512,14 @@ __global__ __launch_bounds__(256) void k_coef_scan(
 
 // Recompute the listed entries in FP64 (a self pair, i == j, is zeroed, as
 // the reference does for an ill-conditioned patch); an entry still bad is
-// zeroed.  Each counts one in *repaired.
+// zeroed (folded set: as folded_bad).  Each counts one in *repaired.
 template <typename TC, bool KAPPA>
 __global__ __launch_bounds__(256) void k_coef_repair(NsList list, const Patch64* __restrict__ patches,
                                                      const int* __restrict__ qual_ptr,
                                                      const Pt64* __restrict__ qual,
                                                      const int* __restrict__ quad_ptr,
                                                      const Pt64* __restrict__ quad, PointPlanes planes,
-                                                     double kappa, double maxv,
+                                                     double kappa, int subtract_1pt, double maxv,
                                                      unsigned* __restrict__ repaired,
                                                      void* __restrict__ coef) {
     const unsigned n = min(*list.count, list.cap);
@@ -503,7 +535,8 @@ __global__ __launch_bounds__(256) void k_coef_repair(NsList list, const Patch64*
             double v[4] = {out[0], out[1], out[2], out[3]};
             if constexpr (sizeof(TC) == 4)
                 for (int q = 0; q < 4; ++q) v[q] = double(float(v[q]));
-            if (coef4_bad(v, maxv)) out[0] = out[1] = out[2] = out[3] = 0.0;
+            if (sizeof(TC) == 8 && !subtract_1pt) folded_bad<KAPPA>(patches, i, j, kappa, maxv, out);
+            else if (coef4_bad(v, maxv)) out[0] = out[1] = out[2] = out[3] = 0.0;
         }
         if constexpr (sizeof(TC) == 4) {
             reinterpret_cast<float4*>(coef)[r.idx] =
@@ -520,27 +553,28 @@ __global__ __launch_bounds__(256) void k_coef_repair(NsList list, const Patch64*
 void launch_coef_scan(hipStream_t s, int fp32, int n_blocks, int n_leaves, const int* blk_ptr,
                       const int* leaf_ptr, const int* leaf_idx, const int* nb_ptr, const int* nb_idx,
                       const int64_t* coef_off, const unsigned* cellkey, int subtract_1pt,
-                      const void* coef, double maxv, const NsList& out) {
+                      const Patch64* patches, double kappa, const void* coef, double maxv, const NsList& out) {
     launch_set_int(s, reinterpret_cast<int*>(out.count), 0);
     if (n_blocks <= 0) return;
     auto k = fp32 ? k_coef_scan<float> : k_coef_scan<double>;
     hipLaunchKernelGGL(k, dim3(n_blocks), dim3(256), 0, s, n_leaves, blk_ptr, leaf_ptr, leaf_idx,
-                       nb_ptr, nb_idx, coef_off, cellkey, subtract_1pt, coef, maxv, out);
+                       nb_ptr, nb_idx, coef_off, cellkey, subtract_1pt, patches, kappa, coef, maxv, out);
     hip_check(hipGetLastError(), "k_coef_scan launch");
 }
 
 void launch_coef_repair(hipStream_t s, int fp32, const NsList& list, const Patch64* patches,
                         const int* qual_ptr, const Pt64* qual, const int* quad_ptr, const Pt64* quad,
-                        const PointPlanes& planes, double kappa, double maxv, unsigned* repaired, void* coef) {
+                        const PointPlanes& planes, double kappa, int subtract_1pt, double maxv,
+                        unsigned* repaired, void* coef) {
     const unsigned blocks = std::max(1u, std::min(256u, (list.cap + 255) / 256));
     if (fp32) {
         auto k = kappa != 0.0 ? k_coef_repair<float, true> : k_coef_repair<float, false>;
         hipLaunchKernelGGL(k, dim3(blocks), dim3(256), 0, s, list, patches, qual_ptr, qual, quad_ptr,
-                           quad, planes, kappa, maxv, repaired, coef);
+                           quad, planes, kappa, subtract_1pt, maxv, repaired, coef);
     } else {
         auto k = kappa != 0.0 ? k_coef_repair<double, true> : k_coef_repair<double, false>;
         hipLaunchKernelGGL(k, dim3(blocks), dim3(256), 0, s, list, patches, qual_ptr, qual, quad_ptr,
-                           quad, planes, kappa, maxv, repaired, coef);
+                           quad, planes, kappa, subtract_1pt, maxv, repaired, coef);
     }
     hip_check(hipGetLastError(), "k_coef_repair launch");
 }
@@ -555,9 +589,10 @@ void launch_near_coeffs_fp64(hipStream_t s, int n_blocks, int n_leaves, const in
     if (n_blocks <= 0) return;
     launch_set_int(s, reinterpret_cast<int*>(guard.count), 0);
     auto k = kappa != 0.0 ? k_near_coeffs<double, true> : k_near_coeffs<double, false>;
+    if (!subtract_1pt) k = kappa != 0.0 ? k_near_coeffs<double, true, true> : k_near_coeffs<double, false, true>;
     hipLaunchKernelGGL(k, dim3(n_blocks), dim3(256), 0, s, n_leaves, blk_ptr, leaf_ptr, leaf_idx,
                        nb_ptr, nb_idx, coef_off, patches, qual_ptr, qual, quad_ptr, quad, planes, kappa,
-                       subtract_1pt, cellkey, NsList{}, guard, maxv, (void*)coef);
+                       cellkey, NsList{}, guard, maxv, (void*)coef);
     hip_check(hipGetLastError(), "k_near_coeffs<double> launch");
 }
 
@@ -962,14 +997,14 @@ __device__ __attribute__((noinline)) float4 fly_redo64(int i, int j, int sub, co
     return coef4_bad(d, maxv) ? make_float4(0.f, 0.f, 0.f, 0.f) : v;
 }
 
-template <typename T, typename TA, bool KAPPA>
+template <typename T, typename TA, bool KAPPA, bool FOLD = false>
 __global__ __launch_bounds__(256, 4) void k_near_fly_part(
     const int4* __restrict__ work, int n_work, const int* __restrict__ leaf_ptr,
     const int* __restrict__ leaf_idx, const int* __restrict__ nb_ptr, const int* __restrict__ nb_idx,
     const Patch64* __restrict__ patches, const int* __restrict__ qual_ptr,
     const Pt<T>* __restrict__ qual, const int* __restrict__ quad_ptr, const Pt<T>* __restrict__ quad,
     const Pt64* __restrict__ qual64, const Pt64* __restrict__ quad64, PointPlanes planes, double kappa,
-    int subtract_1pt, const unsigned* __restrict__ cellkey, int ns64, double maxv, const double* __restrict__ x, int n,
+    const unsigned* __restrict__ cellkey, int ns64, double maxv, const double* __restrict__ x, int n,
     TA* __restrict__ part) {
     // FP32 pass: the near-singular pairs and bad entries of a thread are set
     // aside (column and leaf-pass bit) and integrated in FP64 by the whole
@@ -1020,16 +1055,19 @@ __global__ __launch_bounds__(256, 4) void k_near_fly_part(
                 if (j == i) continue;  // the self pair is the diagonal's (stored as zero)
                 const Patch64 pj = patches[j];
                 const int pb = quad_ptr[j], pn = quad_ptr[j + 1] - pb;
-                const int sub = subtract_1pt && !(cellkey && fmm_cells_adjacent(ki, cellkey[j]));
+                const int sub = !FOLD && !(cellkey && fmm_cells_adjacent(ki, cellkey[j]));
                 T v[4];
                 bool redo = sizeof(T) == 4 && ns64 && near_singular(pi, pj);
                 if (!redo) {
                     pair_coeffs<T, KAPPA>(pi, pj, j, qb, qn, qual, pb, pn, quad, planes, T(kappa), sub, v);
                     const double d[4] = {double(v[0]), double(v[1]), double(v[2]), double(v[3])};
-                    if (coef4_bad(d, maxv)) {
+                    if constexpr (FOLD) {
+                        folded_bad<KAPPA>(patches, i, j, kappa, maxv, v);
+                    } else if constexpr (sizeof(T) == 8) {
                         // FP64 recomputes what FP64 already gave: zero at once
-                        if constexpr (sizeof(T) == 8) v[0] = v[1] = v[2] = v[3] = T(0);
-                        else redo = true;
+                        if (coef4_bad(d, maxv)) v[0] = v[1] = v[2] = v[3] = T(0);
+                    } else {
+                        redo = coef4_bad(d, maxv);
                     }
                 }
                 if constexpr (sizeof(T) == 4) {
@@ -1095,9 +1133,11 @@ static void fly_launch(hipStream_t s, const SpmvPlan& p, const int* leaf_ptr, co
                        const Pt64* quad64, const PointPlanes& planes, double kappa, int subtract_1pt,
                        const unsigned* cellkey, int ns64, double maxv, const double* diag4, const double* x, int n, TA* part, double* y) {
     auto k = kappa != 0.0 ? k_near_fly_part<T, TA, true> : k_near_fly_part<T, TA, false>;
+    if constexpr (sizeof(T) == 8)
+        if (!subtract_1pt) k = kappa != 0.0 ? k_near_fly_part<T, TA, true, true> : k_near_fly_part<T, TA, false, true>;
     hipLaunchKernelGGL(k, dim3(unsigned(p.n_work)), dim3(256), 0, s, p.work, p.n_work, leaf_ptr, leaf_idx,
                        nb_ptr, nb_idx, patches, qual_ptr, qual, quad_ptr, quad, qual64, quad64, planes, kappa,
-                       subtract_1pt, cellkey, ns64, maxv, x, n, part);
+                       cellkey, ns64, maxv, x, n, part);
     hip_check(hipGetLastError(), "k_near_fly_part launch");
     const CopyOffsets co{{0, 0}};
     hipLaunchKernelGGL((k_near_spmv_sum<TA>), dim3(unsigned(p.n_groups), 1u), dim3(256), 0, s, p.groups,

@@ -114,3 +114,54 @@ def test_shared_near_field_of_a_one_leaf_mesh():
     assert rel(src.matvec(x1, "fp64"), y1) < 1e-12
     pose.close()
     src.close()
+
+
+@pytest.mark.parametrize("near", ["precompute", "on_the_fly"])
+@pytest.mark.parametrize("kappa", [0.125, 0.0])
+def test_bad_entries_keep_the_one_point_interaction(near, kappa):
+    """A pair whose integral is not a number counts as one entry repaired and
+    contributes its 1-point interaction, also in the FP64 set that has no far
+    field: quadrature points with NaN normals against the oracle with one
+    point at the centroid in their place."""
+    a = scene((3,), 1500, kappa)
+    n = a["area"].shape[0]
+    p = 3
+    k0, k1 = a["quad_ptr"][p], a["quad_ptr"][p + 1]
+    one = np.concatenate([a["centroid"][p], a["normal"][p], a["area"][p:p + 1]])
+    b = dict(a)
+    b["quad"] = np.concatenate([a["quad"][:k0], one[None], a["quad"][k1:]])
+    b["quad_ptr"] = a["quad_ptr"].copy()
+    b["quad_ptr"][p + 1:] -= k1 - k0 - 1
+    orc = oracle.Oracle(b, kappa, 80.0)
+    x = np.random.default_rng(n).normal(size=2 * n)
+    ref = orc.matvec(x)
+    a["quad"] = a["quad"].copy()
+    a["quad"][k0:k1, 3:6] = np.nan
+    for far in ("auto", "direct"):
+        d = device(a, far=far, kappa=kappa, near=near)
+        for prec, tol in bounds(orc, x, ref).items():
+            assert rel(d.matvec(x, prec), ref) < tol, (far, prec)
+        if near == "precompute":
+            assert d.guard_stats()["fp64"] == n - 1
+            assert d.sanity_check() == 0
+        d.close()
+
+
+def test_guard_bound_without_far_field():
+    """The entries over a low guard bound are the same with the direct far
+    field chosen by size (no far field in FP64) and asked for."""
+    a = scene((3,), 1500)
+    n = a["area"].shape[0]
+    x = np.random.default_rng(n).normal(size=2 * n)
+    out = []
+    for far in ("auto", "direct"):
+        d = device(a, far=far, precs=("fp64",))
+        d.set_guard(1e-3)
+        d.precompute(0.125, "fp64")
+        y = d.matvec(x, "fp64")
+        out.append((d.guard_stats(), d.sanity_check(), y, d.matvec(x, "fp64")))
+        d.close()
+    (sa, ca, ya, za), (sd, cd, yd, zd) = out
+    print(sa, sd, ca, cd, rel(ya, yd), flush=True)
+    assert 0 < sd["fp64"] < n * (n - 1) and sa == sd and ca == cd
+    assert rel(ya, yd) < 1e-12 and rel(za, zd) < 1e-12
