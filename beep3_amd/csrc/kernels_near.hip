@@ -270,7 +270,11 @@ __device__ __forceinline__ void pair_planes(double ox64, double oy64, double oz6
     C += fma(ie1, C0, fma(ie1lo, C0, ie * C1));
 }
 
-template <typename T, bool KAPPA>
+// PLANAR: the point set is in planar runs (planes.gs > 0).  A kernel holds one
+// form or the other, the form not run takes registers from the one that does:
+// FP32 precompute of 10,242 patches, curved triangles 1.45 ms with both and
+// 1.34 apart, planar ones 1.06 and 1.04.
+template <typename T, bool KAPPA, bool PLANAR>
 __device__ __forceinline__ void pair_coeffs(const Patch64& pi, const Patch64& pj, int j, int qb, int qn,
                                             const Pt<T>* __restrict__ qual, int pb, int pn,
                                             const Pt<T>* __restrict__ quad, const PointPlanes& planes, T kappa,
@@ -289,7 +293,7 @@ __device__ __forceinline__ void pair_coeffs(const Patch64& pi, const Patch64& pj
     for (int a = 0; a < qn; ++a) {
         const Pt<T> q = qual[qb + a];
         T a_ = 0, b_ = 0, c_ = 0, d_ = 0;
-        if (planes.gs) {
+        if constexpr (PLANAR) {
             const double ox = dx64 - double(q.x), oy = dy64 - double(q.y), oz = dz64 - double(q.z);
             const double reach = double(planes.radius[j]) + 1e-4;  // |d| > 1e-4 beyond it
             const int runs = pn / planes.gs;
@@ -350,7 +354,7 @@ __device__ __forceinline__ bool folded_bad(const Patch64* __restrict__ patches, 
 // kernel otherwise takes 136 and runs 3 waves per SIMD, 16 % slower.
 // FOLD: a folded set (folded_bad), FP64 only; a variant of its own, so that its
 // guard takes no registers from the other.
-template <typename T, bool KAPPA, bool FOLD = false>
+template <typename T, bool KAPPA, bool PLANAR, bool FOLD>
 __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 5) void k_near_coeffs(
     int n_leaves, const int* __restrict__ blk_ptr, const int* __restrict__ leaf_ptr,
     const int* __restrict__ leaf_idx, const int* __restrict__ nb_ptr,
@@ -387,7 +391,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 5) void k_near_coeffs(
                 return;
             }
         }
-        pair_coeffs<T, KAPPA>(pi, pj, j, qb, qn, qual, pb, pn, quad, planes, kappa, sub, out);
+        pair_coeffs<T, KAPPA, PLANAR>(pi, pj, j, qb, qn, qual, pb, pn, quad, planes, kappa, sub, out);
         bool bad;
         if constexpr (FOLD) {
             bad = folded_bad<KAPPA>(patches, i, j, kappa, maxv, out);
@@ -412,6 +416,15 @@ __global__ __launch_bounds__(256, sizeof(T) == 8 ? 4 : 5) void k_near_coeffs(
     }
 }
 
+// the variant of a kernel for kappa != 0 and planar runs (f returns the kernel)
+template <typename F>
+static auto choose(bool kappa, bool planar, F f) {
+    using std::false_type;
+    using std::true_type;
+    if (planar) return kappa ? f(true_type{}, true_type{}) : f(false_type{}, true_type{});
+    return kappa ? f(true_type{}, false_type{}) : f(false_type{}, false_type{});
+}
+
 void launch_near_coeffs_fp32(hipStream_t s, int n_blocks, int n_leaves, const int* blk_ptr,
                              const int* leaf_ptr, const int* leaf_idx, const int* nb_ptr,
                              const int* nb_idx, const int64_t* coef_off, const Patch64* patches,
@@ -421,7 +434,7 @@ void launch_near_coeffs_fp32(hipStream_t s, int n_blocks, int n_leaves, const in
     if (n_blocks <= 0) return;
     if (ns.rec) launch_set_int(s, reinterpret_cast<int*>(ns.count), 0);
     launch_set_int(s, reinterpret_cast<int*>(guard.count), 0);
-    auto k = kappa != 0.0f ? k_near_coeffs<float, true> : k_near_coeffs<float, false>;
+    auto k = choose(kappa != 0.0f, planes.gs != 0, [](auto K, auto P) { return k_near_coeffs<float, K(), P(), false>; });
     hipLaunchKernelGGL(k, dim3(n_blocks), dim3(256), 0, s, n_leaves, blk_ptr, leaf_ptr, leaf_idx,
                        nb_ptr, nb_idx, coef_off, patches, qual_ptr, qual, quad_ptr, quad, planes, kappa,
                        cellkey, ns, guard, maxv, (void*)coef);
@@ -431,7 +444,7 @@ void launch_near_coeffs_fp32(hipStream_t s, int n_blocks, int n_leaves, const in
 // The near-singular entries of an FP32 coefficient set, in FP64 on the FP64
 // point sets, rounded to FP32.  The record count is read on the device, so
 // the grid is fixed and walks the list with a stride.
-template <bool KAPPA>
+template <bool KAPPA, bool PLANAR>
 __global__ __launch_bounds__(256) void k_near_fix64(NsList ns, const Patch64* __restrict__ patches,
                                                    const int* __restrict__ qual_ptr,
                                                    const Pt64* __restrict__ qual,
@@ -448,7 +461,7 @@ __global__ __launch_bounds__(256) void k_near_fix64(NsList ns, const Patch64* __
         const int qb = qual_ptr[i], qn = qual_ptr[i + 1] - qb;
         const int pb = quad_ptr[j], pn = quad_ptr[j + 1] - pb;
         double out[4];
-        pair_coeffs<double, KAPPA>(pi, pj, j, qb, qn, qual, pb, pn, quad, planes, kappa, r.j2 & 1, out);
+        pair_coeffs<double, KAPPA, PLANAR>(pi, pj, j, qb, qn, qual, pb, pn, quad, planes, kappa, r.j2 & 1, out);
         const float4 o = make_float4(float(out[0]), float(out[1]), float(out[2]), float(out[3]));
         const double v[4] = {o.x, o.y, o.z, o.w};
         if (coef4_bad(v, maxv)) {
@@ -466,7 +479,7 @@ void launch_near_fix64(hipStream_t s, const NsList& ns, const Patch64* patches, 
     if (!ns.rec) return;
     // enough blocks for every CU several times over; each walks the list
     const unsigned blocks = std::max(1u, std::min(2048u, (ns.cap + 255) / 256));
-    auto k = kappa != 0.0 ? k_near_fix64<true> : k_near_fix64<false>;
+    auto k = choose(kappa != 0.0, planes.gs != 0, [](auto K, auto P) { return k_near_fix64<K(), P()>; });
     hipLaunchKernelGGL(k, dim3(blocks), dim3(256), 0, s, ns, patches, qual_ptr, qual, quad_ptr, quad,
                        planes, kappa, maxv, repaired, coef);
     hip_check(hipGetLastError(), "k_near_fix64 launch");
@@ -513,7 +526,7 @@ __global__ __launch_bounds__(256) void k_coef_scan(
 // Recompute the listed entries in FP64 (a self pair, i == j, is zeroed, as
 // the reference does for an ill-conditioned patch); an entry still bad is
 // zeroed (folded set: as folded_bad).  Each counts one in *repaired.
-template <typename TC, bool KAPPA>
+template <typename TC, bool KAPPA, bool PLANAR>
 __global__ __launch_bounds__(256) void k_coef_repair(NsList list, const Patch64* __restrict__ patches,
                                                      const int* __restrict__ qual_ptr,
                                                      const Pt64* __restrict__ qual,
@@ -531,7 +544,7 @@ __global__ __launch_bounds__(256) void k_coef_repair(NsList list, const Patch64*
             const Patch64 pi = patches[i], pj = patches[j];
             const int qb = qual_ptr[i], qn = qual_ptr[i + 1] - qb;
             const int pb = quad_ptr[j], pn = quad_ptr[j + 1] - pb;
-            pair_coeffs<double, KAPPA>(pi, pj, j, qb, qn, qual, pb, pn, quad, planes, kappa, r.j2 & 1, out);
+            pair_coeffs<double, KAPPA, PLANAR>(pi, pj, j, qb, qn, qual, pb, pn, quad, planes, kappa, r.j2 & 1, out);
             double v[4] = {out[0], out[1], out[2], out[3]};
             if constexpr (sizeof(TC) == 4)
                 for (int q = 0; q < 4; ++q) v[q] = double(float(v[q]));
@@ -568,11 +581,11 @@ void launch_coef_repair(hipStream_t s, int fp32, const NsList& list, const Patch
                         unsigned* repaired, void* coef) {
     const unsigned blocks = std::max(1u, std::min(256u, (list.cap + 255) / 256));
     if (fp32) {
-        auto k = kappa != 0.0 ? k_coef_repair<float, true> : k_coef_repair<float, false>;
+        auto k = choose(kappa != 0.0, planes.gs != 0, [](auto K, auto P) { return k_coef_repair<float, K(), P()>; });
         hipLaunchKernelGGL(k, dim3(blocks), dim3(256), 0, s, list, patches, qual_ptr, qual, quad_ptr,
                            quad, planes, kappa, subtract_1pt, maxv, repaired, coef);
     } else {
-        auto k = kappa != 0.0 ? k_coef_repair<double, true> : k_coef_repair<double, false>;
+        auto k = choose(kappa != 0.0, planes.gs != 0, [](auto K, auto P) { return k_coef_repair<double, K(), P()>; });
         hipLaunchKernelGGL(k, dim3(blocks), dim3(256), 0, s, list, patches, qual_ptr, qual, quad_ptr,
                            quad, planes, kappa, subtract_1pt, maxv, repaired, coef);
     }
@@ -588,8 +601,9 @@ void launch_near_coeffs_fp64(hipStream_t s, int n_blocks, int n_leaves, const in
                              double2* coef) {
     if (n_blocks <= 0) return;
     launch_set_int(s, reinterpret_cast<int*>(guard.count), 0);
-    auto k = kappa != 0.0 ? k_near_coeffs<double, true> : k_near_coeffs<double, false>;
-    if (!subtract_1pt) k = kappa != 0.0 ? k_near_coeffs<double, true, true> : k_near_coeffs<double, false, true>;
+    auto k = choose(kappa != 0.0, planes.gs != 0, [&](auto K, auto P) {
+        return subtract_1pt ? k_near_coeffs<double, K(), P(), false> : k_near_coeffs<double, K(), P(), true>;
+    });
     hipLaunchKernelGGL(k, dim3(n_blocks), dim3(256), 0, s, n_leaves, blk_ptr, leaf_ptr, leaf_idx,
                        nb_ptr, nb_idx, coef_off, patches, qual_ptr, qual, quad_ptr, quad, planes, kappa,
                        cellkey, NsList{}, guard, maxv, (void*)coef);
@@ -980,7 +994,7 @@ void launch_direct_matvec(hipStream_t s, int mode, int n, const SpmvPlan& p, con
 // registers from the FP32 loop.  It takes indices, not patch records, and the
 // planes by value, so the caller keeps nothing on the stack for the call (a
 // reference turns the caller's own loads through them into flat loads).
-template <bool KAPPA>
+template <bool KAPPA, bool PLANAR>
 __device__ __attribute__((noinline)) float4 fly_redo64(int i, int j, int sub, const Patch64* __restrict__ patches,
                                                        const int* __restrict__ qual_ptr,
                                                        const Pt64* __restrict__ qual64,
@@ -991,13 +1005,13 @@ __device__ __attribute__((noinline)) float4 fly_redo64(int i, int j, int sub, co
     const int qb = qual_ptr[i], qn = qual_ptr[i + 1] - qb;
     const int pb = quad_ptr[j], pn = quad_ptr[j + 1] - pb;
     double o[4];
-    pair_coeffs<double, KAPPA>(pi, pj, j, qb, qn, qual64, pb, pn, quad64, planes, kappa, sub, o);
+    pair_coeffs<double, KAPPA, PLANAR>(pi, pj, j, qb, qn, qual64, pb, pn, quad64, planes, kappa, sub, o);
     const float4 v = make_float4(float(o[0]), float(o[1]), float(o[2]), float(o[3]));
     const double d[4] = {v.x, v.y, v.z, v.w};
     return coef4_bad(d, maxv) ? make_float4(0.f, 0.f, 0.f, 0.f) : v;
 }
 
-template <typename T, typename TA, bool KAPPA, bool FOLD = false>
+template <typename T, typename TA, bool KAPPA, bool PLANAR, bool FOLD>
 __global__ __launch_bounds__(256, 4) void k_near_fly_part(
     const int4* __restrict__ work, int n_work, const int* __restrict__ leaf_ptr,
     const int* __restrict__ leaf_idx, const int* __restrict__ nb_ptr, const int* __restrict__ nb_idx,
@@ -1059,7 +1073,7 @@ __global__ __launch_bounds__(256, 4) void k_near_fly_part(
                 T v[4];
                 bool redo = sizeof(T) == 4 && ns64 && near_singular(pi, pj);
                 if (!redo) {
-                    pair_coeffs<T, KAPPA>(pi, pj, j, qb, qn, qual, pb, pn, quad, planes, T(kappa), sub, v);
+                    pair_coeffs<T, KAPPA, PLANAR>(pi, pj, j, qb, qn, qual, pb, pn, quad, planes, T(kappa), sub, v);
                     const double d[4] = {double(v[0]), double(v[1]), double(v[2]), double(v[3])};
                     if constexpr (FOLD) {
                         folded_bad<KAPPA>(patches, i, j, kappa, maxv, v);
@@ -1099,8 +1113,8 @@ __global__ __launch_bounds__(256, 4) void k_near_fly_part(
             const int cc = code >> 1;
             const int i = leaf_idx[lp + row0 + owner % Rb];
             const int j = nb_idx[np + col0 + cc];
-            const float4 o = fly_redo64<KAPPA>(i, j, code & 1, patches, qual_ptr, qual64, quad_ptr, quad64, planes,
-                                               kappa, maxv);
+            const float4 o = fly_redo64<KAPPA, PLANAR>(i, j, code & 1, patches, qual_ptr, qual64, quad_ptr,
+                                                       quad64, planes, kappa, maxv);
             const TA xf = xs[0][cc], xh = xs[1][cc];
             dprod[0][e] = TA(o.y) * xf - TA(o.x) * xh;
             dprod[1][e] = TA(o.w) * xf - TA(o.z) * xh;
@@ -1132,9 +1146,10 @@ static void fly_launch(hipStream_t s, const SpmvPlan& p, const int* leaf_ptr, co
                        const Pt<T>* qual, const int* quad_ptr, const Pt<T>* quad, const Pt64* qual64,
                        const Pt64* quad64, const PointPlanes& planes, double kappa, int subtract_1pt,
                        const unsigned* cellkey, int ns64, double maxv, const double* diag4, const double* x, int n, TA* part, double* y) {
-    auto k = kappa != 0.0 ? k_near_fly_part<T, TA, true> : k_near_fly_part<T, TA, false>;
-    if constexpr (sizeof(T) == 8)
-        if (!subtract_1pt) k = kappa != 0.0 ? k_near_fly_part<T, TA, true, true> : k_near_fly_part<T, TA, false, true>;
+    auto k = choose(kappa != 0.0, planes.gs != 0, [&](auto K, auto P) {
+        constexpr bool fold = sizeof(T) == 8;  // an FP64 set only
+        return subtract_1pt ? k_near_fly_part<T, TA, K(), P(), false> : k_near_fly_part<T, TA, K(), P(), fold>;
+    });
     hipLaunchKernelGGL(k, dim3(unsigned(p.n_work)), dim3(256), 0, s, p.work, p.n_work, leaf_ptr, leaf_idx,
                        nb_ptr, nb_idx, patches, qual_ptr, qual, quad_ptr, quad, qual64, quad64, planes, kappa,
                        cellkey, ns64, maxv, x, n, part);
@@ -1173,7 +1188,7 @@ void launch_near_fly(hipStream_t s, int mode, int n, const SpmvPlan& p, const in
 // coefficients computed in FP64 (full rule less the 1-point interaction, as
 // every explicit pair with the direct far field), stored in FP64 and
 // rounded to FP32; bad values zeroed and counted, as the guard does.
-template <bool KAPPA>
+template <bool KAPPA, bool PLANAR>
 __global__ __launch_bounds__(256) void k_pair_coeffs(long long n_pairs, const int* __restrict__ pi_,
                                                     const int* __restrict__ pj_,
                                                     const Patch64* __restrict__ patches,
@@ -1192,7 +1207,7 @@ __global__ __launch_bounds__(256) void k_pair_coeffs(long long n_pairs, const in
         const Patch64 a = patches[i], b = patches[j];
         const int qb = qual_ptr[i], qn = qual_ptr[i + 1] - qb;
         const int pb = quad_ptr[j], pn = quad_ptr[j + 1] - pb;
-        pair_coeffs<double, KAPPA>(a, b, j, qb, qn, qual, pb, pn, quad, planes, kappa, 1, out);
+        pair_coeffs<double, KAPPA, PLANAR>(a, b, j, qb, qn, qual, pb, pn, quad, planes, kappa, 1, out);
         if (coef4_bad(out, maxv)) {
             out[0] = out[1] = out[2] = out[3] = 0.0;
             atomicAdd(repaired, 1u);
@@ -1208,7 +1223,7 @@ void launch_pair_coeffs(hipStream_t s, long long n_pairs, const int* pi, const i
                         const Pt64* quad, const PointPlanes& planes, double kappa, double maxv,
                         unsigned* repaired, float4* c32, double2* c64) {
     if (n_pairs <= 0) return;
-    auto k = kappa != 0.0 ? k_pair_coeffs<true> : k_pair_coeffs<false>;
+    auto k = choose(kappa != 0.0, planes.gs != 0, [](auto K, auto P) { return k_pair_coeffs<K(), P()>; });
     hipLaunchKernelGGL(k, dim3(unsigned((n_pairs + 255) / 256)), dim3(256), 0, s, n_pairs, pi, pj, patches,
                        qual_ptr, qual, quad_ptr, quad, planes, kappa, maxv, repaired, c32, c64);
     hip_check(hipGetLastError(), "k_pair_coeffs launch");

@@ -111,3 +111,39 @@ def test_energy_charges(nc):
     print(nc, rel(ef, rf), rel(eh, rh), flush=True)
     assert rel(ef, rf) < 1e-12 and rel(eh, rh) < 1e-12
     d.close()
+
+
+def test_planar_beside_curved_and_far_from_the_origin():
+    """Scenes that keep a normal per point: a planar mesh beside a curved one,
+    and a mesh so far from the origin that the rounding of its coordinates
+    takes its points off their planes; against the oracle."""
+    mixed = Scene(80.0, 0.125, 6, 0, 60)
+    mixed.add_instance(Mesh.star(2, 8.0, 8, 0.08, 3).set_charges(charges(5, 4, 8.0)), 2.0)
+    bent = Mesh.star(2, 8.0, 8, 0.08, 7).set_charges(charges(5, 6, 8.0))
+    bent.set_curved(True)
+    mixed.add_instance(bent, 3.0, offset=[20.0, 0.0, 0.0])
+    away = Scene(80.0, 0.125, 6, 0, 60)
+    away.add_instance(Mesh.star(2, 8.0, 8, 0.08, 3).set_charges(charges(5, 4, 8.0)), 2.0,
+                      offset=[30000.0, -20000.0, 10000.0])
+    for sc in (mixed, away):
+        a = sc.build().arrays()
+        n = a["area"].shape[0]
+        x = np.random.default_rng(n).normal(size=2 * n)
+        orc = oracle.Oracle(a, 0.125, 80.0)
+        ref = orc.matvec(x)
+        u = 2.0 ** -24 * np.linalg.norm(np.abs(orc.assemble()) @ np.abs(x)) / np.linalg.norm(ref)
+        # differences of coordinates c carry their rounding, 2^-53 c over a
+        # distance of at least a third of a patch (0.5 A), cubed in the kernels
+        far = 2.0 ** -53 * np.abs(a["centroid"]).max() / 0.5 * 3 * 8
+        for near in ("precompute", "on_the_fly"):
+            d = Device(0)
+            d.set_far_field("direct", 5, 40)
+            d.set_geometry(a)
+            d.set_tree(a)
+            d.set_near_mode(near)
+            for p, tol in (("fp64", 1e-12 + far), ("fp32", 32 * u + far)):
+                d.precompute(0.125, p)
+                err = rel(d.matvec(x, p), ref)
+                print(n, near, p, err, tol, flush=True)
+                assert err < tol
+            d.close()
