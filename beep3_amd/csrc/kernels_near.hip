@@ -1024,11 +1024,14 @@ __global__ __launch_bounds__(256, 4) void k_near_fly_part(
     // aside (column and leaf-pass bit) and integrated in FP64 by the whole
     // block after the loop, so a wave does not run the FP64 path for a few of
     // its lanes; each thread then adds its own in the order found.  A thread
-    // that has DEF of them stops there, and the block comes back to its
-    // columns afterwards (more than DEF of one thread's columns are rare).  At
-    // most 128 VGPRs in FP32 too: at 96 the point loop itself reloads spilled
-    // values.  Mat-vec of 40,962 patches: 11.6 ms at 96, 9.0 at 128 (9.6 before
-    // the planar runs).
+    // that has DEF of them passes over further near-singular pairs, and the
+    // block comes back to those afterwards, looking for them alone.  (Stopping
+    // there instead left the thread's other columns to a round with most of
+    // the block idle: mat-vec of 40,962 patches 9.7 ms instead of 7.5, of
+    // 10,242 curved ones 4.4 instead of 2.9.)  A bad entry a full thread finds
+    // (rare) does stop it until the next round.  At most 128 VGPRs in FP32 too:
+    // at 96 the point loop itself reloads spilled values (9.9 ms and 7.7 in
+    // one comparison).
     constexpr int DEF = sizeof(T) == 4 ? 4 : 1;
     __shared__ TA xs[2][SPMV_CW];
     __shared__ TA red[2][256];
@@ -1050,20 +1053,29 @@ __global__ __launch_bounds__(256, 4) void k_near_fly_part(
         xs[0][k] = TA(x[j]);
         xs[1][k] = TA(x[n + j]);
     }
-    // a thread has columns left (this round, the next): red is free until the end
+    // a thread has pairs left (this round, the next): red is free until the end
     int* again = reinterpret_cast<int*>(&red[0][0]);
     int round = 0;
     if (t == 0) again[0] = 0;
     __syncthreads();
     TA af = 0, ah = 0;
     int c = active ? s : nc;  // next column of this thread
+    int cs = c;               // next column it may have passed over, <= c
     for (;;) {
         int nd = 0;  // pairs this thread set aside
-        if (c < nc) {
+        if (cs < nc) {
             const int i = leaf_idx[lp + row0 + r];
             const Patch64 pi = patches[i];
             const int qb = qual_ptr[i], qn = qual_ptr[i + 1] - qb;
             const unsigned ki = cellkey ? cellkey[i] : 0u;
+            if constexpr (sizeof(T) == 4)
+                for (; cs < c && nd < DEF; cs += S) {
+                    const int j = nb_idx[np + col0 + cs];
+                    if (j == i || !near_singular(pi, patches[j])) continue;
+                    dcode[t * DEF + nd] = 2 * cs + !(cellkey && fmm_cells_adjacent(ki, cellkey[j]));
+                    ++nd;
+                }
+            bool room = cs == c;  // none passed over
             for (; c < nc; c += S) {
                 const int j = nb_idx[np + col0 + c];
                 if (j == i) continue;  // the self pair is the diagonal's (stored as zero)
@@ -1072,6 +1084,11 @@ __global__ __launch_bounds__(256, 4) void k_near_fly_part(
                 const int sub = !FOLD && !(cellkey && fmm_cells_adjacent(ki, cellkey[j]));
                 T v[4];
                 bool redo = sizeof(T) == 4 && ns64 && near_singular(pi, pj);
+                if (redo && nd == DEF) {
+                    if (room) cs = c;
+                    room = false;
+                    continue;
+                }
                 if (!redo) {
                     pair_coeffs<T, KAPPA, PLANAR>(pi, pj, j, qb, qn, qual, pb, pn, quad, planes, T(kappa), sub, v);
                     const double d[4] = {double(v[0]), double(v[1]), double(v[2]), double(v[3])};
@@ -1086,7 +1103,7 @@ __global__ __launch_bounds__(256, 4) void k_near_fly_part(
                 }
                 if constexpr (sizeof(T) == 4) {
                     if (redo) {
-                        if (nd == DEF) break;  // goes on here after the set-aside pairs
+                        if (nd == DEF) break;  // a bad entry (rare): goes on here next round
                         dcode[t * DEF + nd] = 2 * c + sub;
                         ++nd;
                         continue;
@@ -1096,12 +1113,13 @@ __global__ __launch_bounds__(256, 4) void k_near_fly_part(
                 af += TA(v[1]) * xf - TA(v[0]) * xh;
                 ah += TA(v[3]) * xf - TA(v[2]) * xh;
             }
+            if (room) cs = c;
         }
         if constexpr (sizeof(T) == 8) break;
         // the set-aside pairs, spread over the block: entry e belongs to
         // thread e / DEF
         for (int k = nd; k < DEF; ++k) dcode[t * DEF + k] = -1;
-        if (c < nc) again[round] = 1;
+        if (cs < nc) again[round] = 1;
         __syncthreads();
         const bool more = again[round];
         round ^= 1;

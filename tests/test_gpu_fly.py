@@ -119,3 +119,57 @@ def test_on_the_fly_with_fmm_full_size(off_centre):
     assert e_orc < 1e-4
     dp.close()
     df.close()
+
+
+def _most_near_singular(a):
+    """The most near-singular pairs of one thread of the on-the-fly kernel:
+    a leaf's rows in groups of 64, its columns in slabs of 512, the 256
+    threads of a block interleaved over a slab's columns."""
+    c, ar = a["centroid"], a["area"]
+    most = 0
+    for l in range(len(a["leaf_ptr"]) - 1):
+        rows = a["leaf_idx"][a["leaf_ptr"][l]:a["leaf_ptr"][l + 1]]
+        cols = a["nb_idx"][a["nb_ptr"][l]:a["nb_ptr"][l + 1]]
+        for r0 in range(0, len(rows), 64):
+            g = rows[r0:r0 + 64]
+            lanes = 256 // len(g)
+            for c0 in range(0, len(cols), 512):
+                k = cols[c0:c0 + 512]
+                ns = np.sum((c[g][:, None] - c[k][None]) ** 2, axis=2) < 2.0 * (ar[g][:, None] + ar[k][None])
+                ns &= g[:, None] != k[None]
+                most = max(most, max(int(ns[:, s::lanes].sum(axis=1).max()) for s in range(lanes)))
+    return most
+
+
+@pytest.mark.parametrize("curved", [False, True])
+@pytest.mark.parametrize("guard", [1e6, 1e-3])
+def test_more_pairs_set_aside_than_a_thread_keeps(curved, guard):
+    """FP32 pairs integrated in FP64 after the loop, more than the four a
+    thread keeps at once (with a low guard bound, bad entries too): on the fly
+    against stored coefficients, whose rounding bounds the difference (32
+    roundings of every product)."""
+    from beep3_amd.scene import Mesh, Scene
+
+    m = Mesh.star(3, 25.0, 8, 0.04, 5)
+    if curved:
+        m.set_curved(True)
+    a = Scene(80.0, 0.125, 6, 0, 1500).add_instance(m, 2.0).build().arrays()
+    n = a["area"].shape[0]
+    assert _most_near_singular(a) > 4
+    x = np.random.default_rng(35).normal(size=2 * n)
+    y = {}
+    for mode in ("precompute", "on_the_fly"):
+        d = Device(0)
+        d.set_far_field("direct", 5, 40)
+        d.set_near_mode(mode)
+        d.set_geometry(a)
+        d.set_tree(a)
+        d.set_guard(guard)
+        d.precompute(0.125, "fp32")
+        y[mode] = [d.matvec(x, p) for p in ("fp32", "fp32_resid")]
+        d.close()
+    orc = oracle.Oracle(a, 0.125, 80.0)
+    for fly, stored in zip(y["on_the_fly"], y["precompute"]):
+        tol = 32 * 2.0 ** -24 * np.linalg.norm(np.abs(orc.assemble()) @ np.abs(x)) / np.linalg.norm(stored)
+        print(curved, guard, rel(fly, stored), tol, flush=True)
+        assert rel(fly, stored) < tol
