@@ -104,7 +104,7 @@ struct beep_hip_ctx {
     // near-SpMV settings per coefficient mode (0: FP64, 1: FP32, 2: FP32
     // coefficients with FP64 sums): residency cap in blocks per CU (0: one
     // block per work item) and loads in flight per thread (x 4 FP64, x 8 FP32)
-    // (SPMV_CAP_AUTO: 1 beside an FMM far field, else uncapped)
+    // (SPMV_CAP_AUTO: see spmv_blocks)
     int spmv_cap[3] = {SPMV_CAP_AUTO, SPMV_CAP_AUTO, SPMV_CAP_AUTO};
     int spmv_depth[3] = {1, 1, 1};
     std::string err;
@@ -425,14 +425,18 @@ bool coef_plan_ok(const beep_hip_ctx* c, int precision) {
     return built == 0 || built == beep_hip_ctx::UID_FOLDED;
 }
 
-// blocks of the near SpMV (0: one per work item)
-int spmv_blocks(const beep_hip_ctx* c, int mode) {
-    const int cap = c->spmv_cap[mode];
-    return (cap == beep_hip_ctx::SPMV_CAP_AUTO ? (c->use_fmm ? 1 : 0) : cap) * c->n_cu;
-}
-
 // the direct far field as symmetric tile pairs (far_sym.hpp)
 bool far_is_sym(const beep_hip_ctx* c) { return !c->use_fmm && c->N <= FAR_SYM_MAX; }
+
+// Blocks of the near SpMV (0: one per work item).  By default one block per
+// CU beside the FMM and beside the direct sum in one direction (23,046 / 40,962
+// patches, FP32: 790 / 2,267 us, uncapped 843 / 2,387), uncapped beside
+// symmetric tile pairs, where the SpMV is too short for it to matter (two
+// copies of 162 to 2,562 patches: within noise).
+int spmv_blocks(const beep_hip_ctx* c, int mode) {
+    const int cap = c->spmv_cap[mode];
+    return (cap == beep_hip_ctx::SPMV_CAP_AUTO ? (far_is_sym(c) ? 0 : 1) : cap) * c->n_cu;
+}
 
 // buffers of a mat-vec's far field
 void far_buffers(beep_hip_ctx* c) {
@@ -521,7 +525,18 @@ void matvec_dev(beep_hip_ctx* c, const double* dx, double* dy, int precision) {
         hip_check(hipEventRecord(c->ev_fork, s), "hipEventRecord");
         hip_check(hipStreamWaitEvent(sf, c->ev_fork, 0), "hipStreamWaitEvent");
     }
-    // near field (explicit pairs) + diagonal into y, launched first: the
+    // The direct sum in one direction takes about ten times its SpMV: launched
+    // first, and the SpMV fills in as its blocks end.  FP64, 40,962 patches:
+    // 5,363 us, after the SpMV 5,490; two copies of 10,242: 1,365 and 1,492.
+    auto far_direct = [&] {
+        launch_fill(sf, n2, 0.0, c->yfar.p);
+        launch_far_pack(sf, c->N, c->patches.p, c->leaf_idx.p, dx, c->src.p);
+        launch_far_direct(sf, far32, c->N, far_direct_splits(c->N, c->n_cu), c->leaf_idx.p, c->patches.p, c->src.p,
+                          c->kappa, c->yfar.p, c->far_part.p);
+    };
+    const bool far_first = !c->use_fmm && !sym && c->overlap && !fold;
+    if (far_first) far_direct();
+    // near field (explicit pairs) + diagonal into y, else launched first: the
     // SpMV is the longer of the two, and the far field's dozen short kernels
     // take the host a while to launch
     if (c->share) {
@@ -562,11 +577,8 @@ void matvec_dev(beep_hip_ctx* c, const double* dx, double* dy, int precision) {
             fmm_evaluate(c->fmm, sf, far32, c->patches.p, dx, c->kappa, c->yfar.p, timed ? &ev[4] : nullptr,
                          c->ev_pack);
             if (p2p_far) fmm_p2p(c->fmm, sf, far32, c->patches.p, c->kappa, c->yfar.p);
-        } else {
-            launch_fill(sf, n2, 0.0, c->yfar.p);
-            launch_far_pack(sf, c->N, c->patches.p, c->leaf_idx.p, dx, c->src.p);
-            launch_far_direct(sf, far32, c->N, far_direct_splits(c->N, c->n_cu), c->leaf_idx.p, c->patches.p,
-                              c->src.p, c->kappa, c->yfar.p, c->far_part.p);
+        } else if (!far_first) {
+            far_direct();
         }
     }
     if (timed) hip_check(hipEventRecord(ev[3], sf), "hipEventRecord");

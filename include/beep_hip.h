@@ -246,10 +246,11 @@ int beep_hip_autotune_leaf(beep_hip_ctx* ctx, int precision, const int* leaf_tar
 
 /* Residency cap of the near-field SpMV: at most blocks_per_cu blocks per
  * compute unit walk the work items (0: one block per work item; default: 1
- * beside an FMM far field, else 0).  A cap leaves room on every CU for the
- * far-field kernels that run on the other stream at the same time; up to
- * 20,480 patches with the direct far field both run in one launch, which no
- * cap applies to.  Sets the cap of every precision. */
+ * beside the FMM and beside the direct far field above 20,480 patches, else
+ * 0).  A cap leaves room on every CU for the far-field kernels that run on
+ * the other stream at the same time; up to 20,480 patches with the direct
+ * far field both run in one launch, which no cap applies to.  Sets the cap
+ * of every precision. */
 int beep_hip_set_spmv_residency(beep_hip_ctx* ctx, int blocks_per_cu);
 /* Autotuner for that cap: times `reps` whole mat-vecs of the given precision
  * (far field overlapped) for each candidate, writes the mean times to ms_out
