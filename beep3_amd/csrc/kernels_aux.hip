@@ -162,23 +162,27 @@ __global__ __launch_bounds__(64) void k_energy_coeffs(int n, const int* __restri
     }
 }
 
-// The same for points in planar runs (PointPlanes).  n.r is one number per run
-// and charge, so a point adds only w/r and w/r^3: 16 FP64 operations, the
-// reciprocal root's among them, against 28 with a normal per point.  The points are read
-// through scalar loads (every lane the same one), with no LDS and no barrier;
-// the coincidence test is run only where a charge is within the patch's reach
-// (rare, so per wave).  Charges two per lane, as above.
+// The same for points in planar runs (PointPlanes) of up to EC_PTS points.  n.r
+// is one number per run and charge, so a point adds only w/r and w/r^3: 16 FP64
+// operations, the reciprocal root's among them, against 28 with a normal per
+// point.  Points through LDS as above, whole runs at a time; the coincidence
+// test is run only where a charge is within the patch's reach (rare, so per
+// wave).  Charges two per lane, as above.  163,842 patches, 1 / 200 / 300
+// charges, whole call: 839 / 1,418 / 1,970 us; 1,020 / 1,800 / 2,546 with a
+// normal per point (and 1,200 / 1,850 / 2,480 by runs with every point read
+// through scalar loads).
 template <bool GUARD>
-__device__ __forceinline__ void energy_run(const Pt64* __restrict__ pts, int gs, double x, double y, double z,
-                                           double& sh, double& sf) {
+__device__ __forceinline__ void energy_run(const double4* pts, int gs, double x, double y, double z, double& sh,
+                                           double& sf) {
     sh = sf = 0.0;
 #pragma unroll 4
     for (int k = 0; k < gs; ++k) {
-        const double rx = x + pts[k].x, ry = y + pts[k].y, rz = z + pts[k].z;
+        const double4 p = pts[k];
+        const double rx = x + p.x, ry = y + p.y, rz = z + p.z;
         const double d2 = rx * rx + ry * ry + rz * rz;
         double id = rsqrt_nr(d2);
         if constexpr (GUARD) id = d2 <= 2.220446049250313e-16 ? 0.0 : id;
-        const double wid = pts[k].w * id;
+        const double wid = p.w * id;
         sh += wid;
         sf = fma(wid, id * id, sf);
     }
@@ -192,40 +196,50 @@ __global__ __launch_bounds__(64) void k_energy_planes(int n, const int* __restri
                                                       const double* __restrict__ xyzq,
                                                       double* __restrict__ ec_f,
                                                       double* __restrict__ ec_h) {
+    __shared__ double4 pxw[EC_PTS];  // point position, w
     const int i = blockIdx.x;
     if (i >= n) return;
-    const int t = threadIdx.x;
-    const int g0 = gal_ptr[i], runs = (gal_ptr[i + 1] - g0) / planes.gs;
+    const int t = threadIdx.x, gs = planes.gs;
+    const int g0 = gal_ptr[i], ng = gal_ptr[i + 1] - g0;
     const int inst = patch_inst[i];
     const int c0 = inst_charge_ptr[inst], c1 = inst_charge_ptr[inst + 1];
     const Patch64 p = patches[i];
-    const double4* plane = planes.plane + g0 / planes.gs;
     const double reach = double(planes.radius[i]) + 1e-7;  // > 1e-7 from every point beyond it
+    const int step = EC_PTS / gs * gs;
     double ef = 0, eh = 0;
-    for (int c = c0 + 2 * t; c < c1; c += 128) {
-        // two charges (the second may be past the end: zero charge); positions
-        // of the centroid as seen from them
-        const bool two = c + 1 < c1;
-        const double ax = p.cx - xyzq[4 * c], ay = p.cy - xyzq[4 * c + 1], az = p.cz - xyzq[4 * c + 2];
-        const double aq = xyzq[4 * c + 3];
-        const double bx = two ? p.cx - xyzq[4 * c + 4] : ax, by = two ? p.cy - xyzq[4 * c + 5] : ay;
-        const double bz = two ? p.cz - xyzq[4 * c + 6] : az, bq = two ? xyzq[4 * c + 7] : 0.0;
-        const double nearest = fmin(ax * ax + ay * ay + az * az, bx * bx + by * by + bz * bz);
-        const bool guard = __any(nearest <= reach * reach);
-        for (int g = 0; g < runs; ++g) {
-            const double4 pl = plane[g];
-            const Pt64* pts = gal + g0 + g * planes.gs;
-            double ha, fa, hb, fb;
-            if (guard) {
-                energy_run<true>(pts, planes.gs, ax, ay, az, ha, fa);
-                energy_run<true>(pts, planes.gs, bx, by, bz, hb, fb);
-            } else {
-                energy_run<false>(pts, planes.gs, ax, ay, az, ha, fa);
-                energy_run<false>(pts, planes.gs, bx, by, bz, hb, fb);
+    for (int a0 = 0; a0 < ng; a0 += step) {
+        const int na = min(step, ng - a0);
+        __syncthreads();  // previous points consumed
+        if (t < na) {
+            const Pt64 q = gal[g0 + a0 + t];
+            pxw[t] = make_double4(q.x, q.y, q.z, q.w);
+        }
+        __syncthreads();
+        const double4* plane = planes.plane + (g0 + a0) / gs;
+        for (int c = c0 + 2 * t; c < c1; c += 128) {
+            // two charges (the second may be past the end: zero charge);
+            // positions of the centroid as seen from them
+            const bool two = c + 1 < c1;
+            const double ax = p.cx - xyzq[4 * c], ay = p.cy - xyzq[4 * c + 1], az = p.cz - xyzq[4 * c + 2];
+            const double aq = xyzq[4 * c + 3];
+            const double bx = two ? p.cx - xyzq[4 * c + 4] : ax, by = two ? p.cy - xyzq[4 * c + 5] : ay;
+            const double bz = two ? p.cz - xyzq[4 * c + 6] : az, bq = two ? xyzq[4 * c + 7] : 0.0;
+            const double nearest = fmin(ax * ax + ay * ay + az * az, bx * bx + by * by + bz * bz);
+            const bool guard = __any(nearest <= reach * reach);
+            for (int k = 0; k < na; k += gs) {
+                const double4 pl = plane[k / gs];
+                double ha, fa, hb, fb;
+                if (guard) {
+                    energy_run<true>(pxw + k, gs, ax, ay, az, ha, fa);
+                    energy_run<true>(pxw + k, gs, bx, by, bz, hb, fb);
+                } else {
+                    energy_run<false>(pxw + k, gs, ax, ay, az, ha, fa);
+                    energy_run<false>(pxw + k, gs, bx, by, bz, hb, fb);
+                }
+                eh = fma(aq, ha, fma(bq, hb, eh));
+                ef = fma(-aq * fa, pl.x * ax + pl.y * ay + pl.z * az + pl.w, ef);
+                ef = fma(-bq * fb, pl.x * bx + pl.y * by + pl.z * bz + pl.w, ef);
             }
-            eh = fma(aq, ha, fma(bq, hb, eh));
-            ef = fma(-aq * fa, pl.x * ax + pl.y * ay + pl.z * az + pl.w, ef);
-            ef = fma(-bq * fb, pl.x * bx + pl.y * by + pl.z * bz + pl.w, ef);
         }
     }
     for (int off = 32; off > 0; off >>= 1) {
@@ -243,7 +257,7 @@ void launch_energy_coeffs(hipStream_t s, int n, const int* gal_ptr, const Pt64* 
                           const int* inst_charge_ptr, const double* xyzq, double* ec_f,
                           double* ec_h) {
     if (n <= 0) return;
-    if (planes.gs)
+    if (planes.gs > 0 && planes.gs <= EC_PTS)
         hipLaunchKernelGGL(k_energy_planes, dim3(n), dim3(64), 0, s, n, gal_ptr, gal, patches, planes,
                            patch_inst, inst_charge_ptr, xyzq, ec_f, ec_h);
     else

@@ -91,7 +91,7 @@ def test_points_that_are_not_runs(case):
     check(a, 0.125)
 
 
-# no charge, one, odd numbers, and charges on and near the surface
+# one charge, odd numbers, and charges on and near the surface
 @pytest.mark.parametrize("nc", [1, 2, 129, 300])
 def test_energy_charges(nc):
     a = arrays(4, 0, 0.1, nc=nc)
@@ -147,3 +147,37 @@ def test_planar_beside_curved_and_far_from_the_origin():
                 print(n, near, p, err, tol, flush=True)
                 assert err < tol
             d.close()
+
+
+def test_energy_without_charges():
+    a = arrays(4, 0, 0.1, nc=3)
+    d = Device(0)
+    d.set_geometry(a)
+    ef, eh = d.energy_coefficients(a["inst_patch_ptr"], np.zeros(2, np.int32), np.zeros((0, 4)))
+    assert np.all(ef == 0) and np.all(eh == 0)
+    d.close()
+
+
+# two runs a patch, shorter and longer than the 64 points staged at a time
+@pytest.mark.parametrize("gs", [3, 4, 20, 64, 65, 100])
+def test_energy_run_lengths(gs):
+    a = dict(arrays(4, 0, 0.1, nc=150))
+    n = a["area"].shape[0]
+    r = np.random.default_rng(gs)
+    nrm = a["normal"][:, None] + 0.1 * r.normal(size=(n, 2, 3))
+    nrm /= np.linalg.norm(nrm, axis=2)[..., None]
+    t = r.normal(size=(n, 2, gs, 3)) * 0.3
+    t -= np.sum(t * nrm[:, :, None], axis=3)[..., None] * nrm[:, :, None]
+    g = np.empty((n, 2, gs, 7))
+    g[..., :3] = a["centroid"][:, None, None] + t
+    g[..., 3:6] = nrm[:, :, None]
+    g[..., 6] = a["area"][:, None, None] / (2 * gs) * r.uniform(0.5, 1.5, size=(n, 2, gs))
+    a["gal"] = np.ascontiguousarray(g.reshape(-1, 7))
+    a["gal_ptr"] = np.arange(n + 1, dtype=np.int32) * (2 * gs)
+    d = Device(0)
+    d.set_geometry(a)
+    ef, eh = d.energy_coefficients(a["inst_patch_ptr"], a["inst_charge_ptr"], a["charges"])
+    rf, rh = oracle.Oracle(a, 0.1, 80.0).energy_coeffs()
+    print(gs, rel(renormalise(ef, a), rf), rel(eh, rh), flush=True)
+    assert rel(renormalise(ef, a), rf) < 1e-12 and rel(eh, rh) < 1e-12
+    d.close()
