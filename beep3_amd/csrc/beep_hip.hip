@@ -120,7 +120,8 @@ struct beep_hip_ctx {
     DevBuf<double4> quad_plane, gal_plane;
     DevBuf<float> quad_radius, gal_radius;
     DevBuf<float4> quad_xyzw;
-    DevBuf<int> plane_bad;
+    DevBuf<int> plane_bad;          // a flag per set
+    bool plane_bad_zero = false;    // both known to be zero
     PointPlanes quad_planes, gal_planes;
     DevBuf<double> stage;  // raw point upload staging (7 doubles per point)
     DevBuf<double> sverts; // surface for point generation
@@ -855,24 +856,43 @@ int beep_hip_destroy(beep_hip_ctx* ctx) {
     return 0;
 }
 
-// The planar runs of gs points of a point set (gs 0: none), or none where any
-// patch's points are not such runs.
-static void point_planes(beep_hip_ctx* ctx, int N, const DevBuf<int>& ptr, const DevBuf<Pt64>& pts, int total, int gs,
-                         DevBuf<double4>& plane, DevBuf<float>& radius, DevBuf<float4>* xyzw, PointPlanes& out) {
-    out = PointPlanes{};
-    if (gs < MIN_RUN || total % gs != 0) return;
-    hipStream_t s = ctx->stream;
-    plane.alloc(size_t(total) / gs);
-    radius.alloc(size_t(N));
-    if (xyzw) xyzw->alloc(size_t(total) + 1);
-    ctx->plane_bad.alloc(1);
-    launch_set_int(s, ctx->plane_bad.p, 0);
-    launch_point_planes(s, N, ptr.p, pts.p, gs, plane.p, radius.p, xyzw ? xyzw->p : nullptr, ctx->plane_bad.p);
-    int bad = 0;
-    hip_check(hipMemcpyAsync(&bad, ctx->plane_bad.p, sizeof(int), hipMemcpyDeviceToHost, s), "D2H point planes");
-    hip_check(hipStreamSynchronize(s), "sync point planes");
-    if (bad == 0) out = PointPlanes{plane.p, radius.p, xyzw ? xyzw->p : nullptr, gs};
-}
+// The planar runs of a geometry's two point sets: launch() starts the check of
+// one set for runs of gs points (gs 0: none), read() waits for both and keeps
+// those all of whose patches are such runs.  One wait for both: at 642 patches
+// it is a good part of set_surface.
+struct PlaneCheck {
+    beep_hip_ctx* ctx;
+    PointPlanes found[2];
+
+    explicit PlaneCheck(beep_hip_ctx* c) : ctx(c) {
+        ctx->quad_planes = ctx->gal_planes = PointPlanes{};
+        ctx->plane_bad.alloc(2);
+        if (!ctx->plane_bad_zero)
+            for (int k = 0; k < 2; ++k) launch_set_int(ctx->stream, ctx->plane_bad.p + k, 0);
+        ctx->plane_bad_zero = false;
+    }
+    void launch(int set, int N, const DevBuf<int>& ptr, const DevBuf<Pt64>& pts, int total, int gs,
+                DevBuf<double4>& plane, DevBuf<float>& radius, DevBuf<float4>* xyzw) {
+        if (gs < MIN_RUN || total % gs != 0) return;
+        hipStream_t s = ctx->stream;
+        plane.alloc(size_t(total) / gs);
+        radius.alloc(size_t(N));
+        if (xyzw) xyzw->alloc(size_t(total) + 1);
+        launch_point_planes(s, N, ptr.p, pts.p, gs, plane.p, radius.p, xyzw ? xyzw->p : nullptr,
+                            ctx->plane_bad.p + set);
+        found[set] = PointPlanes{plane.p, radius.p, xyzw ? xyzw->p : nullptr, gs};
+    }
+    void read() {
+        int bad[2] = {0, 0};
+        hipStream_t s = ctx->stream;
+        if (found[0].gs || found[1].gs)
+            hip_check(hipMemcpyAsync(bad, ctx->plane_bad.p, sizeof(bad), hipMemcpyDeviceToHost, s), "D2H point planes");
+        hip_check(hipStreamSynchronize(s), "sync geometry upload");
+        ctx->plane_bad_zero = bad[0] == 0 && bad[1] == 0;
+        if (bad[0] == 0) ctx->quad_planes = found[0];
+        if (bad[1] == 0) ctx->gal_planes = found[1];
+    }
+};
 
 int beep_hip_set_geometry(beep_hip_ctx* ctx, const beep_hip_geometry* g) {
     return guarded(ctx, [&] {
@@ -924,13 +944,13 @@ int beep_hip_set_geometry(beep_hip_ctx* ctx, const beep_hip_geometry* g) {
         points(g->gal_ptr, ctx->gal_ptr.p, g->gal_pts, ctx->gal64, nullptr);
         // points of planar triangles: the shortest run of equal normals over the
         // first patches gives the length, the device checks every patch
-        point_planes(ctx, N, ctx->quad_ptr, ctx->quad64, g->quad_ptr[N],
-                     beep::shortest_normal_run(N, g->quad_ptr, g->quad_pts), ctx->quad_plane, ctx->quad_radius,
-                     &ctx->quad_xyzw, ctx->quad_planes);
-        point_planes(ctx, N, ctx->gal_ptr, ctx->gal64, g->gal_ptr[N],
-                     beep::shortest_normal_run(N, g->gal_ptr, g->gal_pts), ctx->gal_plane, ctx->gal_radius,
-                     nullptr, ctx->gal_planes);
-        hip_check(hipStreamSynchronize(s), "sync geometry upload");
+        PlaneCheck pc(ctx);
+        pc.launch(0, N, ctx->quad_ptr, ctx->quad64, g->quad_ptr[N],
+                  beep::shortest_normal_run(N, g->quad_ptr, g->quad_pts), ctx->quad_plane, ctx->quad_radius,
+                  &ctx->quad_xyzw);
+        pc.launch(1, N, ctx->gal_ptr, ctx->gal64, g->gal_ptr[N],
+                  beep::shortest_normal_run(N, g->gal_ptr, g->gal_pts), ctx->gal_plane, ctx->gal_radius, nullptr);
+        pc.read();
         geometry_done(ctx, N, g->centroid);
     });
 }
@@ -977,50 +997,50 @@ int beep_hip_set_surface(beep_hip_ctx* ctx, const beep_hip_surface* g) {
         ctx->svt_corner.upload(g->vt_corner, nvt, s);
         if (g->ctl_idx) ctx->sctl_idx.upload(g->ctl_idx, T, s);
         if (NC > 0) ctx->sctl.upload(g->ctl, size_t(63) * NC, s);
-        // one point set per rule: counts (1, or 2 sub-triangles x k points per
-        // triangle around the vertex), then the points on the device
-        std::vector<int> ptr(size_t(N) + 1);
-        auto make = [&](int order, DevBuf<int>& dptr, DevBuf<Pt64>& o64, DevBuf<Pt32>* o32,
-                        int per_area) {
-            RuleDev rd{};
-            if (order != 0) {
-                const beep::Rule& r = beep::rule_for_order(order);
-                rd.k = int(r.w.size());
-                for (int j = 0; j < rd.k; ++j) {
-                    rd.u[j] = r.u[j];
-                    rd.v[j] = r.v[j];
-                    rd.w[j] = r.w[j];
+        // one point set per rule (qualocation, quadrature, galerkin): counts (1,
+        // or 2 sub-triangles x k points per triangle around the vertex) for all
+        // three, then the points on the device
+        const int rules[3] = {g->qual_rule, g->quad_rule, 4};
+        RuleDev rd[3] = {};
+        std::vector<int> ptr[3];
+        for (int q = 0; q < 3; ++q) {
+            if (rules[q] != 0) {
+                const beep::Rule& r = beep::rule_for_order(rules[q]);
+                rd[q].k = int(r.w.size());
+                for (int j = 0; j < rd[q].k; ++j) {
+                    rd[q].u[j] = r.u[j];
+                    rd[q].v[j] = r.v[j];
+                    rd[q].w[j] = r.w[j];
                 }
             }
-            ptr[0] = 0;
+            ptr[q].resize(size_t(N) + 1);
+            ptr[q][0] = 0;
             for (int p = 0; p < N; ++p) {
-                const int64_t c = rd.k == 0 ? 1 : int64_t(2) * (g->vt_ptr[p + 1] - g->vt_ptr[p]) * rd.k;
-                require(ptr[p] + c < int64_t(0x7fffffff), "too many points for 32-bit offsets");
-                ptr[p + 1] = ptr[p] + int(c);
+                const int64_t c = rd[q].k == 0 ? 1 : int64_t(2) * (g->vt_ptr[p + 1] - g->vt_ptr[p]) * rd[q].k;
+                require(ptr[q][p] + c < int64_t(0x7fffffff), "too many points for 32-bit offsets");
+                ptr[q][p + 1] = ptr[q][p] + int(c);
             }
-            dptr.upload(ptr.data(), N + 1, s);
-            o64.alloc(size_t(ptr[N]) + 1);  // one behind the last: PointPlanes
-            if (o32) o32->alloc(size_t(ptr[N]));
+        }
+        auto make = [&](int q, DevBuf<int>& dptr, DevBuf<Pt64>& o64, DevBuf<Pt32>* o32, int per_area) {
+            const size_t total = size_t(ptr[q][N]);
+            dptr.upload(ptr[q].data(), N + 1, s);
+            o64.alloc(total + 1);  // one behind the last: PointPlanes
+            if (o32) o32->alloc(total);
             launch_gen_points(s, N, ctx->sverts.p, ctx->stris.p, ctx->svt_ptr.p, ctx->svt_tri.p,
                               ctx->svt_corner.p, g->ctl_idx ? ctx->sctl_idx.p : nullptr,
-                              NC > 0 ? ctx->sctl.p : nullptr, ctx->patches.p, dptr.p, rd, per_area,
+                              NC > 0 ? ctx->sctl.p : nullptr, ctx->patches.p, dptr.p, rd[q], per_area,
                               o64.p, o32 ? o32->p : nullptr);
-            hip_check(hipStreamSynchronize(s), "sync point generation");  // ptr is reused
         };
-        make(g->qual_rule, ctx->qual_ptr, ctx->qual64, &ctx->qual32, 1);
-        make(g->quad_rule, ctx->quad_ptr, ctx->quad64, &ctx->quad32, 0);
-        const int nq_quad = ptr[N];
-        make(4, ctx->gal_ptr, ctx->gal64, nullptr, 0);
-        const int nq_gal = ptr[N];
+        make(0, ctx->qual_ptr, ctx->qual64, &ctx->qual32, 1);
+        make(1, ctx->quad_ptr, ctx->quad64, &ctx->quad32, 0);
+        make(2, ctx->gal_ptr, ctx->gal64, nullptr, 0);
         // a planar triangle's two sub-triangles share its plane
-        const bool planar = NC == 0;
-        auto runs = [&](int order) {
-            return planar && order != 0 ? 2 * int(beep::rule_for_order(order).w.size()) : 0;
-        };
-        point_planes(ctx, N, ctx->quad_ptr, ctx->quad64, nq_quad, runs(g->quad_rule), ctx->quad_plane,
-                     ctx->quad_radius, &ctx->quad_xyzw, ctx->quad_planes);
-        point_planes(ctx, N, ctx->gal_ptr, ctx->gal64, nq_gal, runs(4), ctx->gal_plane, ctx->gal_radius,
-                     nullptr, ctx->gal_planes);
+        auto runs = [&](int q) { return NC == 0 ? 2 * rd[q].k : 0; };
+        PlaneCheck pc(ctx);
+        pc.launch(0, N, ctx->quad_ptr, ctx->quad64, ptr[1][N], runs(1), ctx->quad_plane, ctx->quad_radius,
+                  &ctx->quad_xyzw);
+        pc.launch(1, N, ctx->gal_ptr, ctx->gal64, ptr[2][N], runs(2), ctx->gal_plane, ctx->gal_radius, nullptr);
+        pc.read();  // host arrays die here
         geometry_done(ctx, N, g->centroid);
     });
 }

@@ -181,3 +181,26 @@ def test_energy_run_lengths(gs):
     print(gs, rel(renormalise(ef, a), rf), rel(eh, rh), flush=True)
     assert rel(renormalise(ef, a), rf) < 1e-12 and rel(eh, rh) < 1e-12
     d.close()
+
+
+def test_one_context_over_point_sets_of_both_forms():
+    """Whether a set is in planar runs is found again for every geometry."""
+    planar = arrays(6, 0, 0.125)
+    bent = {k: (v.copy() if isinstance(v, np.ndarray) else v) for k, v in planar.items()}
+    for s in ("quad", "gal"):
+        k = bent[f"{s}_ptr"][70] + 1
+        bent[s][k, 3:6] = bent[s][k + 12, 3:6]
+    point = arrays(0, 0, 0.125)
+    d = Device(0)
+    d.set_far_field("direct", 5, 40)
+    x = np.random.default_rng(2).normal(size=2 * planar["area"].shape[0])
+    for a in (planar, bent, bent, planar, point, planar):
+        d.set_geometry(a)
+        d.set_tree(a)
+        d.precompute(0.125, "fp64")
+        orc = oracle.Oracle(a, 0.125, 80.0)
+        assert rel(d.matvec(x, "fp64"), orc.matvec(x)) < 1e-12
+        ef, eh = d.energy_coefficients(a["inst_patch_ptr"], a["inst_charge_ptr"], a["charges"])
+        rf, rh = orc.energy_coeffs()
+        assert rel(renormalise(ef, a), rf) < 1e-12 and rel(eh, rh) < 1e-12
+    d.close()
