@@ -2,6 +2,7 @@
 // upload, precompute, mat-vec (do_bem_fmm_iteration), RHS, energy
 // coefficients and the device GMRES / iterative-refinement driver.
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <chrono>
 #include <cmath>
@@ -98,6 +99,7 @@ struct beep_hip_ctx {
     // yfar; the context stream adds it to y (fork / join through events)
     hipStream_t far_stream = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_pack = nullptr;
+    hipEvent_t ev_coef = nullptr;  // the last precompute's coefficients written
     static constexpr int SPMV_CAP_AUTO = -1;
     bool overlap = true;
     int n_cu = 256;               // compute units of the device
@@ -161,10 +163,13 @@ struct beep_hip_ctx {
     long long n_nb = 0;  // neighbourhood entries (nb_ptr[L])
     bool have_tree = false;
     bool all_explicit = false;  // every pair of patches is an explicit pair, once
-    // this context's near field was shared (beep_hip_share_near): its
-    // coefficients store full - 1 point from then on (see folded)
-    bool keep_1pt = false;
+    // this context's near field was shared (beep_hip_share_near): precomputes
+    // store full - 1 point from then on (see folded); of an FP64 set that was
+    // folded by then, full - 1 point for the contexts that share it (share64)
+    std::atomic<bool> keep_1pt{false};
     std::mutex share_mu;
+    DevBuf<double2> coef64_sub;
+    bool have64_sub = false;
 
     // precomputed operator
     DevBuf<double> diag;
@@ -418,6 +423,13 @@ bool folded(const beep_hip_ctx* c, int precision) {
     return !c->use_fmm && !c->share && built_for(c, precision) == beep_hip_ctx::UID_FOLDED;
 }
 
+// the FP64 set (full - 1 point) of h for the contexts that share it; null: share64
+// has to make it first
+const double2* shared64(const beep_hip_ctx* h) {
+    if (h->uid64 != beep_hip_ctx::UID_FOLDED) return h->coef64.p;
+    return h->have64_sub ? h->coef64_sub.p : nullptr;
+}
+
 // this precision's set fits the far field in use (either form of it without
 // the FMM)
 bool coef_plan_ok(const beep_hip_ctx* c, int precision) {
@@ -481,6 +493,8 @@ void matvec_dev(beep_hip_ctx* c, const double* dx, double* dy, int precision) {
     if (c->share) {
         require(precision == BEEP_FP64 ? c->share->have64 : c->share->have32,
                 "the shared near field lacks this precision's coefficients");
+        require(precision != BEEP_FP64 || shared64(c->share),
+                "the shared near field was precomputed anew: call beep_hip_precompute again");
     } else {
         require(coef_plan_ok(c, precision),
                 "near coefficients were precomputed for another far field: call "
@@ -547,7 +561,7 @@ void matvec_dev(beep_hip_ctx* c, const double* dx, double* dy, int precision) {
         const int nco = int(c->share_off.size());
         for (int k = 0; k < nco; k += 2)
             launch_near_spmv(s, mode, c->N, h->spmv, h->leaf_ptr.p, h->leaf_idx.p, h->nb_ptr.p,
-                             h->nb_idx.p, h->coef_off.p, h->coef32.p, h->coef64.p, h->diag.p, dx,
+                             h->nb_idx.p, h->coef_off.p, h->coef32.p, shared64(h), h->diag.p, dx,
                              c->spmv_part.p, dy, spmv_blocks(c, mode), c->spmv_depth[mode], c->spmv_next.p,
                              std::min(2, nco - k), c->share_off.data() + k);
         launch_pair_spmv(s, mode, c->N, c->n_pair_rows, c->pair_rows.p, c->pair_ptr.p, c->pair_col.p,
@@ -816,6 +830,7 @@ int beep_hip_create(int device, beep_hip_ctx** out) {
         hip_check(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming), "hipEventCreate");
         hip_check(hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming), "hipEventCreate");
         hip_check(hipEventCreateWithFlags(&c->ev_pack, hipEventDisableTiming), "hipEventCreate");
+        hip_check(hipEventCreateWithFlags(&c->ev_coef, hipEventDisableTiming), "hipEventCreate");
         for (auto& set : c->ev)
             for (auto& e : set) hip_check(hipEventCreate(&e), "hipEventCreate");
     });
@@ -828,6 +843,7 @@ int beep_hip_create(int device, beep_hip_ctx** out) {
         if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
         if (c->ev_join) (void)hipEventDestroy(c->ev_join);
         if (c->ev_pack) (void)hipEventDestroy(c->ev_pack);
+        if (c->ev_coef) (void)hipEventDestroy(c->ev_coef);
         if (c->far_stream) (void)hipStreamDestroy(c->far_stream);
         if (c->stream) (void)hipStreamDestroy(c->stream);
         return rc;
@@ -850,6 +866,7 @@ int beep_hip_destroy(beep_hip_ctx* ctx) {
     if (ctx->ev_fork) (void)hipEventDestroy(ctx->ev_fork);
     if (ctx->ev_join) (void)hipEventDestroy(ctx->ev_join);
     if (ctx->ev_pack) (void)hipEventDestroy(ctx->ev_pack);
+    if (ctx->ev_coef) (void)hipEventDestroy(ctx->ev_coef);
     if (ctx->far_stream) (void)hipStreamDestroy(ctx->far_stream);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -1054,6 +1071,8 @@ static void begin_tree(beep_hip_ctx* ctx) {
     ctx->all_explicit = ctx->keep_1pt = false;
     set_device(ctx);
     sync_streams(ctx);
+    ctx->coef64_sub.reset();
+    ctx->have64_sub = false;
     ctx->gen++;
 }
 
@@ -1309,15 +1328,47 @@ int beep_hip_get_tree(beep_hip_ctx* ctx, int* leaf_ptr, int* leaf_idx, int* nb_p
     });
 }
 
-// Singular terms and the near coefficients of one precision.  With the FMM
-// the plan is built first: explicit pairs its leaf pass covers keep the full
-// rule (their packed leaf cells are adjacent) and the leaf pass runs over
-// the residual pairs only.
+// the guard's counters, zero at first
+void guard_counters(beep_hip_ctx* ctx) {
+    if (ctx->guard_cnt.p) return;
+    ctx->guard_cnt.alloc(5);
+    for (int k = 0; k < 5; ++k) launch_set_int(ctx->stream, reinterpret_cast<int*>(ctx->guard_cnt.p + k), 0);
+}
+
+// For a context that shares src's near field: src's FP64 set as full - 1
+// point, if src's own is folded.  A set beside src's own (as large again), on
+// ctx's stream and with ctx's guard list: the owner of src may run mat-vecs
+// meanwhile, and other contexts that share it wait here.
+void share64(beep_hip_ctx* ctx, beep_hip_ctx* src) {
+    std::lock_guard<std::mutex> lk(src->share_mu);
+    src->keep_1pt = true;
+    if (!src->have64 || shared64(src)) return;
+    size_t freeb = 0, totalb = 0;
+    hip_check(hipMemGetInfo(&freeb, &totalb), "hipMemGetInfo");
+    const size_t need = coef64_size(src->nnz) * sizeof(double2), have = src->coef64_sub.n * sizeof(double2);
+    require(need <= have || need + (size_t(1) << 30) < freeb + have,
+            "not enough device memory for FP64 coefficients");
+    src->coef64_sub.alloc(coef64_size(src->nnz));
+    hipStream_t s = ctx->stream;
+    ctx->guard_rec.alloc(beep_hip_ctx::GUARD_CAP);
+    guard_counters(ctx);
+    unsigned* gcnt = ctx->guard_cnt.p;
+    const NsList guard{ctx->guard_rec.p, gcnt, beep_hip_ctx::GUARD_CAP};
+    launch_near_coeffs_fp64(s, src->n_coef_blocks, src->L, src->coef_blk.p, src->leaf_ptr.p, src->leaf_idx.p,
+                            src->nb_ptr.p, src->nb_idx.p, src->coef_off.p, src->patches.p, src->qual_ptr.p,
+                            src->qual64.p, src->quad_ptr.p, src->quad64.p, src->quad_planes, src->kappa, 1, nullptr,
+                            guard, src->guard_max, src->coef64_sub.p);
+    launch_coef_repair(s, 0, guard, src->patches.p, src->qual_ptr.p, src->qual64.p, src->quad_ptr.p, src->quad64.p,
+                       src->quad_planes, src->kappa, 1, src->guard_max, gcnt + 1, src->coef64_sub.p);
+    hip_check(hipStreamSynchronize(s), "sync shared coefficients");
+    src->have64_sub = true;
+}
+
 // Precompute of a context whose near field is shared (beep_hip_share_near):
 // the listed pairs' coefficients (both precisions) for the shared sets'
 // kappa; the diagonal and the other explicit pairs are the shared context's.
 void precompute_shared(beep_hip_ctx* ctx, double kappa, int precision) {
-    const beep_hip_ctx* h = ctx->share;
+    beep_hip_ctx* h = ctx->share;
     require(h->have_diag && h->kappa == kappa, "the shared near field has another kappa");
     require(precision == BEEP_FP64 ? h->have64 : h->have32,
             "the shared near field lacks this precision's coefficients");
@@ -1325,10 +1376,10 @@ void precompute_shared(beep_hip_ctx* ctx, double kappa, int precision) {
     ctx->gen++;
     hipStream_t s = ctx->stream;
     ctx->kappa = kappa;
-    if (!ctx->guard_cnt.p) {
-        ctx->guard_cnt.alloc(5);
-        for (int k = 0; k < 5; ++k) launch_set_int(s, reinterpret_cast<int*>(ctx->guard_cnt.p + k), 0);
-    }
+    // the shared sets may have been precomputed anew, and be under way still
+    hip_check(hipStreamWaitEvent(s, h->ev_coef, 0), "hipStreamWaitEvent");
+    if (precision == BEEP_FP64) share64(ctx, h);
+    guard_counters(ctx);
     unsigned* gcnt = ctx->guard_cnt.p;
     launch_set_int(s, reinterpret_cast<int*>(gcnt + 1), 0);
     launch_set_int(s, reinterpret_cast<int*>(gcnt + 2), 0);
@@ -1342,6 +1393,10 @@ void precompute_shared(beep_hip_ctx* ctx, double kappa, int precision) {
     ensure_far(ctx, precision);
 }
 
+// Singular terms and the near coefficients of one precision.  With the FMM
+// the plan is built first: explicit pairs its leaf pass covers keep the full
+// rule (their packed leaf cells are adjacent) and the leaf pass runs over
+// the residual pairs only.
 void precompute_impl(beep_hip_ctx* ctx, double kappa, int precision) {
     if (ctx->share) {
         require(precision == BEEP_FP64 || precision == BEEP_FP32 || precision == BEEP_FP32_RESID,
@@ -1357,18 +1412,16 @@ void precompute_impl(beep_hip_ctx* ctx, double kappa, int precision) {
     sync_streams(ctx);
     ctx->gen++;
     if (ctx->have_diag && kappa != ctx->kappa) {
-        ctx->have32 = ctx->have64 = false;
+        ctx->have32 = ctx->have64 = ctx->have64_sub = false;
         ctx->coef32.reset();
         ctx->coef64.reset();
+        ctx->coef64_sub.reset();
     }
     hipStream_t s = ctx->stream;
     ctx->kappa = kappa;
     ctx->diag.alloc(size_t(4) * ctx->N);
     ctx->guard_rec.alloc(beep_hip_ctx::GUARD_CAP);
-    if (!ctx->guard_cnt.p) {
-        ctx->guard_cnt.alloc(5);
-        for (int k = 0; k < 5; ++k) launch_set_int(s, reinterpret_cast<int*>(ctx->guard_cnt.p + k), 0);
-    }
+    guard_counters(ctx);
     unsigned* gcnt = ctx->guard_cnt.p;
     const NsList guard{ctx->guard_rec.p, gcnt, beep_hip_ctx::GUARD_CAP};
     launch_set_int(s, reinterpret_cast<int*>(gcnt + 3), 0);
@@ -1454,6 +1507,7 @@ void precompute_impl(beep_hip_ctx* ctx, double kappa, int precision) {
         ctx->have32 = true;
         ctx->uid32 = uid;
     }
+    hip_check(hipEventRecord(ctx->ev_coef, s), "hipEventRecord");
     // the rest of the plan, its residual leaf-pass list (with cell keys,
     // the list the coefficients assume) and the kernel tables are built on
     // the host and the far stream while the coefficient kernels run (no
@@ -1511,18 +1565,7 @@ void share_common(beep_hip_ctx* ctx, beep_hip_ctx* src, int n_copies, const int*
             "a shared near field needs stored coefficients (near mode BEEP_NEAR_PRECOMPUTE)");
     require(src->have_geom && src->have_tree && src->have_diag && (src->have32 || src->have64),
             "the shared context must have its geometry, tree and coefficients");
-    {
-        // a folded source (no far field of its own) stores full - 1 point from
-        // now on; the first sharer recomputes its sets, the others wait here
-        std::lock_guard<std::mutex> lk(src->share_mu);
-        src->keep_1pt = true;
-        if (src->have64 && folded(src, BEEP_FP64)) {
-            set_device(src);
-            precompute_impl(src, src->kappa, BEEP_FP64);
-            sync_streams(src);
-        }
-    }
-    require(src->uid32 == 0 && src->uid64 == 0,
+    require(src->uid32 == 0 && (src->uid64 == 0 || src->uid64 == beep_hip_ctx::UID_FOLDED),
             "the shared coefficients must be precomputed with the direct far field");
     require(n_copies >= 1 && copy_offset, "no copies");
     const int N = ctx->N, Ns = src->N;
@@ -1537,6 +1580,7 @@ void share_common(beep_hip_ctx* ctx, beep_hip_ctx* src, int n_copies, const int*
     }
     set_device(ctx);
     sync_streams(ctx);
+    share64(ctx, src);
     hipStream_t s = ctx->stream;
     ctx->gen++;
     ctx->have_tree = false;
@@ -1691,6 +1735,8 @@ int beep_hip_set_near_mode(beep_hip_ctx* ctx, int mode) {
             ctx->coef32.reset();
             ctx->coef64.reset();
         }
+        ctx->coef64_sub.reset();
+        ctx->have64_sub = false;
     });
 }
 
@@ -1769,6 +1815,14 @@ int beep_hip_sanity_check(beep_hip_ctx* ctx, long long* repaired) {
             launch_coef_repair(s, fp32, guard, ctx->patches.p, ctx->qual_ptr.p, ctx->qual64.p,
                                ctx->quad_ptr.p, ctx->quad64.p, ctx->quad_planes, ctx->kappa, sub_1pt,
                                ctx->guard_max, gcnt + 4, coef);
+        }
+        if (ctx->have64_sub) {  // full - 1 point for the contexts that share a folded set
+            launch_coef_scan(s, 0, ctx->n_coef_blocks, ctx->L, ctx->coef_blk.p, ctx->leaf_ptr.p, ctx->leaf_idx.p,
+                             ctx->nb_ptr.p, ctx->nb_idx.p, ctx->coef_off.p, nullptr, 1, ctx->patches.p, ctx->kappa,
+                             ctx->coef64_sub.p, ctx->guard_max, guard);
+            launch_coef_repair(s, 0, guard, ctx->patches.p, ctx->qual_ptr.p, ctx->qual64.p, ctx->quad_ptr.p,
+                               ctx->quad64.p, ctx->quad_planes, ctx->kappa, 1, ctx->guard_max, gcnt + 4,
+                               ctx->coef64_sub.p);
         }
         unsigned h = 0;
         hip_check(hipMemcpyAsync(&h, gcnt + 4, sizeof(h), hipMemcpyDeviceToHost, s), "D2H guard count");
@@ -2422,7 +2476,7 @@ int beep_hip_memory_held(beep_hip_ctx* ctx, size_t* bytes) {
         add(ctx->leaf_ptr); add(ctx->leaf_idx); add(ctx->nb_ptr); add(ctx->nb_idx);
         add(ctx->coef_off); add(ctx->coef_blk); add(ctx->spmv_work); add(ctx->spmv_groups);
         add(ctx->spmv_group_nblk); add(ctx->spmv_part); add(ctx->diag); add(ctx->coef32);
-        add(ctx->coef64); add(ctx->src); add(ctx->xbuf); add(ctx->ybuf); add(ctx->yfar);
+        add(ctx->coef64); add(ctx->coef64_sub); add(ctx->src); add(ctx->xbuf); add(ctx->ybuf); add(ctx->yfar);
         add(ctx->far_part);
         add(ctx->qbuf); add(ctx->rhsbuf); add(ctx->ecf); add(ctx->ech); add(ctx->pinst_d);
         add(ctx->icp_d); add(ctx->V); add(ctx->hvec); add(ctx->partial); add(ctx->wtmp);

@@ -339,8 +339,13 @@ int beep_hip_debug_poke(beep_hip_ctx* ctx, int which, long long entry, const dou
  * repeats).  Takes the place of beep_hip_set_tree; beep_hip_precompute then
  * computes only the listed pairs' coefficients (in FP64, kept in both
  * precisions), for src's kappa.  The FMM leaf pass then covers every
- * neighbouring-leaf pair.  src must outlive this use and not change
- * meanwhile; contexts sharing one src may run concurrently.  Replaces the
+ * neighbouring-leaf pair.  src must outlive this use and not be changed
+ * meanwhile (geometry, tree, precompute); contexts sharing one src, and src's
+ * own mat-vecs, may run concurrently.  Where src holds an FP64 set without a
+ * far field (BEEP_FAR_AUTO, every pair of patches explicit: its entries are
+ * full rules), the first context to share it, or its precompute, computes the
+ * set less the 1-point interaction beside it, for all that share src: the
+ * time and device memory of an FP64 precompute of src.  Replaces the
  * per-pose LocalIntegrations of the reference's pose loop (tools/
  * run_pair.py:34-52 -> beep.cpp:223-290, 768-956), which recomputes the
  * intra-instance pairs for every pose. */

@@ -1,10 +1,13 @@
 """The direct far field as symmetric tile pairs and the FP64 set without a far
 field, against the FP64 CPU oracle, at the edges of the 256- and 64-patch
 tiles and of the SpMV's work items, over every route to them."""
+import threading
+
 import numpy as np
 import pytest
 
 import oracle
+from beep3_amd._lib import BeepError
 from beep3_amd.device import Device
 from beep3_amd.scene import Mesh, Scene
 
@@ -113,6 +116,57 @@ def test_shared_near_field_of_a_one_leaf_mesh():
         assert rel(pose.matvec(x, p), ref) < tol
     assert rel(src.matvec(x1, "fp64"), y1) < 1e-12
     pose.close()
+    src.close()
+
+
+def test_sharing_leaves_the_source_as_it_is():
+    """Sharing only reads the source: its FP64 product keeps its bits, also
+    while another thread shares it; a refused share costs it nothing; and the
+    contexts that share it follow a new precompute of it."""
+    one = scene((3,), 1500)
+    n = one["area"].shape[0]
+    src = device(one)
+    x1 = np.random.default_rng(1).normal(size=2 * n)
+    y1 = src.matvec(x1, "fp64")
+    held = src.memory_held()
+    two = Scene(80.0, 0.125, 6, 0, 1500)
+    m = Mesh.star(3, 25.0, 8, 0.04, 5)
+    two = two.add_instance(m, 2.0).add_instance(m, 2.0, offset=[80.0, 0.0, 0.0]).build().arrays()
+    x = np.random.default_rng(2).normal(size=4 * n)
+    poses = [Device(0) for _ in range(3)]
+    for d in poses:
+        d.set_far_field("direct", 5, 40)
+        d.set_geometry(two)
+    with pytest.raises(BeepError, match="overlap"):
+        poses[0].share_near(src, [0, 0])
+    assert src.memory_held() == held and np.array_equal(src.matvec(x1, "fp64"), y1)
+    out = [None] * 3
+
+    def share(k):
+        poses[k].share_near(src, [0, n])
+        poses[k].precompute(0.125, "fp64")
+        out[k] = poses[k].matvec(x, "fp64")
+
+    threads = [threading.Thread(target=share, args=(k,)) for k in range(3)]
+    for t in threads:
+        t.start()
+    same = [np.array_equal(src.matvec(x1, "fp64"), y1) for _ in range(50)]
+    for t in threads:
+        t.join()
+    assert all(same) and np.array_equal(src.matvec(x1, "fp64"), y1)
+    assert all(np.array_equal(o, out[0]) for o in out)
+    assert src.sanity_check() == 0
+    # a new precompute of a shared source (the set in another form), then of
+    # a new tree (folded again)
+    src.precompute(0.125, "fp64")
+    poses[0].precompute(0.125, "fp64")
+    assert rel(poses[0].matvec(x, "fp64"), out[0]) < 1e-13
+    src.set_tree(one)
+    src.precompute(0.125, "fp64")
+    poses[0].precompute(0.125, "fp64")
+    assert rel(poses[0].matvec(x, "fp64"), out[0]) < 1e-13
+    for d in poses:
+        d.close()
     src.close()
 
 
