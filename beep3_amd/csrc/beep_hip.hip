@@ -441,6 +441,11 @@ bool coef_plan_ok(const beep_hip_ctx* c, int precision) {
 // the direct far field as symmetric tile pairs (far_sym.hpp)
 bool far_is_sym(const beep_hip_ctx* c) { return !c->use_fmm && c->N <= FAR_SYM_MAX; }
 
+// near and far field of a mat-vec in one launch (launch_direct_matvec)
+bool one_launch(const beep_hip_ctx* c, int precision) {
+    return far_is_sym(c) && !folded(c, precision) && c->overlap && !c->share && c->near_mode == BEEP_NEAR_PRECOMPUTE;
+}
+
 // Blocks of the near SpMV (0: one per work item).  By default one block per
 // CU beside the FMM and beside the direct sum in one direction (23,046 / 40,962
 // patches, FP32: 790 / 2,267 us, uncapped 843 / 2,387), uncapped beside
@@ -522,11 +527,11 @@ void matvec_dev(beep_hip_ctx* c, const double* dx, double* dy, int precision) {
         c->ring_head = (c->ring_head + 1) % beep_hip_ctx::RING;
         c->ring_pending += 1;
     };
-    if (sym && !fold && c->overlap && !c->share && c->near_mode == BEEP_NEAR_PRECOMPUTE) {
+    if (one_launch(c, precision)) {
         // near and far field side by side in one launch, one that sums them
         launch_direct_matvec(s, mode, c->N, c->spmv, c->leaf_ptr.p, c->leaf_idx.p, c->nb_ptr.p, c->nb_idx.p,
                              c->coef_off.p, c->coef32.p, c->coef64.p, c->diag.p, c->patches.p, c->kappa, dx,
-                             c->spmv_part.p, c->far_part.p, dy);
+                             c->spmv_depth[mode], c->spmv_part.p, c->far_part.p, dy);
         if (timed) {
             hip_check(hipEventRecord(ev[1], s), "hipEventRecord");
             hip_check(hipEventRecord(ev[3], s), "hipEventRecord");
@@ -1958,7 +1963,7 @@ int beep_hip_matvec_device_noalloc(beep_hip_ctx* ctx, const double* dx, double* 
         if (sym && !fold && !fly) {
             launch_direct_matvec(s, mode, N, ctx->spmv, ctx->leaf_ptr.p, ctx->leaf_idx.p, ctx->nb_ptr.p,
                                  ctx->nb_idx.p, ctx->coef_off.p, ctx->coef32.p, ctx->coef64.p, ctx->diag.p,
-                                 ctx->patches.p, ctx->kappa, dx, spart, far, dy);
+                                 ctx->patches.p, ctx->kappa, dx, ctx->spmv_depth[mode], spart, far, dy);
             return;
         }
         if (fly)
@@ -2064,10 +2069,11 @@ int beep_hip_set_spmv_depth(beep_hip_ctx* ctx, int depth) {
 
 // Times `reps` whole mat-vecs (after one warm-up) for each candidate value of
 // one SpMV setting, keeps the fastest.  `table` is the per-mode setting; the
-// entry of the precision's mode is tuned.
+// entry of the precision's mode is tuned.  applies: the context's mat-vecs use
+// the setting; else one time goes for every candidate and the setting stays.
 static void tune_spmv_setting(beep_hip_ctx* ctx, int precision, int (beep_hip_ctx::*table)[3],
                               const int* values, int n, int reps, bool (*valid)(int),
-                              const char* what, double* ms_out, int* best) {
+                              const char* what, bool applies, double* ms_out, int* best) {
     require(precision == BEEP_FP64 || precision == BEEP_FP32 || precision == BEEP_FP32_RESID,
             "unknown precision");
     int* field = &(ctx->*table)[spmv_mode(precision)];
@@ -2085,10 +2091,11 @@ static void tune_spmv_setting(beep_hip_ctx* ctx, int precision, int (beep_hip_ct
     hip_check(hipEventCreate(&e1), "hipEventCreate");
     const int saved = *field;
     double best_ms = 1e300;
-    int best_v = saved;
+    int best_v = std::find(values, values + n, saved) != values + n ? saved : values[0];
     try {
         for (int k = 0; k < n; ++k) {
-            *field = values[k];
+            if (applies) *field = values[k];
+            else if (k > 0) break;
             matvec_dev(ctx, ctx->xbuf.p, ctx->ybuf.p, precision);  // warm-up
             hip_check(hipEventRecord(e0, ctx->stream), "hipEventRecord");
             for (int r = 0; r < reps; ++r) matvec_dev(ctx, ctx->xbuf.p, ctx->ybuf.p, precision);
@@ -2098,10 +2105,11 @@ static void tune_spmv_setting(beep_hip_ctx* ctx, int precision, int (beep_hip_ct
             hip_check(hipEventElapsedTime(&ms, e0, e1), "hipEventElapsedTime");
             const double per = double(ms) / reps;
             if (ms_out) ms_out[k] = per;
-            if (per < best_ms) {
+            if (applies && per < best_ms) {
                 best_ms = per;
                 best_v = values[k];
             }
+            if (!applies && ms_out) std::fill(ms_out, ms_out + n, per);
         }
     } catch (...) {
         (void)hipEventDestroy(e0);
@@ -2113,7 +2121,7 @@ static void tune_spmv_setting(beep_hip_ctx* ctx, int precision, int (beep_hip_ct
     (void)hipEventDestroy(e1);
     timing_collect(ctx);
     ctx->timing = beep_matvec_timing{};
-    *field = best_v;
+    *field = applies ? best_v : saved;
     ctx->gen++;
     if (best) *best = best_v;
 }
@@ -2123,7 +2131,7 @@ int beep_hip_autotune_spmv(beep_hip_ctx* ctx, int precision, const int* blocks_p
     return guarded(ctx, [&] {
         tune_spmv_setting(ctx, precision, &beep_hip_ctx::spmv_cap, blocks_per_cu, n, reps,
                           [](int v) { return v >= 0 && v <= 64; }, "blocks per CU must be 0..64",
-                          ms_out, best);
+                          !one_launch(ctx, precision), ms_out, best);
     });
 }
 
@@ -2132,7 +2140,7 @@ int beep_hip_autotune_spmv_depth(beep_hip_ctx* ctx, int precision, const int* de
     return guarded(ctx, [&] {
         tune_spmv_setting(ctx, precision, &beep_hip_ctx::spmv_depth, depths, n, reps,
                           [](int v) { return v == 1 || v == 2 || v == 4; },
-                          "SpMV depth must be 1, 2 or 4", ms_out, best);
+                          "SpMV depth must be 1, 2 or 4", true, ms_out, best);
     });
 }
 

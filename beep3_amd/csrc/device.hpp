@@ -294,7 +294,7 @@ void launch_far_sym_add(hipStream_t s, int fp32, int n, const int* order, const 
 void launch_direct_matvec(hipStream_t s, int mode, int n, const SpmvPlan& p, const int* leaf_ptr,
                           const int* leaf_idx, const int* nb_ptr, const int* nb_idx, const int64_t* coef_off,
                           const float4* coef32, const double2* coef64, const double* diag4, const Patch64* patches,
-                          double kappa, const double* x, void* part, void* far_part, double* y);
+                          double kappa, const double* x, int depth, void* part, void* far_part, double* y);
 // y += direct far field; n_split > 1 needs part: 2 n n_split doubles
 void launch_far_direct(hipStream_t s, int fp32, int n, int n_split, const int* order,
                        const Patch64* patches, const Src64* src, double kappa, double* y,

@@ -959,17 +959,23 @@ static void direct_matvec(hipStream_t s, int n, const SpmvPlan& p, const int* le
 void launch_direct_matvec(hipStream_t s, int mode, int n, const SpmvPlan& p, const int* leaf_ptr,
                           const int* leaf_idx, const int* nb_ptr, const int* nb_idx, const int64_t* coef_off,
                           const float4* coef32, const double2* coef64, const double* diag4, const Patch64* patches,
-                          double kappa, const double* x, void* part, void* far_part, double* y) {
+                          double kappa, const double* x, int depth, void* part, void* far_part, double* y) {
     if (p.n_work <= 0) return;
-    if (mode == 0)
-        direct_matvec<double, double, 4, double>(s, n, p, leaf_ptr, leaf_idx, nb_ptr, nb_idx, coef_off, coef64,
-                                                 diag4, patches, kappa, x, (double*)part, (double*)far_part, y);
-    else if (mode == 1)
-        direct_matvec<float, float, 8, float>(s, n, p, leaf_ptr, leaf_idx, nb_ptr, nb_idx, coef_off, coef32, diag4,
-                                              patches, kappa, x, (float*)part, (float*)far_part, y);
-    else
-        direct_matvec<float, double, 8, double>(s, n, p, leaf_ptr, leaf_idx, nb_ptr, nb_idx, coef_off, coef32,
-                                                diag4, patches, kappa, x, (double*)part, (double*)far_part, y);
+    if (depth != 1 && depth != 2 && depth != 4) throw std::runtime_error("SpMV depth must be 1, 2 or 4");
+    auto go = [&](auto tc, auto ta, auto u, const void* coef) {  // u: loads in flight at depth 1
+        using TC = decltype(tc);
+        using TA = decltype(ta);
+        using TF = std::conditional_t<std::is_same<TA, float>::value, float, double>;
+        constexpr int U = u();
+        auto f = depth == 1   ? direct_matvec<TC, TA, U, TF>
+                 : depth == 2 ? direct_matvec<TC, TA, 2 * U, TF>
+                              : direct_matvec<TC, TA, 4 * U, TF>;
+        f(s, n, p, leaf_ptr, leaf_idx, nb_ptr, nb_idx, coef_off, coef, diag4, patches, kappa, x, (TA*)part,
+          (TF*)far_part, y);
+    };
+    if (mode == 0) go(double(), double(), std::integral_constant<int, 4>(), coef64);
+    else if (mode == 1) go(float(), float(), std::integral_constant<int, 8>(), coef32);
+    else go(float(), double(), std::integral_constant<int, 8>(), coef32);
 }
 
 // ---------------------------------------------------------------------------

@@ -151,8 +151,11 @@ typedef struct {
  * far field runs on a second stream while the near SpMV runs on the context
  * stream: near_ms and far_ms are then both measured from the start of the
  * mat-vec and total_ms is the whole mat-vec (max of the two + the final add).
- * With overlap off both run on the context stream, the near part first:
- * far_ms is then measured from the end of the near part. */
+ * Up to 20,480 patches with the direct far field and stored coefficients both
+ * run in one launch, and the one after it adds them up: near_ms and far_ms
+ * are then both the whole mat-vec.  An FP64 set without a far field has
+ * far_ms = near_ms.  With overlap off both run on the context stream, the
+ * near part first: far_ms is then measured from the end of the near part. */
 typedef struct {
     double near_ms;     /* last mat-vec: near-field SpMV + diagonal */
     double far_ms;      /* last mat-vec: far field */
@@ -214,9 +217,10 @@ int beep_hip_set_surface(beep_hip_ctx* ctx, const beep_hip_surface* surface);
 #define BEEP_FAR_PW 2
 int beep_hip_set_far_field(beep_hip_ctx* ctx, int mode, int order, int leaf_target);
 
-/* Far field on a second HIP stream, concurrent with the near-field SpMV
- * (on = 1, the default), or both on the context stream (on = 0).  The same
- * kernels run in the same order on each stream, so y is bit-identical.  This
+/* Far field concurrent with the near-field SpMV (on = 1, the default; on a
+ * second HIP stream, or in the same launch up to 20,480 patches with the
+ * direct far field), or one after the other on the context stream (on = 0).
+ * The same sums are formed in the same order, so y is bit-identical.  This
  * replaces the reference's "near field, then FMM" sequence
  * (beep.cpp:1517-1535), whose GPU near field finishes before the CPU FMM
  * starts (beep.cpp:1041-1045). */
@@ -256,7 +260,9 @@ int beep_hip_set_spmv_residency(beep_hip_ctx* ctx, int blocks_per_cu);
  * (far field overlapped) for each candidate, writes the mean times to ms_out
  * (may be NULL), keeps the fastest for mat-vecs of that precision (BEEP_FP64,
  * BEEP_FP32 and BEEP_FP32_RESID each keep their own) and returns it in
- * *best. */
+ * *best.  Where the mat-vec is one launch and no cap applies, all candidates
+ * get the same time, *best is the cap set or else the first candidate, and
+ * the cap set stays. */
 int beep_hip_autotune_spmv(beep_hip_ctx* ctx, int precision, const int* blocks_per_cu, int n,
                            int reps, double* ms_out, int* best);
 /* Coefficient loads each SpMV thread keeps in flight: 4 x depth (FP64

@@ -75,6 +75,32 @@ def test_direct_matvec_against_oracle(levels, nbsize, kappa):
     d.close()
 
 
+@pytest.mark.parametrize("levels,nbsize", [((3,), 1500), ((3, 2), 100), ((4,), 60)])
+def test_spmv_settings_of_the_one_launch(levels, nbsize):
+    """Near and far field in one launch: the load depth applies and changes no
+    bits, and can be tuned; no residency cap applies, so its tuner gives every
+    candidate one time and keeps the setting."""
+    a = scene(levels, nbsize)
+    n = a["area"].shape[0]
+    x = np.random.default_rng(n).normal(size=2 * n)
+    d = device(a, far="direct")
+    for p in ("fp64", "fp32", "fp32_resid"):
+        d.set_spmv_depth(1)
+        d.set_spmv_residency(1)  # not among the candidates below
+        y = d.matvec(x, p)
+        for depth in (2, 4):
+            d.set_spmv_depth(depth)
+            assert np.array_equal(d.matvec(x, p), y), (depth, p)
+        best, table = d.autotune_spmv_depth(p, (1, 2, 4), reps=2)
+        assert table[best] == min(table.values())
+        best, table = d.autotune_spmv(p, (3, 0, 2), reps=2)
+        assert best == 3 and len(set(table.values())) == 1
+        d.set_spmv_residency(2)
+        assert d.autotune_spmv(p, (3, 0, 2), reps=2)[0] == 2
+        assert np.array_equal(d.matvec(x, p), y)
+    d.close()
+
+
 @pytest.mark.parametrize("levels,nbsize", [((3,), 1500), ((3, 2), 100)])
 def test_direct_matvec_on_the_fly(levels, nbsize):
     a = scene(levels, nbsize)
