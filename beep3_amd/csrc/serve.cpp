@@ -51,7 +51,7 @@ void check_hip(beep_hip_ctx* c, int rc, const char* what) {
 
 // device bytes a scene will need in a context (upper estimate, reconciled
 // with beep_hip_memory_held after the request): point sets in both
-// precisions, coefficients of the solve's precisions, GMRES basis and
+// precisions and their planes, coefficients of the solve's precisions, GMRES basis and
 // per-patch FMM storage (tables, expansions, M2L slots: about 12 KB/patch)
 double estimate_bytes(const beep_scene* s, const beep_server_opts& o, bool stored) {
     const double N = double(s->centroid.size());
@@ -70,6 +70,9 @@ double estimate_bytes(const beep_scene* s, const beep_server_opts& o, bool store
         nnz = N * std::min(N, double(s->nbsize) + 1.0);
     }
     double b = 96.0 * (nq + nd) + 64.0 * ng + 64.0 * N;
+    // planar runs (of four points and more): positions and weights of the
+    // quadrature points again, a plane per run, two radii per patch
+    b += 16.0 * nd + 32.0 / 4.0 * (nd + ng) + 8.0 * N;
     if (stored && o.solve_mode != BEEP_SOLVE_FP64) b += 16.0 * nnz;
     if (stored && o.solve_mode == BEEP_SOLVE_FP64) b += 32.0 * nnz;
     b += 16.0 * N * double(o.max_iter + 1) + 16.0 * N * 8.0;

@@ -89,3 +89,21 @@ def test_estimate_counts_stored_coefficients():
     nnz = int(np.sum(np.diff(a["leaf_ptr"]) * np.diff(a["nb_ptr"])))
     assert fly > 0 and stored - fly == 16.0 * nnz
     srv.close()
+
+
+def test_estimate_counts_every_copy_of_the_points():
+    """What a quadrature point adds to the admission estimate covers all that
+    a context keeps of it: 56 bytes in FP64, 32 in FP32, 16 as position and
+    weight, and its part of its run's 32-byte plane (rule 6: runs of 12,
+    rule 16: of 32)."""
+    srv = Server(slots=1)
+    est, n = [], []
+    for quad in (6, 16):
+        sc = Scene(80.0, 0.125, quad, 0, 1500).add_instance(Mesh.icosphere(2, 2.0), 2.0)
+        est.append(srv.estimate(sc)[1])
+        a = sc.arrays()
+        n.append(int(a["quad_ptr"][-1]))
+    srv.close()
+    need = (56 + 32 + 16) * (n[1] - n[0]) + 32 * (n[1] / 32 - n[0] / 12)
+    print("estimates", est, "points", n, "needed", need)
+    assert est[1] - est[0] >= need
