@@ -94,9 +94,14 @@ def near_bytes(a, coef_bytes):
 # read 1 GiB for a 1 GiB device copy.  "spmv": the FP64 near-SpMV launch set
 # (k_near_spmv_part<double,double,*> + k_near_spmv_sum<double>; the depth
 # variants read the same); "fmm": one whole FP64 mat-vec with the Chebyshev
-# far field (SpMV, far field and the residual leaf pass).
-MEASURED_TRAFFIC = {("globular", "spmv", "fp64"): 8.309e9,
-                    ("globular", "fmm", "fp64"): 9.390e9}
+# far field (SpMV, far field and the residual leaf pass), leaf target 64.
+MEASURED_TRAFFIC = {("globular", "spmv", "fp64"): 8.162e9,
+                    ("globular", "fmm", "fp64"): 9.219e9}
+# Matrix FLOP that the order-5 M2L executes over its algorithmic FLOP, from
+# SQ_INSTS_VALU_MFMA_MOPS on the same surface (16.31 of 25.11 GFLOP,
+# profiles/mfma_counters_m2l_pw_163842.md): blocks of 75^2 + 50^2 for the
+# offsets with a symmetry, padded to tiles of 16
+M2L_EXECUTED = {5: 0.650}
 
 
 def cpu_model():
@@ -480,9 +485,10 @@ def main():
     best_d32 = min(alone, key=lambda k: alone[k][2])
     near_alone, far_alone = alone[best_d64][0], alone[best_d64][1]
     near32_alone, far32_alone = alone[best_d32][2], alone[best_d32][3]
-    # back to the tuned settings of every precision (or the library defaults);
-    # a tuner run over a single candidate sets one precision's value
-    dev.set_spmv_residency(1)
+    # back to the tuned settings of every precision (or the library defaults:
+    # no cap beside the symmetric direct far field, else one block per CU); a
+    # tuner run over a single candidate sets one precision's value
+    dev.set_spmv_residency(0 if dev.far_info()["mode"] == 0 and N <= 20480 else 1)
     dev.set_spmv_depth(1)
     for p in (("fp64", "fp32", "fp32_resid") if tune else ()):
         dev.autotune_spmv_depth(p, (tune[f"spmv_{p}"]["depth"],), reps=1)
@@ -521,18 +527,21 @@ def main():
     m2l = None
     if fi["mode"] == 1 and fi["m2l_pairs"] > 0:
         # algorithmic GEMM flops of M2L: 3 products of the P^3 x P^3 table with
-        # a source expansion per box pair (the block-diagonal form executes a
-        # little over half of them), over the k_m2l + k_m2l_sum time of a
+        # a source expansion per box pair, over the k_m2l + k_m2l_sum time of a
         # serialised mat-vec (and, beside it, of the overlapped one, where
-        # the SpMV shares the chip)
+        # the SpMV shares the chip); the share of the matrix peak is of the
+        # products executed (orders whose count was measured)
         NP = fi["order"] ** 3
         flops = 2.0 * 3 * NP * NP * fi["m2l_pairs"]
-        m2l = {"pairs": fi["m2l_pairs"], "gflop_per_launch": flops / 1e9}
+        executed = M2L_EXECUTED.get(fi["order"])
+        m2l = {"pairs": fi["m2l_pairs"], "gflop_per_launch": flops / 1e9,
+               "gflop_executed": flops * executed / 1e9 if executed else None}
         for p, peak in (("fp64", MFMA_FP64_TFLOPS), ("fp32", MFMA_FP32_TFLOPS)):
             ms = m2l_alone.get(p, 0.0)
             if ms > 0:
                 m2l[p] = {"ms": ms, "tflops": flops / (ms * 1e-3) / 1e12,
-                          "frac_of_mfma_peak": flops / (ms * 1e-3) / 1e12 / peak,
+                          "frac_of_mfma_peak": (flops * executed / (ms * 1e-3) / 1e12 / peak
+                                                if executed else None),
                           "ms_overlapped": rates[p]["m2l_ms"]}
     extra = {
         "near_spmv_alone_roofline": near_alone_roofline,
