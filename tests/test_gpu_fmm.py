@@ -196,3 +196,99 @@ def test_fmm_small_scenes(order, leaf):
         df.set_overlap(True)
     dd.close()
     df.close()
+
+
+def _basis(P, u):
+    """S_k(u) and its derivative at the P Chebyshev nodes, k last."""
+    k = np.arange(P)
+    th = (2 * k + 1) * np.pi / (2 * P)
+    j = np.arange(1, P)
+    tn = np.cos(np.outer(th, j))                       # T_j(xi_k)
+    T = np.stack([np.polynomial.chebyshev.Chebyshev.basis(q)(u) for q in j], axis=-1)
+    dT = np.stack([np.polynomial.chebyshev.Chebyshev.basis(q).deriv()(u) for q in j], axis=-1)
+    return 1.0 / P + 2.0 / P * T @ tn.T, 2.0 / P * dT @ tn.T, np.cos(th)
+
+
+def _interpolated_minus_exact(a, kappa, P, depth, x):
+    """What the order-P interpolation changes in the mat-vec: over the patch
+    pairs whose boxes separate at a level >= 2 (boxes not adjacent, parents
+    adjacent), the interaction between Chebyshev nodes less the exact 1-point
+    one.  Anterpolation straight to every level's boxes: passing through the
+    children is the same polynomial."""
+    c, nrm, ar, ie = a["centroid"], a["normal"], a["area"], 1.0 / a["eps"]
+    n = c.shape[0]
+    lo, hi = c.min(axis=0), c.max(axis=0)
+    edge = float(np.max(hi - lo)) * (1.0 + 1e-9) + 1e-9
+    x0 = (lo + hi) / 2 - edge / 2
+    sh, dv = ar * x[n:], (ar * x[:n])[:, None] * nrm
+
+    def cells(level):
+        m = 1 << level
+        return np.clip(np.floor((c - x0) / edge * m).astype(int), 0, m - 1)
+
+    yf, yh = np.zeros(n), np.zeros(n)
+    offsets = set()
+    for level in range(2, depth + 1):
+        cl = cells(level)
+        box, of = np.unique(cl, axis=0, return_inverse=True)
+        of = of.ravel()
+        h = edge / (1 << level)
+        ctr = x0 + (box[of] + 0.5) * h
+        (sx, dx, xi), (sy, dy, _), (sz, dz, _) = (_basis(P, (c[:, k] - ctr[:, k]) * 2 / h) for k in range(3))
+        S = np.einsum("ia,ib,ic->iabc", sx, sy, sz).reshape(n, -1)
+        G = np.stack([np.einsum("ia,ib,ic->iabc", *t).reshape(n, -1)
+                      for t in ((dx, sy, sz), (sx, dy, sz), (sx, sy, dz))]) * (2 / h)
+        dg = np.einsum("ik,kim->im", dv, G)
+        c1 = sh[:, None] * S - dg
+        M = np.zeros((len(box), 3, P ** 3))
+        np.add.at(M, of, np.stack([ie[:, None] * dg - sh[:, None] * S, c1, ie[:, None] * c1], axis=1))
+        t = box[:, None] - box[None]               # target - source
+        far = (np.abs(t).max(axis=2) > 1) & (np.abs(box[:, None] // 2 - box[None] // 2).max(axis=2) <= 1)
+        node = np.stack(np.meshgrid(xi, xi, xi, indexing="ij"), axis=-1).reshape(-1, 3) / 2
+        L = np.zeros_like(M)
+        for off in {tuple(v) for v in t[far]}:
+            offsets.add(tuple(sorted(abs(int(v)) for v in off)))
+            B, A = np.nonzero(far & np.all(t == off, axis=2))
+            r = h * np.linalg.norm(np.array(off) + node[:, None] - node[None], axis=2)  # target, source node
+            L[B, 0] += M[A, 0] @ (1 / r).T         # a target meets an offset once
+            for e in (1, 2):
+                L[B, e] += M[A, e] @ (np.exp(-kappa * r) / r).T
+        yf += np.einsum("im,im->i", S, L[of, 0] + L[of, 1])
+        yh += np.einsum("ik,kim,im->i", nrm, G, L[of, 0] + L[of, 2])
+        # the exact 1-point interaction of the same pairs
+        for i in range(n):
+            j = np.nonzero(far[of[i]][of])[0]
+            d = c[j] - c[i]
+            r = np.linalg.norm(d, axis=1)
+            e, kr = np.exp(-kappa * r), kappa * r
+            g1, l1 = e * (1 + kr) / r ** 3, 1 / r ** 3
+            dd, nd = np.einsum("jk,jk->j", dv[j], d), d @ nrm[i]
+            yf[i] -= np.sum(sh[j] * (e - 1) / r + dd * (g1 - ie[j] * l1))
+            yh[i] -= np.sum(-sh[j] * nd * l1 + ie[j] * ((dv[j] @ nrm[i]) * (l1 - g1) + sh[j] * nd * g1
+                                                        - dd * nd * (3 - e * (kr * kr + 3 * kr + 3)) / r ** 5))
+    return np.concatenate([yf, yh]) / (4 * np.pi), offsets
+
+
+@pytest.mark.parametrize("order", [3, 4, 5, 6])
+@pytest.mark.parametrize("kappa,leaf", [(0.125, 40), (0.125, 5), (0.0, 10)])
+def test_m2l_against_dense_interpolation(order, kappa, leaf):
+    """The FP64 far field against the same interpolation with dense
+    node-to-node tables on the host, to rounding: every pair of boxes once,
+    in the right node order, at every order and for offsets with each kind of
+    symmetry and with none, (3, 2, 1)."""
+    sc = Scene(80.0, kappa, 6, 0, 100)
+    for k, lv in enumerate((3, 2)):
+        sc.add_instance(Mesh.star(lv, 25.0, 8, 0.04, 9 + k), 2.0, offset=[60.0 * k, 0.0, 5.0 * k])
+    a = sc.build().arrays()
+    x = np.random.default_rng(order).normal(size=2 * a["area"].shape[0])
+    dd = _device(a, kappa, "direct", precs=("fp64",))
+    df = _device(a, kappa, "fmm", order, leaf, precs=("fp64",))
+    depth = df.far_info()["leaf_level"]
+    y, ref = df.matvec(x, "fp64"), dd.matvec(x, "fp64")
+    change, offsets = _interpolated_minus_exact(a, kappa, order, depth, x)
+    err = float(np.linalg.norm((y - ref) - change) / np.linalg.norm(ref))
+    print(order, kappa, leaf, depth, len(offsets), rel(y, ref), err, flush=True)
+    assert depth >= 3 and (1, 2, 3) in offsets and {(0, 0, 2), (1, 2, 2), (0, 1, 2)} <= offsets
+    assert err < 1e-12
+    dd.close()
+    df.close()
