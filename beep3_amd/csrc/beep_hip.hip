@@ -2399,6 +2399,20 @@ int beep_hip_fmm_symmetry(int tx, int ty, int tz, int order, int* canon_xyz, int
     }
 }
 
+int beep_hip_selftest_math(beep_hip_ctx* ctx, int which, int n, const double* x, double* y) {
+    return guarded(ctx, [&] {
+        require((which == 0 || which == 1) && n > 0 && x && y, "bad arguments");
+        set_device(ctx);
+        DevBuf<double> dx, dy;
+        dx.upload(x, size_t(n), ctx->stream);
+        dy.alloc(size_t(n));
+        launch_math_selftest(ctx->stream, which, n, dx.p, dy.p);
+        hip_check(hipMemcpyAsync(y, dy.p, sizeof(double) * size_t(n), hipMemcpyDeviceToHost, ctx->stream),
+                  "D2H selftest");
+        hip_check(hipStreamSynchronize(ctx->stream), "sync selftest");
+    });
+}
+
 int beep_hip_selftest_mfma(beep_hip_ctx* ctx, int fp32, const double* a, const double* b,
                            double* d) {
     return guarded(ctx, [&] {

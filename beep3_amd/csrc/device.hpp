@@ -360,6 +360,8 @@ void launch_point_planes(hipStream_t s, int n, const int* ptr, const Pt64* pts, 
 void launch_to_local(hipStream_t s, int n, int k0, const double* raw, const int* ptr, int N,
                      const Patch64* patches, Pt64* out64, Pt32* out32);
 void launch_mfma_selftest(hipStream_t s, const double* a, const double* b, int fp32, double* out);
+// y[k] = rsqrt_nr(x[k]) (which 0) or exp_neg64(x[k]) (1)
+void launch_math_selftest(hipStream_t s, int which, int n, const double* x, double* y);
 void launch_scale_copy(hipStream_t s, int n, const double* x, const double* scale_ptr,
                        double scale, double* y);
 

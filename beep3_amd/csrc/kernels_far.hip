@@ -191,6 +191,18 @@ void launch_far_direct(hipStream_t s, int fp32, int n, int n_split, const int* o
 
 FarSymShape far_sym_plan(int n) { return far_sym_shape(n); }
 
+__global__ __launch_bounds__(256) void k_math_selftest(int which, int n, const double* __restrict__ x,
+                                                      double* __restrict__ y) {
+    const int k = blockIdx.x * 256 + threadIdx.x;
+    if (k < n) y[k] = which ? exp_neg64(x[k]) : rsqrt_nr(x[k]);
+}
+
+void launch_math_selftest(hipStream_t s, int which, int n, const double* x, double* y) {
+    if (n <= 0) return;
+    hipLaunchKernelGGL(k_math_selftest, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, which, n, x, y);
+    hip_check(hipGetLastError(), "k_math_selftest launch");
+}
+
 // The symmetric tile pairs as a launch of their own (a near field on the fly
 // or shared, or the streams not overlapped; else k_direct_part).
 template <typename T>

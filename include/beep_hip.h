@@ -443,6 +443,9 @@ int beep_hip_solve_device(beep_hip_ctx* ctx, const double* d_b, double* d_x,
  * result layout the M2L kernels rely on. */
 int beep_hip_selftest_mfma(beep_hip_ctx* ctx, int fp32, const double* a, const double* b,
                            double* d);
+/* Diagnostic: the FP64 kernels' reciprocal root of x[k] > 0 (which 0) or
+ * e^-x[k], x[k] >= 0 (1), n host values to y. */
+int beep_hip_selftest_math(beep_hip_ctx* ctx, int which, int n, const double* x, double* y);
 
 /* Diagnostic (host only): the M2L symmetry used by the FMM.  For a source
  * box at offset t = (tx, ty, tz) (box units, 2 <= max |t_k| <= 3) returns
