@@ -471,15 +471,20 @@ void far_buffers(beep_hip_ctx* c) {
 
 // The stream of the FMM's leaf pass (20 to 80 us): the shorter of the two.
 // Estimates from runs of each alone: the SpMV streams 6 TB/s; the Chebyshev far
-// field takes 1.9 (FP64) or 1.1 ns (FP32) per M2L pair at order 5, about as
-// the cube of the order, and half of that again around it.  Not beside the
-// plane waves (longer than their SpMV at every size) or a near field on the
-// fly.  163,842 patches, FP64: the last kernels after the SpMV 100 -> 25 us.
+// field takes 60 us for its chain of dependent launches and 1.9 (FP64) or 1.1
+// ns (FP32) per M2L pair at order 5, about as the cube of the order, and half
+// of that again around it.  Not beside the plane waves (longer than their SpMV
+// at every size) or a near field on the fly.  Both sides measured at 10,242,
+// 40,962 and 163,842 patches, orders 3 to 6, leaf targets 30 and 64, all three
+// precisions: the line falls on the faster side or within 1 % of it in all 72.
+// Mat-vecs in us, pass after the SpMV / on the far stream, leaf target 64,
+// FP64: 10,242 patches order 5 182 / 198; 40,962 order 4 463 / 445, order 6
+// 710 / 720; 163,842 order 5 1,794 / 1,763; FP32: 40,962 order 5 296 / 316.
 bool leaf_pass_on_far(const beep_hip_ctx* c, int mode) {
     if (c->share || c->near_mode != BEEP_NEAR_PRECOMPUTE || c->fmm->engine != 0) return false;
     const double near_us = double(c->nnz) * (mode == 0 ? 32.0 : 16.0) / 6e6;
     const double p = c->fmm->P / 5.0;
-    const double far_us = double(c->fmm->n_pairs) * (mode == 1 ? 1.1e-3 : 1.9e-3) * p * p * p * 1.5;
+    const double far_us = 60.0 + double(c->fmm->n_pairs) * (mode == 1 ? 1.1e-3 : 1.9e-3) * p * p * p * 1.5;
     return near_us > far_us;
 }
 
