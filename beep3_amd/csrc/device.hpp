@@ -127,17 +127,18 @@ struct DevArena {
 // its unit normal (a planar triangle's points): per run the normal n and n.p
 // (local frame, FP64), and per patch an upper bound of |p|; for FP32 kernels the
 // points again as position and weight alone.  Both point arrays have one unused
-// entry behind the last (the kernels load one point ahead).  gs = 0: no such structure (curved triangles).  Run of a patch's first
-// point k: k / gs.
+// entry behind the last (the kernels load one point ahead).  gs = 0: no such
+// structure (curved triangles).  Run of a patch's first point k: k / gs.
 struct PointPlanes {
     const double4* plane = nullptr;
     const float* radius = nullptr;
     const float4* xyzw = nullptr;
     int gs = 0;
 };
-// Shorter runs keep a normal per point: the FP32 precompute of 4,002 patches with
-// one point per sub-triangle (runs of 2) took 241 us so and 257 us by runs.  8 is
-// the next length a rule gives: 483 us and 384 us by runs (FP64: 935 and 699).
+// Shorter runs keep a normal per point: 10,242 patches with one point per
+// sub-triangle (runs of 2), FP32, take 488 us so and 516 by runs, on the fly 784
+// and 1,127 (FP64 697 and 680, 1,030 and 1,029).  8 is the next length a rule
+// gives: FP32 998 us and 800 by runs, FP64 1,843 and 1,416.
 constexpr int MIN_RUN = 4;
 
 // ---- launchers (defined in the .hip files) ----

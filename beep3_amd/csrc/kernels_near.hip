@@ -204,8 +204,8 @@ __device__ __forceinline__ int find_leaf(const int* __restrict__ blk_ptr, int n_
 // 46 and 71 with a normal per point.  The next point is loaded while this one is
 // worked on: without that the FP32 loop waits for the L1 at every point and
 // gains nothing (setup below: 23.8 ms).  Before and after, 72 points a patch:
-// whole setup with a mat-vec, FP32, 163,842 patches, 22.4 -> 17.3 ms; precompute
-// alone, FP64, 4,002 patches, 1.30 -> 0.95 ms.
+// whole setup with a mat-vec, FP32, 163,842 patches, 22.4 -> 16.8 ms; precompute
+// alone, FP64, 10,242 patches, 2.65 -> 1.96 ms.
 template <typename T>
 struct PlanePoint {
     T x, y, z, w;
@@ -892,13 +892,13 @@ void launch_near_spmv(hipStream_t s, int mode, int n, const SpmvPlan& p, const i
 // side, the far ones spread evenly over the grid, so the SpMV's HBM time and
 // the far field's VALU time overlap without a second stream, its fork / join
 // events and the launches of a separate chain (fill, pack, sum, add).  The
-// sums are those of k_near_spmv_part and of the far field alone, so the
-// launches may also be made apart (n_far or n_near 0), for the same bits.
+// sums are those of k_near_spmv_part and k_far_sym, which run apart give the
+// same bits.
 // Whole mat-vecs against two streams with the one-directional far field:
 // 2,562 patches FP32 130 -> 54 us, 10,242 FP64 457 -> 223 us, 11,304 FP32
 // coefficients with FP64 sums 465 -> 250 us.  Up to FAR_SYM_MAX patches the
-// partial sums (n^2 / 32 values of partner sums, 13 MB at the limit) stay
-// cheap; above, the FMM is the default and the direct sum a reference.
+// partial sums (n^2 / 256 values of partner sums, 13 MB in FP64 at the limit)
+// stay cheap; above, the FMM is the default and the direct sum a reference.
 template <typename TC, typename TA, int U, typename TF>
 __global__ __launch_bounds__(256) void k_direct_part(
     int n_near, int n_far, const int4* __restrict__ work, const int* __restrict__ leaf_ptr,

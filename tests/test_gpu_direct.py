@@ -1,6 +1,7 @@
 """The direct far field as symmetric tile pairs and the FP64 set without a far
 field, against the FP64 CPU oracle, at the edges of the 256- and 64-patch
-tiles and of the SpMV's work items, over every route to them."""
+tiles and of the SpMV's work items, over the routes to them (without
+allocations: test_zz_no_alloc.py)."""
 import threading
 
 import numpy as np
