@@ -27,12 +27,15 @@ def _device(b, Dp, far, precs):
     return d, sc, a
 
 
-@pytest.mark.parametrize("case", ["born_direct", "off_centre_fmm"])
+# born_auto: one leaf, no far field in FP64; off_centre_direct: above the
+# symmetric far field's sizes
+@pytest.mark.parametrize("case", ["born_direct", "born_auto", "off_centre_fmm", "off_centre_direct"])
 def test_graph_replay_matches_eager(case):
-    if case == "born_direct":
-        b, Dp, far = configs.born_ion(), 2.0, "direct"
+    far = case.split("_")[-1]
+    if case.startswith("born"):
+        b, Dp = configs.born_ion(), 2.0
     else:
-        b, Dp, far = configs.off_centre(), 4.0, "fmm"
+        b, Dp = configs.off_centre(), 4.0
     d, sc, a = _device(b, Dp, far, ("fp64", "fp32"))
     rhs = d.rhs(a["charges"], b.Dsolvent)
     out = {}
